@@ -407,7 +407,9 @@ kf_status kf_block_bitmaps(kf_context* ctx, uint32_t* observed, uint32_t* skip, 
 
 /* ---- MarchingCubes::extract (marching_cubes.cpp:478-507) on the device:
  * cell classification, stream-compacted triangles and the reference's
- * first-encounter vertex welding order. */
+ * first-encounter vertex welding order.  The mesh stays in device memory of
+ * its own (36 B a vertex, 12 B a triangle) until kf_mesh_free, and may outlive
+ * the context; kf_mesh_copy transfers it. */
 kf_status kf_mesh_extract(kf_context* ctx, float min_weight, kf_mesh** out);
 kf_status kf_mesh_size(const kf_mesh* mesh, int64_t* vertices, int64_t* triangles);
 kf_status kf_mesh_copy(const kf_mesh* mesh, float* positions, float* normals, float* colors,

@@ -698,6 +698,8 @@ void kf_destroy(kf_context* ctx) {
   dfree(ctx->block_of_slot);
   dfree(ctx->work);
   dfree(ctx->sparse);
+  for (auto& b : ctx->mesh_scratch) dfree(b.p);
+  if (ctx->mesh_totals != nullptr) (void)hipHostFree(ctx->mesh_totals);
   if (ctx->icp_host != nullptr) (void)hipHostFree(ctx->icp_host);
   for (auto& e : ctx->ev)
     if (e != nullptr) (void)hipEventDestroy(e);

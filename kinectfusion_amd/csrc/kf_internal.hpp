@@ -413,6 +413,11 @@ struct LevelBuffers {
   uint32_t* model_col = nullptr;
 };
 
+struct DeviceBlock {
+  void* p = nullptr;
+  size_t bytes = 0;
+};
+
 }  // namespace kf
 
 struct kf_context {
@@ -499,6 +504,10 @@ struct kf_context {
   uint16_t* prev_coarse = nullptr;
   float* twist = nullptr;
   bool timed_learned = false;
+  // mesh extraction: device scratch kept between calls (bit maps; active
+  // cells; vertices) and the pinned counts its scans write
+  kf::DeviceBlock mesh_scratch[3];
+  unsigned long long* mesh_totals = nullptr;
 };
 
 namespace kf {
