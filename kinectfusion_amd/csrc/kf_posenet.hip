@@ -174,53 +174,71 @@ __global__ void __launch_bounds__(256) gemm_kernel(Gemm g) {
   f32x4 acc[2][2];
   for (int i = 0; i < 2; ++i)
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0F, 0.0F, 0.0F, 0.0F};
-  for (int k0 = kb; k0 < ke; k0 += BK) {
-    const int k = k0 + sc;
-    const bool kin = k < ke;
+  // The staged values of one K step, all reads in flight together: an address
+  // past an edge is clamped and its value zeroed, since a guarded read would
+  // wait for the one before it.
+  uint16_t av[kRowsPerThread], bv[kRowsPerThread];
+  auto stage = [&](int k0) {
+    const int k = k0 + sc, kc = min(k, ke - 1);
     int ky = 0, kx = 0, ch = 0;
     if (implicit) {
-      const int tap = k / g.conv.C;
-      ch = k - tap * g.conv.C;
+      const int tap = kc / g.conv.C;
+      ch = kc - tap * g.conv.C;
       ky = tap / 3;
       kx = tap - ky * 3;
     }
 #pragma unroll
     for (int i = 0; i < kRowsPerThread; ++i) {
       const int r = sr + kStageRows * i;
-      const int m = m0 + r, n = n0 + r;
-      uint16_t av = 0;
-      if (kin) {
-        if (!implicit) {
-          if (m < g.M) av = g.a[m * g.sam + k * g.sak];
+      const int m = min(m0 + r, g.M - 1), n = min(n0 + r, g.N - 1);
+      if (!implicit) {
+        av[i] = g.a[m * g.sam + kc * g.sak];
+      } else {
+        const int yi = min(max(oy[i] + ky, 0), g.conv.H - 1), xi = min(max(ox[i] + kx, 0), g.conv.W - 1);
+        if (g.conv.raw_prev != nullptr) {
+          const uint16_t* src = ch == 0 ? g.conv.raw_prev : g.conv.raw_cur;
+          av[i] = src[ob[i] * g.conv.raw_stride + yi * g.conv.W + xi];
         } else {
-          const int yi = oy[i] + ky, xi = ox[i] + kx;
-          if (yi >= 0 && yi < g.conv.H && xi >= 0 && xi < g.conv.W) {
-            if (g.conv.raw_prev != nullptr) {
-              const uint16_t* src = ch == 0 ? g.conv.raw_prev : g.conv.raw_cur;
-              av = raw_to_input(src[ob[i] * g.conv.raw_stride + yi * g.conv.W + xi], g.conv.inv_scale);
-            } else {
-              av = g.conv.x[((static_cast<long long>(ob[i]) * g.conv.H + yi) * g.conv.W + xi) * g.conv.C + ch];
-            }
-          }
+          av[i] = g.conv.x[((static_cast<long long>(ob[i]) * g.conv.H + yi) * g.conv.W + xi) * g.conv.C + ch];
         }
       }
-      As[r][sc] = av;
-      Bs[r][sc] = (n < g.N && kin) ? g.b[k * g.sbk + n * g.sbn] : static_cast<uint16_t>(0);
+      bv[i] = g.b[kc * g.sbk + n * g.sbn];
+    }
+#pragma unroll
+    for (int i = 0; i < kRowsPerThread; ++i) {
+      const int r = sr + kStageRows * i;
+      bool in = k < ke && m0 + r < g.M;
+      if (implicit) {
+        const int yi = oy[i] + ky, xi = ox[i] + kx;
+        in = k < ke && yi >= 0 && yi < g.conv.H && xi >= 0 && xi < g.conv.W;
+        if (g.conv.raw_prev != nullptr) av[i] = raw_to_input(av[i], g.conv.inv_scale);
+      }
+      av[i] = in ? av[i] : static_cast<uint16_t>(0);
+      bv[i] = k < ke && n0 + r < g.N ? bv[i] : static_cast<uint16_t>(0);
+    }
+  };
+  stage(kb);
+  for (int k0 = kb; k0 < ke; k0 += BK) {
+#pragma unroll
+    for (int i = 0; i < kRowsPerThread; ++i) {
+      As[sr + kStageRows * i][sc] = av[i];
+      Bs[sr + kStageRows * i][sc] = bv[i];
     }
     __syncthreads();
+    if (k0 + BK < ke) stage(k0 + BK);  // the next step's reads run behind this step's MFMAs
     {  // the staged 32 k as one 16x16x32 step
-      s16x8 av[2], bv[2];
+      s16x8 af[2], bf[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        av[i] = *reinterpret_cast<const s16x8*>(&As[wm + i * 16 + li][lq * 8]);
-        bv[i] = *reinterpret_cast<const s16x8*>(&Bs[wn + i * 16 + li][lq * 8]);
+        af[i] = *reinterpret_cast<const s16x8*>(&As[wm + i * 16 + li][lq * 8]);
+        bf[i] = *reinterpret_cast<const s16x8*>(&Bs[wn + i * 16 + li][lq * 8]);
       }
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av[i]),
-                                                              __builtin_bit_cast(bf16x8, bv[j]), acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[i]),
+                                                              __builtin_bit_cast(bf16x8, bf[j]), acc[i][j], 0, 0, 0);
     }
     __syncthreads();
   }
@@ -242,7 +260,7 @@ __global__ void __launch_bounds__(256) gemm_kernel(Gemm g) {
       }
 }
 
-// Sum of the split partials in split order 0, 1, ... (eight reads in
+// Sum of the split partials in split order 0, 1, ... (sixteen reads in
 // flight per thread), then the epilogue.
 __global__ void gemm_finish_kernel(Gemm g, int splits) {
   const long long total = static_cast<long long>(g.M) * g.N;
@@ -250,16 +268,64 @@ __global__ void gemm_finish_kernel(Gemm g, int splits) {
   if (i >= total) return;
   const float* p = g.partial + i;
   float s = 0.0F;
-  int z = 0;
-  for (; z + 8 <= splits; z += 8) {
-    float v[8];
+  constexpr int kRun = 16;
+  for (int z = 0; z < splits; z += kRun) {
+    float v[kRun];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = p[(z + j) * total];
+    for (int j = 0; j < kRun; ++j) v[j] = p[min(z + j, splits - 1) * total];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) s += v[j];
+    for (int j = 0; j < kRun; ++j) s += z + j < splits ? v[j] : 0.0F;  // + 0 past the end leaves the sum as it is
   }
-  for (; z < splits; ++z) s += p[z * total];
   gemm_store(g, static_cast<int>(i / g.N), static_cast<int>(i % g.N), s);
+}
+
+// Sums down the columns of x[rows][n], the rows in order 0, 1, ...: the order
+// is serial per column, so the reads must not be.  A workgroup stages its 32
+// columns 256 rows at a time in LDS (32 reads per thread in flight, the next
+// piece's reads issued before this one is added) and one thread per column
+// adds them.  A thread per column reading its rows itself took 175 us for
+// 1200 rows of 16 columns; this takes MEASURE_ROWSUM us.
+constexpr int kSumCols = 32, kSumRows = 256;
+struct RowSum {
+  const float* x;
+  int rows, n;
+};
+template <typename Store>
+__device__ inline void row_sum(const RowSum& r, int c0, Store&& store) {
+  __shared__ float piece[kSumRows][kSumCols + 1];
+  constexpr int kReads = kSumRows * kSumCols / 256;
+  const int col = threadIdx.x & (kSumCols - 1), row = threadIdx.x / kSumCols;
+  const bool in = c0 + col < r.n;
+  float v[kReads];
+  auto read = [&](int r0) {
+#pragma unroll
+    for (int j = 0; j < kReads; ++j) {
+      // clamped, not skipped: a guarded read would wait for the one before
+      v[j] = r.x[static_cast<long long>(min(r0 + row + j * (256 / kSumCols), r.rows - 1)) * r.n + min(c0 + col, r.n - 1)];
+    }
+  };
+  float s = 0.0F;
+  read(0);
+  for (int r0 = 0; r0 < r.rows; r0 += kSumRows) {
+#pragma unroll
+    for (int j = 0; j < kReads; ++j) piece[row + j * (256 / kSumCols)][col] = v[j];
+    __syncthreads();
+    if (r0 + kSumRows < r.rows) read(r0 + kSumRows);
+    if (threadIdx.x < kSumCols) {
+      const int n = min(kSumRows, r.rows - r0);
+#pragma unroll 16
+      for (int i = 0; i < n; ++i) s += piece[i][threadIdx.x];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x < kSumCols && in) store(c0 + col, s);
+}
+
+// The split partials of a long reduction (more splits than one piece's worth
+// of reads in flight per thread), then the epilogue.
+__global__ void __launch_bounds__(256) gemm_finish_rows_kernel(Gemm g, int splits) {
+  row_sum(RowSum{g.partial, splits, g.M * g.N}, static_cast<int>(blockIdx.x) * kSumCols,
+          [&](int i, float s) { gemm_store(g, i / g.N, i % g.N, s); });
 }
 
 // ---------------------------------------------------------------------------
@@ -340,8 +406,10 @@ __global__ void __launch_bounds__(Waves * 64) gemm_small_kernel(Gemm g, int vec_
           af[c] = *reinterpret_cast<const s16x8*>(g.a + m * g.sam + k);
         } else {
 #pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (k + j < g.K) af[c][j] = as_short(g.a[m * g.sam + (k + j) * g.sak]);
+          for (int j = 0; j < 8; ++j) {  // clamped and zeroed: guarded reads would wait for one another
+            const short v = as_short(g.a[m * g.sam + min(k + j, g.K - 1) * g.sak]);
+            af[c][j] = k + j < g.K ? v : short{0};
+          }
         }
       }
       if (nok) {
@@ -349,8 +417,10 @@ __global__ void __launch_bounds__(Waves * 64) gemm_small_kernel(Gemm g, int vec_
           bfr[c] = *reinterpret_cast<const s16x8*>(g.b + n * g.sbn + k);
         } else {
 #pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (k + j < g.K) bfr[c][j] = as_short(g.b[(k + j) * g.sbk + n * g.sbn]);
+          for (int j = 0; j < 8; ++j) {
+            const short v = as_short(g.b[min(k + j, g.K - 1) * g.sbk + n * g.sbn]);
+            bfr[c][j] = k + j < g.K ? v : short{0};
+          }
         }
       }
     }
@@ -390,56 +460,77 @@ __global__ void input_kernel(const uint16_t* prev0, const uint16_t* cur0, long l
   x0[o + 1] = to_bf16(c);
 }
 
-// col[m][k]: m = (b * Ho + yo) * Wo + xo, k = (ky * 3 + kx) * C + c.
-__global__ void im2col_kernel(const uint16_t* x, uint16_t* col, int batch, int H, int W, int C, int Ho,
-                              int Wo) {
-  const int K = 9 * C;
-  const long long total = static_cast<long long>(batch) * Ho * Wo * K;
-  for (long long e = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; e < total;
-       e += static_cast<long long>(gridDim.x) * blockDim.x) {
-    const long long m = e / K;
-    const int k = static_cast<int>(e % K);
-    const int tap = k / C, c = k % C;
-    const int ky = tap / 3, kx = tap % 3;
-    const int xo = static_cast<int>(m % Wo);
-    const long long t = m / Wo;
-    const int yo = static_cast<int>(t % Ho);
-    const int b = static_cast<int>(t / Ho);
+// col[m][k]: m = (b * Ho + yo) * Wo + xo, k = (ky * 3 + kx) * C + c.  Run
+// consecutive channels of one tap per thread as one word (2 channels: 4 bytes,
+// otherwise 8: 16 bytes), so a thread's index divisions are paid once per word.
+template <int Run>
+struct Channels {
+  uint16_t v[Run];
+} __attribute__((aligned(Run * 2)));
+template <int Run>
+__global__ void __launch_bounds__(256) im2col_kernel(const uint16_t* x, uint16_t* col, int batch, int H, int W, int C,
+                                                     int Ho, int Wo) {
+  const unsigned per = static_cast<unsigned>(9 * C / Run), groups = static_cast<unsigned>(C / Run);
+  const unsigned total = static_cast<unsigned>(batch * Ho * Wo) * per;  // < 2^32: at most 4096 x 4800 x 18
+  for (unsigned e = blockIdx.x * 256U + threadIdx.x; e < total; e += gridDim.x * 256U) {
+    const unsigned m = e / per, r = e - m * per;
+    const int tap = static_cast<int>(r / groups), c = static_cast<int>(r - tap * groups) * Run;
+    const int ky = tap / 3, kx = tap - ky * 3;
+    const unsigned t = m / static_cast<unsigned>(Wo);
+    const int xo = static_cast<int>(m - t * Wo), b = static_cast<int>(t / static_cast<unsigned>(Ho));
+    const int yo = static_cast<int>(t) - b * Ho;
     const int yi = 2 * yo - 1 + ky, xi = 2 * xo - 1 + kx;
-    col[e] = (yi >= 0 && yi < H && xi >= 0 && xi < W)
-                 ? x[((static_cast<long long>(b) * H + yi) * W + xi) * C + c]
-                 : static_cast<uint16_t>(0);
+    Channels<Run> v{};
+    if (yi >= 0 && yi < H && xi >= 0 && xi < W)
+      v = *reinterpret_cast<const Channels<Run>*>(x + ((static_cast<size_t>(b) * H + yi) * W + xi) * C + c);
+    *reinterpret_cast<Channels<Run>*>(col + static_cast<size_t>(e) * Run) = v;
   }
 }
 
 // dx[b][yi][xi][c] = sum over the taps that read it of dcol, in (ky, kx)
-// order, times the ReLU mask of the layer input; bf16 out.
-__global__ void col2im_kernel(const float* dcol, const uint16_t* xin, uint16_t* dx, int batch, int H, int W,
-                              int C, int Ho, int Wo) {
-  const long long total = static_cast<long long>(batch) * H * W * C;
-  const int K = 9 * C;
-  for (long long e = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; e < total;
-       e += static_cast<long long>(gridDim.x) * blockDim.x) {
-    float s = 0.0F;
-    if (from_bf16(xin[e]) > 0.0F) {
-      const int c = static_cast<int>(e % C);
-      const long long p = e / C;
-      const int xi = static_cast<int>(p % W);
-      const long long t = p / W;
-      const int yi = static_cast<int>(t % H);
-      const int b = static_cast<int>(t / H);
-      for (int ky = 0; ky < 3; ++ky) {
-        const int ty = yi + 1 - ky;
-        if (ty < 0 || (ty & 1) != 0 || (ty >> 1) >= Ho) continue;
-        for (int kx = 0; kx < 3; ++kx) {
-          const int tx = xi + 1 - kx;
-          if (tx < 0 || (tx & 1) != 0 || (tx >> 1) >= Wo) continue;
-          const long long m = (static_cast<long long>(b) * Ho + (ty >> 1)) * Wo + (tx >> 1);
-          s += dcol[m * K + (ky * 3 + kx) * C + c];
-        }
+// order, times the ReLU mask of the layer input; bf16 out.  Four channels per
+// thread (C is a multiple of 16); at most four taps read a pixel, and their
+// reads are issued together.
+__global__ void __launch_bounds__(256) col2im_kernel(const float* dcol, const uint16_t* xin, uint16_t* dx, int batch,
+                                                     int H, int W, int C, int Ho, int Wo) {
+  const unsigned groups = static_cast<unsigned>(C / 4);
+  const unsigned total = static_cast<unsigned>(batch * H * W) * groups;
+  for (unsigned e = blockIdx.x * 256U + threadIdx.x; e < total; e += gridDim.x * 256U) {
+    const unsigned p = e / groups;
+    const int c = static_cast<int>(e - p * groups) * 4;
+    const unsigned t = p / static_cast<unsigned>(W);
+    const int xi = static_cast<int>(p - t * W), b = static_cast<int>(t / static_cast<unsigned>(H));
+    const int yi = static_cast<int>(t) - b * H;
+    // taps with (yi + 1 - ky) even: ky = 1, or 0 and 2; along x alike
+    const int ky0 = (yi & 1) != 0 ? 0 : 1, kx0 = (xi & 1) != 0 ? 0 : 1;
+    float4 v[2][2];
+    bool in[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int ky = ky0 + 2 * i, kx = kx0 + 2 * j, ty = yi + 1 - ky, tx = xi + 1 - kx;
+        in[i][j] = ky < 3 && kx < 3 && ty >= 0 && (ty >> 1) < Ho && tx >= 0 && (tx >> 1) < Wo;
+        const size_t m = in[i][j] ? (static_cast<size_t>(b) * Ho + (ty >> 1)) * Wo + (tx >> 1) : 0;
+        const int tap = in[i][j] ? ky * 3 + kx : 0;
+        v[i][j] = *reinterpret_cast<const float4*>(dcol + (m * 9 + tap) * C + c);
       }
-    }
-    dx[e] = to_bf16(s);
+    const Channels<4> act = *reinterpret_cast<const Channels<4>*>(xin + static_cast<size_t>(e) * 4);
+    float s[4] = {0.0F, 0.0F, 0.0F, 0.0F};
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if (!in[i][j]) continue;
+        s[0] += v[i][j].x;
+        s[1] += v[i][j].y;
+        s[2] += v[i][j].z;
+        s[3] += v[i][j].w;
+      }
+    Channels<4> out;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) out.v[q] = to_bf16(from_bf16(act.v[q]) > 0.0F ? s[q] : 0.0F);
+    *reinterpret_cast<Channels<4>*>(dx + static_cast<size_t>(e) * 4) = out;
   }
 }
 
@@ -484,8 +575,20 @@ __global__ void __launch_bounds__(256) colsum_chunk_kernel(const uint16_t* x, in
     const int groups = 256 / cols;  // row lanes per column
     const int col = threadIdx.x % cols, grp = threadIdx.x / cols;
     float s = 0.0F;
-    if (grp < groups)
-      for (int r = r0 + grp; r < r1; r += groups) s += from_bf16(x[static_cast<long long>(r) * N + nb + col]);
+    if (grp < groups) {
+      // sixteen rows in flight, added in row order
+      constexpr int kRun = 16;
+      for (int r = r0 + grp; r < r1; r += kRun * groups) {
+        uint16_t v[kRun];
+#pragma unroll
+        for (int j = 0; j < kRun; ++j) {
+          // clamped, not skipped: a guarded read would wait for the one before
+          v[j] = x[static_cast<long long>(min(r + j * groups, r1 - 1)) * N + nb + col];
+        }
+#pragma unroll
+        for (int j = 0; j < kRun; ++j) s += r + j * groups < r1 ? from_bf16(v[j]) : 0.0F;  // + 0 past the end
+      }
+    }
     red[threadIdx.x] = s;
     __syncthreads();
     if (threadIdx.x < cols) {
@@ -496,12 +599,8 @@ __global__ void __launch_bounds__(256) colsum_chunk_kernel(const uint16_t* x, in
     __syncthreads();
   }
 }
-__global__ void colsum_final_kernel(const float* part, int chunks, int N, float* out) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  float s = 0.0F;
-  for (int c = 0; c < chunks; ++c) s += part[static_cast<long long>(c) * N + n];
-  out[n] = s;
+__global__ void __launch_bounds__(256) colsum_final_kernel(const float* part, int chunks, int N, float* out) {
+  row_sum(RowSum{part, chunks, N}, static_cast<int>(blockIdx.x) * kSumCols, [&](int c, float s) { out[c] = s; });
 }
 
 __global__ void adam_kernel(float* w, const float* g, float* m, float* v, uint16_t* wh, long long n, float lr,
@@ -601,7 +700,11 @@ void gemm(kf_posenet* net, hipStream_t s, Gemm g) {
   hipLaunchKernelGGL(gemm_kernel, dim3(tm, tn, splits), dim3(256), 0, s, g);
   if (splits > 1) {
     const long long total = static_cast<long long>(g.M) * g.N;
-    hipLaunchKernelGGL(gemm_finish_kernel, dim3(blocks_for(total)), dim3(256), 0, s, g, splits);
+    // few outputs with many splits: staged; otherwise a thread per output
+    if (splits > 64)
+      hipLaunchKernelGGL(gemm_finish_rows_kernel, dim3(blocks_for(total, kSumCols)), dim3(256), 0, s, g, splits);
+    else
+      hipLaunchKernelGGL(gemm_finish_kernel, dim3(blocks_for(total)), dim3(256), 0, s, g, splits);
   }
   KF_HIP(hipGetLastError());
 }
@@ -624,7 +727,7 @@ Gemm make_gemm(const uint16_t* a, long long sam, long long sak, const uint16_t* 
 void colsum(kf_posenet* net, hipStream_t s, const uint16_t* x, int M, int N, float* out) {
   const int chunks = (M + kColRows - 1) / kColRows;
   hipLaunchKernelGGL(colsum_chunk_kernel, dim3(chunks), dim3(256), 0, s, x, M, N, net->colpart);
-  hipLaunchKernelGGL(colsum_final_kernel, dim3(blocks_for(N)), dim3(256), 0, s, net->colpart, chunks, N, out);
+  hipLaunchKernelGGL(colsum_final_kernel, dim3(blocks_for(N, kSumCols)), dim3(256), 0, s, net->colpart, chunks, N, out);
   KF_HIP(hipGetLastError());
 }
 
@@ -636,8 +739,12 @@ void forward(kf_posenet* net, hipStream_t s, int batch) {
     const Shape& sh = net->shapes[l];
     const int M = batch * pixels(sh), K = sh.fan_in;
     const long long total = static_cast<long long>(M) * K;
-    hipLaunchKernelGGL(im2col_kernel, dim3(std::min(blocks_for(total), 8192)), dim3(256), 0, s, net->act[l],
-                       net->col[l], batch, sh.hin, sh.win, sh.cin, sh.hout, sh.wout);
+    if (sh.cin % 8 == 0)
+      hipLaunchKernelGGL(im2col_kernel<8>, dim3(std::min(blocks_for(total / 8), 8192)), dim3(256), 0, s, net->act[l],
+                         net->col[l], batch, sh.hin, sh.win, sh.cin, sh.hout, sh.wout);
+    else
+      hipLaunchKernelGGL(im2col_kernel<2>, dim3(std::min(blocks_for(total / 2), 8192)), dim3(256), 0, s, net->act[l],
+                         net->col[l], batch, sh.hin, sh.win, sh.cin, sh.hout, sh.wout);
     Gemm g = make_gemm(net->col[l], K, 1, net->wh + sh.w_off, 1, K, M, sh.cout, K);
     g.bias = net->w + sh.b_off;
     g.relu = 1;
@@ -722,7 +829,7 @@ void backward(kf_posenet* net, hipStream_t s, const float* targets, int batch) {
     d.ofn = 1;
     gemm(net, s, d);
     const long long total = static_cast<long long>(batch) * sh.hin * sh.win * sh.cin;
-    hipLaunchKernelGGL(col2im_kernel, dim3(std::min(blocks_for(total), 8192)), dim3(256), 0, s, net->tmp,
+    hipLaunchKernelGGL(col2im_kernel, dim3(std::min(blocks_for(total / 4), 8192)), dim3(256), 0, s, net->tmp,
                        net->act[l], net->dz[1 - cur], batch, sh.hin, sh.win, sh.cin, sh.hout, sh.wout);
     KF_HIP(hipGetLastError());
     cur = 1 - cur;
