@@ -22,6 +22,7 @@
 // training is deterministic.
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "kf_internal.hpp"
@@ -128,8 +129,7 @@ struct Gemm {
 };
 
 constexpr int BM = 64, BN = 64, BK = 32, LDK = BK + 8;  // 80-byte rows: 16-byte fragment reads stay aligned
-constexpr int kStageRows = 256 / BK;           // rows one pass of the workgroup stages
-constexpr int kRowsPerThread = BM / kStageRows;  // 8
+static_assert(BM == 64 && BN == 64 && BK == 32, "the staging modes map 256 threads to 64 x 32 values");
 constexpr int kMaxTiles = 256;                   // at most this many tiles split K
 
 __device__ inline uint16_t raw_to_input(uint16_t r, float inv_scale) {
@@ -143,6 +143,138 @@ __device__ inline void gemm_store(const Gemm& g, int m, int n, float v) {
   if (g.outh != nullptr) g.outh[m * g.ohm + n * g.ohn] = to_bf16(v);
 }
 
+// How a workgroup stages an operand's 64 rows (m or n) x 32 k of one K step
+// (eight values a thread), by what lies next to each other in memory:
+//  kStageRows8   eight k of a row per 16-byte read (k contiguous, rows 16-byte aligned)
+//  kStageRows2   two k per 4-byte read (k contiguous, even row length)
+//  kStageCols    two rows of two k each: rows contiguous, so a read holds two rows of
+//           one k, and two reads are transposed in registers (weight and input
+//           gradients, whose operands are stored k-major; lanes run along the
+//           rows, so a wave's reads are whole lines)
+//  kStageScalar  one value at a time
+//  kStageConv8   the im2col matrix of a convolution, eight channels of a tap per
+//           16-byte read
+//  kStageConv    the same one value at a time (the raw depth pair)
+// Every address past an edge is clamped and its value zeroed: a guarded read
+// would wait for the one before it.  The values and their places are the same
+// in every mode, so the sums are too.
+// What bounds a tile is the read round per K step.  One value at a time, lanes
+// along k, the gradients of 64 pairs took 390 us in these GEMMs (56 us for the
+// second layer's weight gradient, whose reads were strided); the modes take
+// 155 us (18 us).
+enum StageMode { kStageScalar = 0, kStageRows8, kStageRows2, kStageCols, kStageConv8, kStageConv };
+
+template <int Mode>
+struct Stage {
+  uint32_t v[4];  // eight bf16 values
+  // rows of thread t: kStageRows8 / kStageConv8: t / 4, k 8 (t % 4); kStageRows2: t / 16 + 16 i, k 2 (t % 16);
+  // kStageCols: 2 (t % 32), 2 (t % 32) + 1, k 2 (t / 32) + 16 i; kStageScalar / kStageConv: t / 32 + 8 i, k t % 32
+  __device__ inline void read(const uint16_t* p, long long srow, long long sk, int row0, int rows, int k0, int ke,
+                              const ConvView& cv, const int* org) {
+    const int t = static_cast<int>(threadIdx.x);
+    if constexpr (Mode == kStageRows8) {
+      const int r = row0 + (t >> 2), k = k0 + (t & 3) * 8;
+      // ke is a multiple of 8 (the host's check), so the eight lie inside or outside together
+      const uint4 q = *reinterpret_cast<const uint4*>(p + min(r, rows - 1) * srow + min(k, ke - 8));
+      const bool in = r < rows && k < ke;
+      v[0] = in ? q.x : 0U;
+      v[1] = in ? q.y : 0U;
+      v[2] = in ? q.z : 0U;
+      v[3] = in ? q.w : 0U;
+    } else if constexpr (Mode == kStageRows2) {
+      const int k = k0 + (t & 15) * 2;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        v[i] = *reinterpret_cast<const uint32_t*>(p + min(row0 + (t >> 4) + 16 * i, rows - 1) * srow + min(k, ke - 2));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = row0 + (t >> 4) + 16 * i < rows && k < ke ? v[i] : 0U;
+    } else if constexpr (Mode == kStageCols) {
+      const int r = row0 + (t & 31) * 2;
+      const uint16_t* base = p + min(r, rows - 2);  // rows is even
+      uint32_t q[4];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          q[2 * i + j] = *reinterpret_cast<const uint32_t*>(base + min(k0 + (t >> 5) * 2 + 16 * i + j, ke - 1) * sk);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int k = k0 + (t >> 5) * 2 + 16 * i;
+        const uint32_t a = r < rows && k < ke ? q[2 * i] : 0U, b = r < rows && k + 1 < ke ? q[2 * i + 1] : 0U;
+        v[2 * i] = (a & 0xFFFFU) | (b << 16);      // row r, k and k + 1
+        v[2 * i + 1] = (a >> 16) | (b & 0xFFFF0000U);  // row r + 1
+      }
+    } else if constexpr (Mode == kStageConv8) {
+      // org: the receptive-field origin (oy, ox, pair) of this thread's row
+      const int k = k0 + (t & 3) * 8, kc = min(k, ke - 8);
+      const int tap = kc / cv.C, ch = kc - tap * cv.C, ky = tap / 3, kx = tap - ky * 3;
+      const int yi = org[0] + ky, xi = org[1] + kx;
+      const int yc = min(max(yi, 0), cv.H - 1), xc = min(max(xi, 0), cv.W - 1);
+      const uint4 q = *reinterpret_cast<const uint4*>(
+          cv.x + ((static_cast<long long>(org[2]) * cv.H + yc) * cv.W + xc) * cv.C + ch);
+      const bool in = k < ke && yi == yc && xi == xc;
+      v[0] = in ? q.x : 0U;
+      v[1] = in ? q.y : 0U;
+      v[2] = in ? q.z : 0U;
+      v[3] = in ? q.w : 0U;
+    } else {
+      const int k = k0 + (t & 31), kc = min(k, ke - 1);
+      uint16_t h[8];
+      int ky = 0, kx = 0, ch = 0;
+      if constexpr (Mode == kStageConv) {
+        const int tap = kc / cv.C;
+        ch = kc - tap * cv.C;
+        ky = tap / 3;
+        kx = tap - ky * 3;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if constexpr (Mode == kStageConv) {
+          const int yc = min(max(org[3 * i] + ky, 0), cv.H - 1), xc = min(max(org[3 * i + 1] + kx, 0), cv.W - 1);
+          if (cv.raw_prev != nullptr)
+            h[i] = (ch == 0 ? cv.raw_prev : cv.raw_cur)[org[3 * i + 2] * cv.raw_stride + yc * cv.W + xc];
+          else
+            h[i] = cv.x[((static_cast<long long>(org[3 * i + 2]) * cv.H + yc) * cv.W + xc) * cv.C + ch];
+        } else {
+          h[i] = p[min(row0 + (t >> 5) + 8 * i, rows - 1) * srow + kc * sk];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        bool in = k < ke && row0 + (t >> 5) + 8 * i < rows;
+        if constexpr (Mode == kStageConv) {
+          const int yi = org[3 * i] + ky, xi = org[3 * i + 1] + kx;
+          in = k < ke && yi >= 0 && yi < cv.H && xi >= 0 && xi < cv.W;
+          if (cv.raw_prev != nullptr) h[i] = raw_to_input(h[i], cv.inv_scale);
+        }
+        h[i] = in ? h[i] : static_cast<uint16_t>(0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = h[2 * i] | (static_cast<uint32_t>(h[2 * i + 1]) << 16);
+    }
+  }
+  __device__ inline void write(uint16_t (*lds)[LDK]) const {
+    const int t = static_cast<int>(threadIdx.x);
+    if constexpr (Mode == kStageRows8 || Mode == kStageConv8) {
+      *reinterpret_cast<uint4*>(&lds[t >> 2][(t & 3) * 8]) = make_uint4(v[0], v[1], v[2], v[3]);
+    } else if constexpr (Mode == kStageRows2) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<uint32_t*>(&lds[(t >> 4) + 16 * i][(t & 15) * 2]) = v[i];
+    } else if constexpr (Mode == kStageCols) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          *reinterpret_cast<uint32_t*>(&lds[(t & 31) * 2 + j][(t >> 5) * 2 + 16 * i]) = v[2 * i + j];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        lds[(t >> 5) + 8 * i][t & 31] = static_cast<uint16_t>((i & 1) != 0 ? v[i >> 1] >> 16 : v[i >> 1]);
+    }
+  }
+};
+
+template <int ModeA, int ModeB>
 __global__ void __launch_bounds__(256) gemm_kernel(Gemm g) {
   __shared__ __align__(16) uint16_t As[BM][LDK];
   __shared__ __align__(16) uint16_t Bs[BN][LDK];
@@ -152,80 +284,39 @@ __global__ void __launch_bounds__(256) gemm_kernel(Gemm g) {
   const int ke = min(g.K, kb + g.kchunk);
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
   const int li = lane & 15, lq = lane >> 4;
-  // This thread stages column `sc` of rows sr + kStageRows * i of both tiles.
-  const int sc = tid & (BK - 1), sr = tid >> 5;
-  const bool implicit = g.a == nullptr;
-  // Implicit im2col: the receptive-field origin of each staged row is fixed
-  // over the K loop (rows past M get an origin no tap reaches).
-  int oy[kRowsPerThread], ox[kRowsPerThread], ob[kRowsPerThread];
+  // im2col: the receptive-field origin of this thread's rows is fixed over
+  // the K loop (rows past M get an origin no tap reaches)
+  constexpr int kOrigins = ModeA == kStageConv ? 8 : 1;
+  int org[3 * kOrigins];
+  if constexpr (ModeA == kStageConv || ModeA == kStageConv8) {
 #pragma unroll
-  for (int i = 0; i < kRowsPerThread; ++i) {
-    oy[i] = -4;
-    ox[i] = -4;
-    ob[i] = 0;
-    const int m = m0 + sr + kStageRows * i;
-    if (implicit && m < g.M) {
-      const int xo = m % g.conv.Wo, t = m / g.conv.Wo;
-      oy[i] = 2 * (t % g.conv.Ho) - 1;
-      ox[i] = 2 * xo - 1;
-      ob[i] = t / g.conv.Ho;
+    for (int i = 0; i < kOrigins; ++i) {
+      const int m = m0 + (ModeA == kStageConv ? (tid >> 5) + 8 * i : tid >> 2);
+      org[3 * i] = org[3 * i + 1] = -4;
+      org[3 * i + 2] = 0;
+      if (m < g.M) {
+        const int xo = m % g.conv.Wo, t = m / g.conv.Wo;
+        org[3 * i] = 2 * (t % g.conv.Ho) - 1;
+        org[3 * i + 1] = 2 * xo - 1;
+        org[3 * i + 2] = t / g.conv.Ho;
+      }
     }
   }
   f32x4 acc[2][2];
   for (int i = 0; i < 2; ++i)
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0F, 0.0F, 0.0F, 0.0F};
-  // The staged values of one K step, all reads in flight together: an address
-  // past an edge is clamped and its value zeroed, since a guarded read would
-  // wait for the one before it.
-  uint16_t av[kRowsPerThread], bv[kRowsPerThread];
-  auto stage = [&](int k0) {
-    const int k = k0 + sc, kc = min(k, ke - 1);
-    int ky = 0, kx = 0, ch = 0;
-    if (implicit) {
-      const int tap = kc / g.conv.C;
-      ch = kc - tap * g.conv.C;
-      ky = tap / 3;
-      kx = tap - ky * 3;
-    }
-#pragma unroll
-    for (int i = 0; i < kRowsPerThread; ++i) {
-      const int r = sr + kStageRows * i;
-      const int m = min(m0 + r, g.M - 1), n = min(n0 + r, g.N - 1);
-      if (!implicit) {
-        av[i] = g.a[m * g.sam + kc * g.sak];
-      } else {
-        const int yi = min(max(oy[i] + ky, 0), g.conv.H - 1), xi = min(max(ox[i] + kx, 0), g.conv.W - 1);
-        if (g.conv.raw_prev != nullptr) {
-          const uint16_t* src = ch == 0 ? g.conv.raw_prev : g.conv.raw_cur;
-          av[i] = src[ob[i] * g.conv.raw_stride + yi * g.conv.W + xi];
-        } else {
-          av[i] = g.conv.x[((static_cast<long long>(ob[i]) * g.conv.H + yi) * g.conv.W + xi) * g.conv.C + ch];
-        }
-      }
-      bv[i] = g.b[kc * g.sbk + n * g.sbn];
-    }
-#pragma unroll
-    for (int i = 0; i < kRowsPerThread; ++i) {
-      const int r = sr + kStageRows * i;
-      bool in = k < ke && m0 + r < g.M;
-      if (implicit) {
-        const int yi = oy[i] + ky, xi = ox[i] + kx;
-        in = k < ke && yi >= 0 && yi < g.conv.H && xi >= 0 && xi < g.conv.W;
-        if (g.conv.raw_prev != nullptr) av[i] = raw_to_input(av[i], g.conv.inv_scale);
-      }
-      av[i] = in ? av[i] : static_cast<uint16_t>(0);
-      bv[i] = k < ke && n0 + r < g.N ? bv[i] : static_cast<uint16_t>(0);
-    }
-  };
-  stage(kb);
+  Stage<ModeA> sa;
+  Stage<ModeB> sb;
+  sa.read(g.a, g.sam, g.sak, m0, g.M, kb, ke, g.conv, org);
+  sb.read(g.b, g.sbn, g.sbk, n0, g.N, kb, ke, g.conv, org);
   for (int k0 = kb; k0 < ke; k0 += BK) {
-#pragma unroll
-    for (int i = 0; i < kRowsPerThread; ++i) {
-      As[sr + kStageRows * i][sc] = av[i];
-      Bs[sr + kStageRows * i][sc] = bv[i];
-    }
+    sa.write(As);
+    sb.write(Bs);
     __syncthreads();
-    if (k0 + BK < ke) stage(k0 + BK);  // the next step's reads run behind this step's MFMAs
+    if (k0 + BK < ke) {  // the next step's reads run behind this step's MFMAs
+      sa.read(g.a, g.sam, g.sak, m0, g.M, k0 + BK, ke, g.conv, org);
+      sb.read(g.b, g.sbn, g.sbk, n0, g.N, k0 + BK, ke, g.conv, org);
+    }
     {  // the staged 32 k as one 16x16x32 step
       s16x8 af[2], bf[2];
 #pragma unroll
@@ -284,7 +375,7 @@ __global__ void gemm_finish_kernel(Gemm g, int splits) {
 // columns 256 rows at a time in LDS (32 reads per thread in flight, the next
 // piece's reads issued before this one is added) and one thread per column
 // adds them.  A thread per column reading its rows itself took 175 us for
-// 1200 rows of 16 columns; this takes MEASURE_ROWSUM us.
+// 1200 rows of 16 columns; this takes 12 us.
 constexpr int kSumCols = 32, kSumRows = 256;
 struct RowSum {
   const float* x;
@@ -464,9 +555,7 @@ __global__ void input_kernel(const uint16_t* prev0, const uint16_t* cur0, long l
 // consecutive channels of one tap per thread as one word (2 channels: 4 bytes,
 // otherwise 8: 16 bytes), so a thread's index divisions are paid once per word.
 template <int Run>
-struct Channels {
-  uint16_t v[Run];
-} __attribute__((aligned(Run * 2)));
+using Channels = std::conditional_t<Run == 8, uint4, uint32_t>;
 template <int Run>
 __global__ void __launch_bounds__(256) im2col_kernel(const uint16_t* x, uint16_t* col, int batch, int H, int W, int C,
                                                      int Ho, int Wo) {
@@ -480,10 +569,10 @@ __global__ void __launch_bounds__(256) im2col_kernel(const uint16_t* x, uint16_t
     const int xo = static_cast<int>(m - t * Wo), b = static_cast<int>(t / static_cast<unsigned>(Ho));
     const int yo = static_cast<int>(t) - b * Ho;
     const int yi = 2 * yo - 1 + ky, xi = 2 * xo - 1 + kx;
-    Channels<Run> v{};
-    if (yi >= 0 && yi < H && xi >= 0 && xi < W)
-      v = *reinterpret_cast<const Channels<Run>*>(x + ((static_cast<size_t>(b) * H + yi) * W + xi) * C + c);
-    *reinterpret_cast<Channels<Run>*>(col + static_cast<size_t>(e) * Run) = v;
+    const int yc = min(max(yi, 0), H - 1), xc = min(max(xi, 0), W - 1);
+    Channels<Run> v = *reinterpret_cast<const Channels<Run>*>(x + ((static_cast<size_t>(b) * H + yc) * W + xc) * C + c);
+    if (yi != yc || xi != xc) v = Channels<Run>{};
+    reinterpret_cast<Channels<Run>*>(col)[e] = v;
   }
 }
 
@@ -515,7 +604,7 @@ __global__ void __launch_bounds__(256) col2im_kernel(const float* dcol, const ui
         const int tap = in[i][j] ? ky * 3 + kx : 0;
         v[i][j] = *reinterpret_cast<const float4*>(dcol + (m * 9 + tap) * C + c);
       }
-    const Channels<4> act = *reinterpret_cast<const Channels<4>*>(xin + static_cast<size_t>(e) * 4);
+    const uint2 act = reinterpret_cast<const uint2*>(xin)[e];
     float s[4] = {0.0F, 0.0F, 0.0F, 0.0F};
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -527,10 +616,11 @@ __global__ void __launch_bounds__(256) col2im_kernel(const float* dcol, const ui
         s[2] += v[i][j].z;
         s[3] += v[i][j].w;
       }
-    Channels<4> out;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) out.v[q] = to_bf16(from_bf16(act.v[q]) > 0.0F ? s[q] : 0.0F);
-    *reinterpret_cast<Channels<4>*>(dx + static_cast<size_t>(e) * 4) = out;
+    auto masked = [](uint32_t a, float v) -> uint32_t {
+      return to_bf16(from_bf16(static_cast<uint16_t>(a)) > 0.0F ? v : 0.0F);
+    };
+    reinterpret_cast<uint2*>(dx)[e] = make_uint2(masked(act.x, s[0]) | (masked(act.x >> 16, s[1]) << 16),
+                                                 masked(act.y, s[2]) | (masked(act.y >> 16, s[3]) << 16));
   }
 }
 
@@ -661,6 +751,59 @@ T* nalloc(size_t count) {
   return static_cast<T*>(p);
 }
 
+// The staging mode of an operand with row stride srow and k stride sk over
+// `rows` rows and K (a kchunk is a multiple of 32, so K decides the k edges): the widest
+// read that the order, strides and alignment allow.
+int stage_mode(const uint16_t* p, long long srow, long long sk, int rows, int K) {
+  const auto at = reinterpret_cast<uintptr_t>(p);
+  if (sk == 1 && srow % 8 == 0 && K % 8 == 0 && (at & 15U) == 0U) return kStageRows8;
+  if (sk == 1 && srow % 2 == 0 && K % 2 == 0 && (at & 3U) == 0U) return kStageRows2;
+  if (srow == 1 && sk % 2 == 0 && rows % 2 == 0 && (at & 3U) == 0U) return kStageCols;
+  return kStageScalar;
+}
+
+template <int ModeA>
+void launch_gemm_b(const Gemm& g, int mode_b, dim3 grid, hipStream_t s) {
+  switch (mode_b) {
+    case kStageRows8:
+      hipLaunchKernelGGL((gemm_kernel<ModeA, kStageRows8>), grid, dim3(256), 0, s, g);
+      break;
+    case kStageRows2:
+      hipLaunchKernelGGL((gemm_kernel<ModeA, kStageRows2>), grid, dim3(256), 0, s, g);
+      break;
+    case kStageCols:
+      hipLaunchKernelGGL((gemm_kernel<ModeA, kStageCols>), grid, dim3(256), 0, s, g);
+      break;
+    default:
+      hipLaunchKernelGGL((gemm_kernel<ModeA, kStageScalar>), grid, dim3(256), 0, s, g);
+      break;
+  }
+}
+
+void launch_gemm(const Gemm& g, dim3 grid, hipStream_t s) {
+  const int mode_b = stage_mode(g.b, g.sbn, g.sbk, g.N, g.K);
+  if (g.a == nullptr) {
+    const bool vec = g.conv.raw_prev == nullptr && g.conv.C % 8 == 0 && (reinterpret_cast<uintptr_t>(g.conv.x) & 15U) == 0U;
+    if (vec) launch_gemm_b<kStageConv8>(g, mode_b, grid, s);
+    else launch_gemm_b<kStageConv>(g, mode_b, grid, s);
+    return;
+  }
+  switch (stage_mode(g.a, g.sam, g.sak, g.M, g.K)) {
+    case kStageRows8:
+      launch_gemm_b<kStageRows8>(g, mode_b, grid, s);
+      break;
+    case kStageRows2:
+      launch_gemm_b<kStageRows2>(g, mode_b, grid, s);
+      break;
+    case kStageCols:
+      launch_gemm_b<kStageCols>(g, mode_b, grid, s);
+      break;
+    default:
+      launch_gemm_b<kStageScalar>(g, mode_b, grid, s);
+      break;
+  }
+}
+
 void gemm(kf_posenet* net, hipStream_t s, Gemm g) {
   const int tm = (g.M + BM - 1) / BM, tn = (g.N + BN - 1) / BN;
   const int tiles = tm * tn;
@@ -697,7 +840,7 @@ void gemm(kf_posenet* net, hipStream_t s, Gemm g) {
   g.kchunk = ((g.K + splits - 1) / splits + BK - 1) / BK * BK;
   splits = (g.K + g.kchunk - 1) / g.kchunk;
   g.partial = splits > 1 ? net->partial : nullptr;
-  hipLaunchKernelGGL(gemm_kernel, dim3(tm, tn, splits), dim3(256), 0, s, g);
+  launch_gemm(g, dim3(tm, tn, splits), s);
   if (splits > 1) {
     const long long total = static_cast<long long>(g.M) * g.N;
     // few outputs with many splits: staged; otherwise a thread per output
