@@ -558,6 +558,7 @@ kf_status kf_create(const kf_config* cfg, kf_context** out) {
       ctx->hash_table = dalloc<unsigned long long>(ctx->buckets);
       ctx->hash_stamp = dalloc<uint32_t>(ctx->buckets);
       ctx->block_of_slot = dalloc<uint32_t>(ctx->capacity);
+      ctx->slot_of_block = dalloc<uint32_t>(slot_index_entries(ctx->grid));
       ctx->work = dalloc<uint32_t>(ctx->capacity);
       ctx->sparse = dalloc<uint32_t>(8);
     } else {
@@ -611,7 +612,10 @@ kf_status kf_create(const kf_config* cfg, kf_context** out) {
       KF_HIP(hipMemsetAsync(ctx->part_bits, 0, ctx->part_words * 4, ctx->stream));
       if (c.storage == KF_STORAGE_HASHED) {
         const BlockMap cm = coarse_map(ctx->grid);
-        ctx->coarse_bits = dalloc<uint32_t>((static_cast<size_t>(cm.bx) * cm.by * cm.bz + 31) / 32);
+        const size_t ncells = static_cast<size_t>(cm.bx) * cm.by * cm.bz;
+        ctx->coarse = dalloc<uint8_t>(ncells);
+        ctx->coarse_xy = dalloc<uint8_t>(ncells);
+        ctx->coarse_busy = dalloc<unsigned long long>(static_cast<size_t>((cm.bx + 63) / 64) * cm.by * cm.bz);
         const size_t nb = static_cast<size_t>(bm.bx) * bm.by * bm.bz;
         ctx->nbr_obs = dalloc<uint32_t>(nb);
         KF_HIP(hipMemsetAsync(ctx->nbr_obs, 0, nb * 4, ctx->stream));
@@ -683,7 +687,9 @@ void kf_destroy(kf_context* ctx) {
   dfree(ctx->part_bits);
   dfree(ctx->free_bits);
   dfree(ctx->class_bits);
-  dfree(ctx->coarse_bits);
+  dfree(ctx->coarse);
+  dfree(ctx->coarse_xy);
+  dfree(ctx->coarse_busy);
   dfree(ctx->nbr_obs);
   dfree(ctx->counters);
   dfree(ctx->fused);
@@ -696,6 +702,7 @@ void kf_destroy(kf_context* ctx) {
   dfree(ctx->hash_table);
   dfree(ctx->hash_stamp);
   dfree(ctx->block_of_slot);
+  dfree(ctx->slot_of_block);
   dfree(ctx->work);
   dfree(ctx->sparse);
   for (auto& b : ctx->mesh_scratch) dfree(b.p);

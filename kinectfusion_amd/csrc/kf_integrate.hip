@@ -777,31 +777,91 @@ __global__ void __launch_bounds__(64) skip_map_rows_kernel(const uint32_t* __res
   class_bits[2 * t + 1] = class_word(sk >> 16, fr >> 16);
 }
 
-// coarse bit of a cell of 4^3 blocks = every block of it (inside the grid)
-// is a skip block.  One thread per cell; a wave's 64 consecutive cells form
-// two words.
-__global__ void __launch_bounds__(256) coarse_skip_kernel(const uint32_t* __restrict__ skip,
-                                                           uint32_t* __restrict__ coarse, BlockMap bm, BlockMap cm,
-                                                           int ncells) {
-  const int c = static_cast<int>(blockIdx.x * 256 + threadIdx.x);
-  bool all = false;
-  if (c < ncells) {
-    const int cx = c % cm.bx, cy = (c / cm.bx) % cm.by, cz = c / (cm.bx * cm.by);
-    all = true;
-    for (int z = cz * 4; z < min(cz * 4 + 4, bm.bz) && all; ++z)
-      for (int y = cy * 4; y < min(cy * 4 + 4, bm.by) && all; ++y)
-        for (int x = cx * 4; x < min(cx * 4 + 4, bm.bx); ++x)
-          if (!bm.bit(skip, bm.flat(x, y, z))) {
-            all = false;
-            break;
-          }
-  }
-  const unsigned long long m = __ballot(all);
+// Distances of the raycaster's cells of 4^3 blocks from the nearest cell that
+// is not all skip blocks, in cells and the maximum norm, 0 for such a cell and
+// at most kCoarseReach + 1: every cell nearer than that is all skip blocks, so
+// a ray crosses them all at once.  The maximum norm separates: the distance
+// along x, then over y the least max(|dy|, that), then over z.
+//
+// 1. One wave per 64 cells of a row: bit x of a row's words, a cell that is
+// not all skip blocks.  aligned: rows of blocks are whole words (a cell's four
+// blocks are four bits of one word, its 16 rows read together).
+__global__ void __launch_bounds__(256) coarse_busy_kernel(const uint32_t* __restrict__ skip,
+                                                           unsigned long long* __restrict__ busy, BlockMap bm,
+                                                           BlockMap cm, int words, bool aligned) {
   const int lane = threadIdx.x & 63;
-  const int word0 = (blockIdx.x * 256 + (threadIdx.x & ~63)) >> 5;
-  const int nwords = (ncells + 31) >> 5;
-  if (lane == 0 && word0 < nwords) coarse[word0] = static_cast<uint32_t>(m);
-  if (lane == 32 && word0 + 1 < nwords) coarse[word0 + 1] = static_cast<uint32_t>(m >> 32);
+  const int w = static_cast<int>(blockIdx.x * 4U + (threadIdx.x >> 6));
+  if (w >= words * cm.by * cm.bz) return;
+  const int row = w / words, cx = (w - row * words) * 64 + lane, cy = row % cm.by, cz = row / cm.by;
+  bool all = true;
+  if (cx < cm.bx) {
+    if (aligned) {
+      uint32_t v[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        // a row past the grid repeats the last one
+        const int y = min(cy * 4 + (k & 3), bm.by - 1), z = min(cz * 4 + (k >> 2), bm.bz - 1);
+        v[k] = skip[bm.flat(cx * 4, y, z) >> 5];
+      }
+      uint32_t m = 0xFFFFFFFFU;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) m &= v[k];
+      all = ((m >> ((cx * 4) & 31)) & 0xFU) == 0xFU;
+    } else {
+      for (int z = cz * 4; z < min(cz * 4 + 4, bm.bz) && all; ++z)
+        for (int y = cy * 4; y < min(cy * 4 + 4, bm.by) && all; ++y)
+          for (int x = cx * 4; x < min(cx * 4 + 4, bm.bx); ++x)
+            if (!bm.bit(skip, bm.flat(x, y, z))) {
+              all = false;
+              break;
+            }
+    }
+  }
+  const unsigned long long m = __ballot(!all);
+  if (lane == 0) busy[w] = m;
+}
+
+// Distance along x from cell x to the nearest set bit of its row, capped.
+__device__ inline int row_distance(const unsigned long long* __restrict__ row, int words, int x) {
+  const int w = x >> 6, b = x & 63;
+  const unsigned long long self = row[w];
+  const unsigned long long prev = w > 0 ? row[w - 1] : 0ULL, next = w + 1 < words ? row[w + 1] : 0ULL;
+  // bits x, x + 1, ... from bit 0 up; bits x, x - 1, ... from bit 63 down
+  const unsigned long long up = (self >> b) | (b != 0 ? next << (64 - b) : 0ULL);
+  const unsigned long long down = (self << (63 - b)) | (b != 63 ? prev >> (b + 1) : 0ULL);
+  const int right = up != 0ULL ? __builtin_ctzll(up) : 64, left = down != 0ULL ? __builtin_clzll(down) : 64;
+  return min(right, left);
+}
+
+// 2. over x and y.
+__global__ void __launch_bounds__(256) coarse_distance_xy_kernel(const unsigned long long* __restrict__ busy,
+                                                                  uint8_t* __restrict__ out, BlockMap cm, int words,
+                                                                  int ncells) {
+  const int c = static_cast<int>(blockIdx.x * 256 + threadIdx.x);
+  if (c >= ncells) return;
+  const int x = c % cm.bx, y = (c / cm.bx) % cm.by, z = c / (cm.bx * cm.by);
+  int d = kCoarseReach + 1;
+#pragma unroll 8
+  for (int dy = -kCoarseReach; dy <= kCoarseReach; ++dy) {
+    const int yy = min(max(y + dy, 0), cm.by - 1);  // a clamped row is no nearer than it is
+    d = min(d, max(abs(yy - y), row_distance(busy + static_cast<size_t>(z * cm.by + yy) * words, words, x)));
+  }
+  out[c] = static_cast<uint8_t>(d);
+}
+
+// 3. over z.
+__global__ void __launch_bounds__(256) coarse_distance_z_kernel(const uint8_t* __restrict__ xy,
+                                                                 uint8_t* __restrict__ out, BlockMap cm, int ncells) {
+  const int c = static_cast<int>(blockIdx.x * 256 + threadIdx.x);
+  if (c >= ncells) return;
+  const int slice = cm.bx * cm.by, z = c / slice;
+  int d = kCoarseReach + 1;
+#pragma unroll
+  for (int dz = -kCoarseReach; dz <= kCoarseReach; ++dz) {
+    const int zz = min(max(z + dz, 0), cm.bz - 1);
+    d = min(d, max(abs(zz - z), static_cast<int>(xy[c + (zz - z) * slice])));
+  }
+  out[c] = static_cast<uint8_t>(d);
 }
 
 // Neighbour masks of the non-skip blocks: bit (dz + 1) * 9 + (dy + 1) * 3 +
@@ -1006,6 +1066,7 @@ __global__ void __launch_bounds__(256) assign_slots_kernel(HashView hv, const ui
       if (s < capacity) {
         slot = s;
         block_of_slot[s] = key;
+        hv.slots[key] = s;
       } else {
         slot = kNoSlot;
         atomicAdd(&sp[4], 1U);
@@ -1104,12 +1165,16 @@ __global__ void __launch_bounds__(256) integrate_blocks_kernel(Grid g, FramePara
   }
 }
 
-__global__ void fill_table_kernel(unsigned long long* table, uint32_t* stamp, size_t buckets, uint32_t* sp) {
+__global__ void fill_table_kernel(unsigned long long* table, uint32_t* stamp, size_t buckets, uint32_t* sp,
+                                  uint32_t* slots, size_t nslots) {
   for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < buckets;
        i += static_cast<size_t>(gridDim.x) * blockDim.x) {
     table[i] = kHashEmpty;
     stamp[i] = 0U;
   }
+  for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < nslots;
+       i += static_cast<size_t>(gridDim.x) * blockDim.x)
+    slots[i] = kNoSlot;
   if (blockIdx.x == 0 && threadIdx.x < 8) sp[threadIdx.x] = 0U;
 }
 
@@ -1214,7 +1279,7 @@ __global__ void expand_hashed_kernel(Grid g, HashView hv, const typename VoxelIO
        i += static_cast<size_t>(gridDim.x) * blockDim.x) {
     const int x = static_cast<int>(i % g.nx), y = static_cast<int>((i / g.nx) % g.ny);
     const int z = static_cast<int>(i / (static_cast<size_t>(g.nx) * g.ny));
-    const uint32_t slot = hv.find(hv.key_of(x, y, z));
+    const uint32_t slot = hv.slots[hv.key_of(x, y, z)];
     const size_t pi = static_cast<size_t>(slot) * kBlockVoxels + intra_of(x, y, z);
     out[i] = slot == kNoSlot ? VoxelIO<Kind>::fresh() : pool[pi];
     if (cout_ != nullptr) cout_[i] = slot == kNoSlot ? make_float4(0.0F, 0.0F, 0.0F, 0.0F) : cpool[pi];
@@ -1251,7 +1316,7 @@ bool hashed(const kf_context* ctx) { return ctx->cfg.storage == KF_STORAGE_HASHE
 
 HashView hash_view(const kf_context* ctx) {
   const BlockMap bm = block_map(ctx->grid);
-  return HashView{ctx->hash_table, static_cast<uint32_t>(ctx->buckets - 1), bm.bx, bm.by, bm.bz};
+  return HashView{ctx->hash_table, static_cast<uint32_t>(ctx->buckets - 1), bm.bx, bm.by, bm.bz, ctx->slot_of_block};
 }
 
 void launch_expand_hashed(kf_context* ctx, void* voxels, float4* colors) {
@@ -1277,7 +1342,7 @@ void launch_expand_hashed(kf_context* ctx, void* voxels, float4* colors) {
 
 void launch_fill_pool(kf_context* ctx) {
   hipLaunchKernelGGL(fill_table_kernel, dim3(2048), dim3(256), 0, ctx->stream, ctx->hash_table, ctx->hash_stamp,
-                     ctx->buckets, ctx->sparse);
+                     ctx->buckets, ctx->sparse, ctx->slot_of_block, slot_index_entries(ctx->grid));
   KF_HIP(hipGetLastError());
 }
 
@@ -1321,11 +1386,15 @@ void launch_skip_map(kf_context* ctx, bool end_frame) {
                        end_frame ? ctx->icp : nullptr,
                        ctx->trajectory, keep);
   }
-  if (ctx->coarse_bits != nullptr) {
+  if (ctx->coarse != nullptr) {
     const BlockMap cm = coarse_map(ctx->grid);
-    const int ncells = cm.bx * cm.by * cm.bz;
-    hipLaunchKernelGGL(coarse_skip_kernel, dim3((ncells + 255) / 256), dim3(256), 0, ctx->stream, ctx->skip_bits,
-                       ctx->coarse_bits, bm, cm, ncells);
+    const int ncells = cm.bx * cm.by * cm.bz, words = (cm.bx + 63) / 64, rows = cm.by * cm.bz;
+    hipLaunchKernelGGL(coarse_busy_kernel, dim3((words * rows + 3) / 4), dim3(256), 0, ctx->stream, ctx->skip_bits,
+                       ctx->coarse_busy, bm, cm, words, bm.bx % 32 == 0);
+    hipLaunchKernelGGL(coarse_distance_xy_kernel, dim3((ncells + 255) / 256), dim3(256), 0, ctx->stream,
+                       ctx->coarse_busy, ctx->coarse_xy, cm, words, ncells);
+    hipLaunchKernelGGL(coarse_distance_z_kernel, dim3((ncells + 255) / 256), dim3(256), 0, ctx->stream, ctx->coarse_xy,
+                       ctx->coarse, cm, ncells);
   }
   if (ctx->nbr_obs != nullptr)
     hipLaunchKernelGGL(neighbour_mask_kernel, dim3((nblocks + 255) / 256), dim3(256), 0, ctx->stream, ctx->obs_bits,

@@ -235,25 +235,14 @@ struct HashView {
   unsigned long long* table;  // (key << 32) | slot, kHashEmpty when free
   uint32_t mask;              // buckets - 1 (buckets a power of two)
   int bx, by, bz;             // blocks per axis
+  // pool slot of every block of the grid by key, kNoSlot where none (and one
+  // spare entry): what readers use, one read instead of a probe and its walk
+  uint32_t* slots;
   __host__ __device__ inline uint32_t bucket(uint32_t key) const {
     return static_cast<uint32_t>((static_cast<unsigned long long>(key) * 0x9E3779B97F4A7C15ULL) >> 32) & mask;
   }
   __host__ __device__ inline uint32_t key_of(int x, int y, int z) const {
     return static_cast<uint32_t>(((z >> 3) * by + (y >> 3)) * bx + (x >> 3));
-  }
-  // Pool slot of a block, or kNoSlot when the block holds no voxels.
-  __device__ inline uint32_t find(uint32_t key) const {
-    uint32_t h = bucket(key);
-    for (uint32_t probe = 0; probe <= mask; ++probe) {
-      const unsigned long long e = table[h];
-      if (e == kHashEmpty) return kNoSlot;
-      if (static_cast<uint32_t>(e >> 32) == key) {
-        const uint32_t slot = static_cast<uint32_t>(e);
-        return slot == kPendingSlot ? kNoSlot : slot;
-      }
-      h = (h + 1) & mask;
-    }
-    return kNoSlot;
   }
 };
 
@@ -461,9 +450,13 @@ struct kf_context {
   // both classes of block b in one word for the raycaster: bit 2 (b % 16) of
   // word b / 16 is its skip bit, the bit above it its free bit
   uint32_t* class_bits = nullptr;
-  // hashed storage: one bit per cell of 4^3 blocks, set when every block of
-  // the cell is a skip block (the raycaster steps over such a cell at once)
-  uint32_t* coarse_bits = nullptr;
+  // hashed storage: per cell of 4^3 blocks, its distance (maximum norm, in
+  // cells) from the nearest cell that is not all skip blocks, 0 for such a
+  // cell (the raycaster crosses the cells nearer than that at once); and the
+  // two passes before it, bit rows of such cells and distances over x and y
+  uint8_t* coarse = nullptr;
+  unsigned long long* coarse_busy = nullptr;
+  uint8_t* coarse_xy = nullptr;
   // hashed storage: per non-skip block, bit (dz + 1) * 9 + (dy + 1) * 3 +
   // (dx + 1) set when the block at that offset holds an observed voxel
   uint32_t* nbr_obs = nullptr;
@@ -492,6 +485,7 @@ struct kf_context {
   unsigned long long* hash_table = nullptr;
   uint32_t* hash_stamp = nullptr;     // frame id of the last visit, per bucket
   uint32_t* block_of_slot = nullptr;  // block key of every pool slot
+  uint32_t* slot_of_block = nullptr;  // pool slot of every block of the grid (kNoSlot: none), plus a spare entry
   uint32_t* work = nullptr;           // pool slots to integrate this frame
   // [0] slots requested (allocated + overflowing), [1] work count,
   // [2] table entries, [3] frame id, [4] overflowing requests
@@ -588,7 +582,13 @@ struct BlockMap {
 inline BlockMap block_map(const Grid& g) {
   return BlockMap{(g.nx + 7) / 8, (g.ny + 7) / 8, (g.nz + 7) / 8};
 }
-// cells of 4^3 blocks (32^3 voxels)
+inline size_t slot_index_entries(const Grid& g) {
+  const BlockMap b = block_map(g);
+  return static_cast<size_t>(b.bx) * b.by * b.bz + 1;
+}
+// cells of 4^3 blocks (32^3 voxels), and the largest distance looked for among
+// them
+constexpr int kCoarseReach = 15;
 inline BlockMap coarse_map(const Grid& g) {
   const BlockMap b = block_map(g);
   return BlockMap{(b.bx + 3) / 4, (b.by + 3) / 4, (b.bz + 3) / 4};

@@ -47,7 +47,7 @@ __device__ inline void raycast_pixel(const Sampler<Kind, Store>& vol, const RayP
                                      int y, float4* __restrict__ pts, float4* __restrict__ nrm,
                                      uint32_t* __restrict__ col, const uint32_t* __restrict__ class_bits,
                                      const uint32_t* __restrict__ nbr_obs, const BlockMap& bm,
-                                     const uint32_t* __restrict__ coarse_bits, const BlockMap& cm) {
+                                     const uint8_t* __restrict__ coarse, const BlockMap& cm) {
   const size_t i = static_cast<size_t>(y) * rp.w + x;
   // RaycastOptions::seed_from_previous (raycasting.hpp:122-131): start just
   // in front of the surface this pixel found in the previous raycast into
@@ -141,10 +141,10 @@ __device__ inline void raycast_pixel(const Sampler<Kind, Store>& vol, const RayP
     // only unobserved blocks is a sample without TSDF as well, decided
     // without a read.
     //
-    // coarse_bits (optional) marks cells of 4^3 blocks that are all skip
-    // blocks: a skip block in such a cell is stepped over the whole cell's
-    // safe interior at once, so a ray crossing unobserved space reads one
-    // class per 32^3-voxel cell instead of one per block.
+    // coarse (hashed store) holds, per cell of 4^3 blocks, its distance from
+    // the nearest cell that is not all skip blocks: a skip block in a cell at
+    // distance d > 0 is stepped over with all cells nearer than d at once, so
+    // a ray crossing unobserved space reads a few classes, not one per block.
     constexpr float kSafe = 0.05F;
     // len <= max_depth is len < depth_lim: a run of steps lasts while len < min(exit, depth_lim)
     const float depth_lim = nextafterf(rp.max_depth, __builtin_inff());
@@ -164,110 +164,162 @@ __device__ inline void raycast_pixel(const Sampler<Kind, Store>& vol, const RayP
         return advance_to(l, step, lim, last);
       }
     };
-    // Empty blocks pay where a sample costs a hash probe before its corner
-    // reads; a direct store reads the corners at once, and the extra class
-    // word per block was slower there (-1.4 % headline frame rate).
-    constexpr bool kEmptyClass = !Store::kDirect;
     float enter = 0.0F, exit = -1.0F;
-    while (len <= rp.max_depth) {
-      if (len > len_stop) break;
-      const V3 point = add3(pose.t, scale3(dir, len));
-      const V3 gc = vol.grid_coords(point);
-      if (vol.contains(gc)) {
-        // the block of this sample, classified exactly as the sampler sees it
-        const int gx = static_cast<int>(gc.x) >> 3, gy = static_cast<int>(gc.y) >> 3, gz = static_cast<int>(gc.z) >> 3;
-        const int fb = bm.flat(gx, gy, gz);
-        if (fb != cur_blk) {
-          // the block's skip and free bits: one word, one read
-          cur_blk = fb;
-          const uint32_t cls = class_bits[fb >> 4] >> (2U * static_cast<uint32_t>(fb & 15));
-          // a skip block holds no observed voxel, a free block only
-          // observed ones: the three bits give four exclusive classes
-          const uint32_t skip = cls & 1U, fre = (cls >> 1) & 1U;
-          if constexpr (kEmptyClass) cur_nbr = nbr_obs[fb];
-          const uint32_t seen = kEmptyClass ? (cur_nbr >> 13) & 1U : 1U;
-          bool coarse = false;
-          if (coarse_bits != nullptr) {
-            const int cf = cm.flat(gx >> 2, gy >> 2, gz >> 2);
-            coarse = ((coarse_bits[cf >> 5] >> (cf & 31)) & 1U) != 0U;
+    if constexpr (Store::kDirect) {
+      while (len <= rp.max_depth) {
+        if (len > len_stop) break;
+        const V3 point = add3(pose.t, scale3(dir, len));
+        const V3 gc = vol.grid_coords(point);
+        if (vol.contains(gc)) {
+          // the block of this sample, classified exactly as the sampler sees it
+          const int gx = static_cast<int>(gc.x) >> 3, gy = static_cast<int>(gc.y) >> 3, gz = static_cast<int>(gc.z) >> 3;
+          const int fb = bm.flat(gx, gy, gz);
+          if (fb != cur_blk) {
+            // the block's skip and free bits: one word, one read
+            cur_blk = fb;
+            const uint32_t cls = class_bits[fb >> 4] >> (2U * static_cast<uint32_t>(fb & 15));
+            cur_skip = (cls & 1U) != 0U;
+            cur_free = (cls & 2U) != 0U;
+            if (cur_skip || cur_free) {
+              const V3 go = vol.grid_coords(pose.t), gd = scale3(dir, vol.inv_voxel);
+              enter = -3.0e38F;
+              exit = 3.0e38F;
+              box_span(gx << 3, 8, go.x, gd.x, vol.g.nx, kSafe, enter, exit);
+              box_span(gy << 3, 8, go.y, gd.y, vol.g.ny, kSafe, enter, exit);
+              box_span(gz << 3, 8, go.z, gd.z, vol.g.nz, kSafe, enter, exit);
+            }
           }
-          cur_skip = skip != 0U;
-          cur_free = fre != 0U;
-          cur_empty = (skip | seen) == 0U;
-          if (cur_skip || cur_free || cur_empty) {
-            const V3 go = vol.grid_coords(pose.t), gd = scale3(dir, vol.inv_voxel);
-            const float margin = cur_empty ? 0.5F + kSafe : kSafe;
-            const int size = coarse ? 32 : 8, sh3 = coarse ? 5 : 3;
-            enter = -3.0e38F;
-            exit = 3.0e38F;
-            box_span((gx << 3) >> sh3 << sh3, size, go.x, gd.x, vol.g.nx, margin, enter, exit);
-            box_span((gy << 3) >> sh3 << sh3, size, go.y, gd.y, vol.g.ny, margin, enter, exit);
-            box_span((gz << 3) >> sh3 << sh3, size, go.z, gd.z, vol.g.nz, margin, enter, exit);
-          }
-        }
-        if (cur_skip) {  // no corner is observed: no TSDF
-          have_prev = false;
-          len += base_step;
-          if (len >= enter) len = run_to(len, base_step, fminf(exit, depth_lim), unused_last);
-          continue;
-        }
-        if (cur_free) {  // every corner reads exactly 1: no read, free steps
-          if (have_prev && prev_t < 0.0F) break;
-          have_prev = true;
-          prev_t = 1.0F;
-          float last = len;
-          len += free_step;
-          if (len >= enter) len = run_to(len, free_step, fminf(exit, depth_lim), last);
-          prev_p = add3(pose.t, scale3(dir, last));  // the last free sample's point
-          continue;
-        }
-        if (cur_empty && len >= enter && len < exit) {  // a stencil inside an empty block: no TSDF
-          have_prev = false;
-          len += base_step;
-          len = run_to(len, base_step, fminf(exit, depth_lim), unused_last);
-          continue;
-        }
-        if (cur_empty) {
-          // the stencil's corners c0 and c0 + 1 per axis (c0 = floor(g - 0.5),
-          // as the sampler computes it) lie in the blocks -1, 0 or +1 from
-          // this one; bit (dz + 1) * 9 + (dy + 1) * 3 + (dx + 1) of `reach`
-          // marks each block the stencil reaches
-          auto axis = [](float g, int b) {
-            const int c0 = static_cast<int>(floorf(g - 0.5F));
-            return (1U << ((c0 >> 3) - b + 1)) | (1U << (((c0 + 1) >> 3) - b + 1));
-          };
-          const uint32_t xs = axis(gc.x, gx), ys = axis(gc.y, gy), zs = axis(gc.z, gz);
-          const uint32_t yx = ((ys & 1U) != 0U ? xs : 0U) | ((ys & 2U) != 0U ? xs << 3 : 0U) |
-                              ((ys & 4U) != 0U ? xs << 6 : 0U);
-          const uint32_t reach = ((zs & 1U) != 0U ? yx : 0U) | ((zs & 2U) != 0U ? yx << 9 : 0U) |
-                                 ((zs & 4U) != 0U ? yx << 18 : 0U);
-          if ((reach & cur_nbr) == 0U) {  // no observed corner: no TSDF
+          if (cur_skip) {  // no corner is observed: no TSDF
             have_prev = false;
             len += base_step;
+            if (len >= enter) len = run_to(len, base_step, fminf(exit, depth_lim), unused_last);
+            continue;
+          }
+          if (cur_free) {  // every corner reads exactly 1: no read, free steps
+            if (have_prev && prev_t < 0.0F) break;
+            have_prev = true;
+            prev_t = 1.0F;
+            float last = len;
+            len += free_step;
+            if (len >= enter) len = run_to(len, free_step, fminf(exit, depth_lim), last);
+            prev_p = add3(pose.t, scale3(dir, last));  // the last free sample's point
             continue;
           }
         }
+        float t;
+        if (!vol.tsdf(point, rp.require_all != 0, t, slots)) {
+          have_prev = false;
+          len += base_step;
+          continue;
+        }
+        if (have_prev && prev_t > 0.0F && t <= 0.0F) {
+          const float gap = prev_t - t;
+          const float alpha = gap != 0.0F ? prev_t / gap : 0.0F;
+          surface = add3(prev_p, scale3(sub3(point, prev_p), alpha));
+          hit = true;
+          break;
+        }
+        if (have_prev && prev_t < 0.0F && t > 0.0F) break;
+        have_prev = true;
+        prev_t = t;
+        prev_p = point;
+        const float pre = t * vol.g.trunc * rp.step_scale;
+        const float step = fmax_ref(base_step, pre);
+        len += t > 0.0F ? step : base_step;
       }
-      float t;
-      if (!vol.tsdf(point, rp.require_all != 0, t, slots)) {
-        have_prev = false;
-        len += base_step;
-        continue;
+    } else {
+      // A hashed store's samples cost two rounds of reads, and its rays cross
+      // long stretches without any.  Every kind of known sample takes one piece
+      // of code (a wave runs each piece that any of its lanes needs): the run's
+      // step, its end and whether its samples read 1, then one advance.
+      while (len <= rp.max_depth && len <= len_stop) {
+        const V3 point = add3(pose.t, scale3(dir, len));
+        const V3 gc = vol.grid_coords(point);
+        bool known = true, ones = false;  // outside the grid: no TSDF
+        float lim = -1.0F;
+        if (vol.contains(gc)) {
+          const int gx = static_cast<int>(gc.x) >> 3, gy = static_cast<int>(gc.y) >> 3, gz = static_cast<int>(gc.z) >> 3;
+          const int fb = bm.flat(gx, gy, gz);
+          if (fb != cur_blk) {
+            cur_blk = fb;
+            const uint32_t cls = class_bits[fb >> 4] >> (2U * static_cast<uint32_t>(fb & 15));
+            const int reach = coarse[cm.flat(gx >> 2, gy >> 2, gz >> 2)];
+            cur_skip = (cls & 1U) != 0U;
+            cur_free = (cls & 2U) != 0U;
+            cur_nbr = 0U;
+            if (!cur_skip) cur_nbr = nbr_obs[fb];
+            cur_empty = !cur_skip && ((cur_nbr >> 13) & 1U) == 0U;
+            if (cur_skip || cur_free || cur_empty) {
+              const V3 go = vol.grid_coords(pose.t), gd = scale3(dir, vol.inv_voxel);
+              const float margin = cur_empty ? 0.5F + kSafe : kSafe;
+              // the block, or the cells nearer than the nearest busy one
+              const int sh = reach > 0 ? 2 : 0, r = max(reach - 1, 0), size = (2 * r + 1) << (3 + sh);
+              enter = -3.0e38F;
+              exit = 3.0e38F;
+              box_span(((gx >> sh) - r) << (3 + sh), size, go.x, gd.x, vol.g.nx, margin, enter, exit);
+              box_span(((gy >> sh) - r) << (3 + sh), size, go.y, gd.y, vol.g.ny, margin, enter, exit);
+              box_span(((gz >> sh) - r) << (3 + sh), size, go.z, gd.z, vol.g.nz, margin, enter, exit);
+            }
+          }
+          if (cur_empty) {
+            // deep inside an empty block no corner is observed; elsewhere the
+            // stencil's corners c0 and c0 + 1 per axis (c0 = floor(g - 0.5),
+            // as the sampler computes it) lie in the blocks -1, 0 or +1 from
+            // this one; bit (dz + 1) * 9 + (dy + 1) * 3 + (dx + 1) of `reach`
+            // marks each block the stencil reaches
+            if (len >= enter && len < exit) {
+              lim = exit;
+            } else {
+              auto axis = [](float g, int b) {
+                const int c0 = static_cast<int>(floorf(g - 0.5F));
+                return (1U << ((c0 >> 3) - b + 1)) | (1U << (((c0 + 1) >> 3) - b + 1));
+              };
+              const uint32_t xs = axis(gc.x, gx), ys = axis(gc.y, gy), zs = axis(gc.z, gz);
+              const uint32_t yx = ((ys & 1U) != 0U ? xs : 0U) | ((ys & 2U) != 0U ? xs << 3 : 0U) |
+                                  ((ys & 4U) != 0U ? xs << 6 : 0U);
+              const uint32_t reach = ((zs & 1U) != 0U ? yx : 0U) | ((zs & 2U) != 0U ? yx << 9 : 0U) |
+                                     ((zs & 4U) != 0U ? yx << 18 : 0U);
+              known = (reach & cur_nbr) == 0U;
+            }
+          } else if (cur_skip || cur_free) {
+            ones = cur_free;
+            lim = exit;
+          } else {
+            known = false;
+          }
+        }
+        if (known) {
+          if (ones && have_prev && prev_t < 0.0F) break;
+          have_prev = ones;
+          prev_t = 1.0F;
+          const float step = ones ? free_step : base_step;
+          float last = len;
+          len += step;
+          if (len >= enter) len = run_to(len, step, fminf(lim, depth_lim), last);
+          if (ones) prev_p = add3(pose.t, scale3(dir, last));  // the last free sample's point
+          continue;
+        }
+        float t;
+        if (!vol.tsdf(point, rp.require_all != 0, t, slots)) {
+          have_prev = false;
+          len += base_step;
+          continue;
+        }
+        if (have_prev && prev_t > 0.0F && t <= 0.0F) {
+          const float gap = prev_t - t;
+          const float alpha = gap != 0.0F ? prev_t / gap : 0.0F;
+          surface = add3(prev_p, scale3(sub3(point, prev_p), alpha));
+          hit = true;
+          break;
+        }
+        if (have_prev && prev_t < 0.0F && t > 0.0F) break;
+        have_prev = true;
+        prev_t = t;
+        prev_p = point;
+        const float pre = t * vol.g.trunc * rp.step_scale;
+        const float step = fmax_ref(base_step, pre);
+        len += t > 0.0F ? step : base_step;
       }
-      if (have_prev && prev_t > 0.0F && t <= 0.0F) {
-        const float gap = prev_t - t;
-        const float alpha = gap != 0.0F ? prev_t / gap : 0.0F;
-        surface = add3(prev_p, scale3(sub3(point, prev_p), alpha));
-        hit = true;
-        break;
-      }
-      if (have_prev && prev_t < 0.0F && t > 0.0F) break;
-      have_prev = true;
-      prev_t = t;
-      prev_p = point;
-      const float pre = t * vol.g.trunc * rp.step_scale;
-      const float step = fmax_ref(base_step, pre);
-      len += t > 0.0F ? step : base_step;
     }
     if (hit) {
       V3 n;
@@ -292,13 +344,21 @@ __device__ inline void raycast_pixel(const Sampler<Kind, Store>& vol, const RayP
   col[i] = C;
 }
 
-// Pixel of thread t (0..255) of 16 x 16 tile `tile` in a grid `tiles_x`
-// tiles wide: each wave takes an 8 x 8 quadrant (neighbouring rays march
-// alike, so a squarer wave diverges less than a 16 x 4 strip).
-__device__ inline void tile_pixel(int tile, int tiles_x, int t, int& x, int& y) {
-  x = (tile % tiles_x) * 16 + ((t >> 6) & 1) * 8 + (t & 7);
-  y = (tile / tiles_x) * 16 + (t >> 7) * 8 + ((t >> 3) & 7);
-}
+// A wave's rays are a block of 2^lw x 2^lh pixels and a workgroup is 2 x 2
+// such blocks (neighbouring rays march alike, so a squarer block diverges less
+// than a strip).  Pixel of thread t (0..255) of tile `tile` in a grid `tiles_x`
+// tiles wide; false for a lane without a ray.
+struct RayTile {
+  int lw, lh;
+  __host__ __device__ inline int width() const { return 2 << lw; }
+  __host__ __device__ inline int height() const { return 2 << lh; }
+  __device__ inline bool pixel(int tile, int tiles_x, int t, int& x, int& y) const {
+    const int lane = t & 63, wave = t >> 6;
+    x = (((tile % tiles_x) * 2 + (wave & 1)) << lw) + (lane & ((1 << lw) - 1));
+    y = (((tile / tiles_x) * 2 + (wave >> 1)) << lh) + (lane >> lw);
+    return lane < (1 << (lw + lh));
+  }
+};
 
 // The raycast options of the context's level `level` (its camera and size).
 inline RayParams ray_params(const kf_context* ctx, int level) {

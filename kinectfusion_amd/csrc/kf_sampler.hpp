@@ -66,9 +66,16 @@ struct DenseStore {
   __device__ inline Raw voxel_cached(const Grid& g, int x, int y, int z, SlotCache&) const {
     return vox[g.flat(x, y, z)];
   }
-  __device__ inline float4 color(const Grid& g, int x, int y, int z) const { return colors[g.flat(x, y, z)]; }
-  __device__ inline float4 color_cached(const Grid& g, int x, int y, int z, SlotCache&) const {
-    return colors[g.flat(x, y, z)];
+  // The colour voxels of the corners of the 2^3 stencil with base corner
+  // (x, y, z), four of them (z fixed): a corner outside the grid reads a
+  // clamped one, which the caller drops.
+  __device__ inline void colors4(const Grid& g, int x, int y, int z, float4 (&c)[4]) const {
+    const int x0 = min(max(x, 0), g.nx - 1), x1 = min(x + 1, g.nx - 1), y0 = min(max(y, 0), g.ny - 1),
+              y1 = min(y + 1, g.ny - 1), zc = min(max(z, 0), g.nz - 1);
+    c[0] = colors[g.flat(x0, y0, zc)];
+    c[1] = colors[g.flat(x1, y0, zc)];
+    c[2] = colors[g.flat(x0, y1, zc)];
+    c[3] = colors[g.flat(x1, y1, zc)];
   }
   __device__ inline bool has_colors() const { return colors != nullptr; }
 };
@@ -76,7 +83,7 @@ struct DenseStore {
 template <int Kind>
 struct HashedStore {
   using Raw = typename VoxelIO<Kind>::Raw;
-  static constexpr bool kDirect = false;  // a voxel needs a hash probe first
+  static constexpr bool kDirect = false;  // a voxel needs its block's slot first
   HashView hv;
   const Raw* __restrict__ pool;
   const float4* __restrict__ cpool;
@@ -84,76 +91,44 @@ struct HashedStore {
     const uint32_t key = hv.key_of(x, y, z);
     if (key != cache.key) {
       cache.key = key;
-      cache.slot = hv.find(key);
+      cache.slot = hv.slots[key];
     }
     return cache.slot;
   }
+  // A corner's voxel: an unallocated block's read goes to slot 0 and is
+  // replaced, since a guarded read would wait for the one before it.
+  __device__ inline size_t at(uint32_t slot, int x, int y, int z) const {
+    return static_cast<size_t>(slot == kNoSlot ? 0U : slot) * kBlockVoxels + intra_of(x, y, z);
+  }
   __device__ inline Raw voxel_cached(const Grid&, int x, int y, int z, SlotCache& cache) const {
     const uint32_t slot = slot_of(x, y, z, cache);
-    return slot == kNoSlot ? VoxelIO<Kind>::fresh() : pool[static_cast<size_t>(slot) * kBlockVoxels + intra_of(x, y, z)];
-  }
-  __device__ inline Raw voxel(const Grid& g, int x, int y, int z) const {
-    SlotCache cache;
-    return voxel_cached(g, x, y, z, cache);
-  }
-  __device__ inline float4 color_cached(const Grid&, int x, int y, int z, SlotCache& cache) const {
-    const uint32_t slot = slot_of(x, y, z, cache);
-    return slot == kNoSlot ? make_float4(0.0F, 0.0F, 0.0F, 0.0F)
-                           : cpool[static_cast<size_t>(slot) * kBlockVoxels + intra_of(x, y, z)];
-  }
-  __device__ inline float4 color(const Grid& g, int x, int y, int z) const {
-    SlotCache cache;
-    return color_cached(g, x, y, z, cache);
+    const Raw v = pool[at(slot, x, y, z)];
+    return slot == kNoSlot ? VoxelIO<Kind>::fresh() : v;
   }
   __device__ inline bool has_colors() const { return cpool != nullptr; }
-  // The pool slots of the eight corners (x fastest) of the 2^3 stencil with
-  // base corner (x, y, z); bit c of `in` marks a corner inside the grid.
-  // The first probe of every corner outside the cached block is issued
-  // before any is examined, so a stencil across block faces costs one round
-  // of table reads, not one per block; a probe that meets another key walks
-  // the chain.  The cache then holds the block of corner `own`.
-  __device__ inline void slots8(int x, int y, int z, unsigned in, int own, uint32_t (&slot)[8],
-                                SlotCache& cache) const {
-    uint32_t key[8];
-    uint2 e[8];
+  // The pool slots of the corners of the 2^3 stencil with base corner (x, y, z)
+  // in the z-layer z, x fastest: two x-neighbouring index entries per read
+  // (the index has one entry to spare).  Corners outside the grid read a
+  // clamped block's slot, which the caller drops.
+  __device__ inline void slots4(const Grid& g, int x, int y, int z, uint32_t (&slot)[4]) const {
+    const int x0 = max(x, 0) >> 3, x1 = min(x + 1, g.nx - 1) >> 3, y0 = max(y, 0) >> 3, y1 = min(y + 1, g.ny - 1) >> 3,
+              zc = min(max(z, 0), g.nz - 1) >> 3;
+    const uint32_t* p = hv.slots + (static_cast<size_t>(zc) * hv.by + y0) * hv.bx + x0;
+    const u32x2_a4 a = *reinterpret_cast<const u32x2_a4*>(p);
+    const u32x2_a4 b = *reinterpret_cast<const u32x2_a4*>(p + (y1 != y0 ? hv.bx : 0));
+    slot[0] = a.x;
+    slot[1] = x1 != x0 ? a.y : a.x;
+    slot[2] = b.x;
+    slot[3] = x1 != x0 ? b.y : b.x;
+  }
+  __device__ inline void colors4(const Grid& g, int x, int y, int z, float4 (&c)[4]) const {
+    uint32_t slot[4];
+    slots4(g, x, y, z, slot);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      key[c] = hv.key_of(x + (c & 1), y + ((c >> 1) & 1), z + (c >> 2));
-      e[c] = make_uint2(0xFFFFFFFFU, 0xFFFFFFFFU);  // kHashEmpty
-      if (((in >> c) & 1U) != 0U && key[c] != cache.key)
-        e[c] = reinterpret_cast<const uint2*>(hv.table)[hv.bucket(key[c])];
-    }
-    unsigned walk = 0U;
+    for (int i = 0; i < 4; ++i) c[i] = cpool[at(slot[i], x + (i & 1), y + (i >> 1), z)];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      uint32_t sl = kNoSlot;
-      if (((in >> c) & 1U) != 0U) {
-        if (key[c] == cache.key) {
-          sl = cache.slot;
-        } else if (e[c].y == key[c]) {
-          sl = e[c].x == kPendingSlot ? kNoSlot : e[c].x;
-        } else if (e[c].x != 0xFFFFFFFFU || e[c].y != 0xFFFFFFFFU) {
-          walk |= 1U << c;  // the home bucket holds another key
-        }
-      }
-      slot[c] = sl;
-    }
-    if (walk != 0U) {
-#pragma unroll
-      for (int c = 0; c < 8; ++c)
-        if (((walk >> c) & 1U) != 0U) slot[c] = hv.find(key[c]);
-    }
-    if (((in >> own) & 1U) != 0U) {
-      uint32_t k = 0U, sl = 0U;
-#pragma unroll
-      for (int c = 0; c < 8; ++c)
-        if (c == own) {
-          k = key[c];
-          sl = slot[c];
-        }
-      cache.key = k;
-      cache.slot = sl;
-    }
+    for (int i = 0; i < 4; ++i)
+      if (slot[i] == kNoSlot) c[i] = make_float4(0.0F, 0.0F, 0.0F, 0.0F);
   }
 };
 
@@ -165,8 +140,10 @@ struct Sampler {
   float inv_voxel;
 
   __device__ inline bool contains(V3 p) const {
-    return p.x >= 0.0F && p.y >= 0.0F && p.z >= 0.0F && p.x < static_cast<float>(g.nx) &&
-           p.y < static_cast<float>(g.ny) && p.z < static_cast<float>(g.nz);
+    // one condition, not six branches
+    return (static_cast<int>(p.x >= 0.0F) & static_cast<int>(p.y >= 0.0F) & static_cast<int>(p.z >= 0.0F) &
+            static_cast<int>(p.x < static_cast<float>(g.nx)) & static_cast<int>(p.y < static_cast<float>(g.ny)) &
+            static_cast<int>(p.z < static_cast<float>(g.nz))) != 0;
   }
   __device__ inline V3 grid_coords(V3 p) const {
     return scale3(sub3(p, mk3(g.ox, g.oy, g.oz)), inv_voxel);
@@ -191,9 +168,17 @@ struct Sampler {
     st.by = static_cast<int>(fl.y);
     st.bz = static_cast<int>(fl.z);
     st.fr = sub3(gg, fl);
-    st.interior = st.bx >= 0 && st.by >= 0 && st.bz >= 0 && st.bx + 1 < g.nx && st.by + 1 < g.ny &&
-                  st.bz + 1 < g.nz;
+    st.interior = (static_cast<int>(st.bx >= 0) & static_cast<int>(st.by >= 0) & static_cast<int>(st.bz >= 0) &
+                   static_cast<int>(st.bx + 1 < g.nx) & static_cast<int>(st.by + 1 < g.ny) &
+                   static_cast<int>(st.bz + 1 < g.nz)) != 0;
     return st;
+  }
+  // Bit c (x fastest): corner c of the stencil lies inside the grid.
+  __device__ inline unsigned corners_inside(const Stencil& st) const {
+    const unsigned mx = (st.bx >= 0 ? 0x55U : 0U) | (st.bx + 1 < g.nx ? 0xAAU : 0U);
+    const unsigned my = (st.by >= 0 ? 0x33U : 0U) | (st.by + 1 < g.ny ? 0xCCU : 0U);
+    const unsigned mz = (st.bz >= 0 ? 0x0FU : 0U) | (st.bz + 1 < g.nz ? 0xF0U : 0U);
+    return mx & my & mz;
   }
   // Loads of the eight corners (z -> y -> x order); bit c of `inb` marks a
   // corner inside the grid.
@@ -205,25 +190,18 @@ struct Sampler {
         return;
       }
     } else {
-      // the eight slots first (their probes together), then the voxels
-      inb = 0U;
-      if (st.ok) {
+      // the eight slots in one round of reads, then the eight voxels
+      inb = corners_inside(st);
+      if (!st.ok) return;
+      uint32_t lo[4], hi[4];
+      s.slots4(g, st.bx, st.by, st.bz, lo);
+      s.slots4(g, st.bx, st.by, st.bz + 1, hi);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          const int x = st.bx + (c & 1), y = st.by + ((c >> 1) & 1), z = st.bz + (c >> 2);
-          if (st.interior || (x >= 0 && y >= 0 && z >= 0 && x < g.nx && y < g.ny && z < g.nz)) inb |= 1U << c;
-        }
-      }
-      // the corner holding the stencil's point: base + 1 where the fraction is >= 0.5
-      const int own = (st.fr.x >= 0.5F ? 1 : 0) | (st.fr.y >= 0.5F ? 2 : 0) | (st.fr.z >= 0.5F ? 4 : 0);
-      uint32_t slot[8];
-      s.slots8(st.bx, st.by, st.bz, inb, own, slot, cache);
+      for (int c = 0; c < 8; ++c)
+        raw[c] = s.pool[s.at(c < 4 ? lo[c & 3] : hi[c & 3], st.bx + (c & 1), st.by + ((c >> 1) & 1), st.bz + (c >> 2))];
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const int x = st.bx + (c & 1), y = st.by + ((c >> 1) & 1), z = st.bz + (c >> 2);
-        raw[c] = slot[c] == kNoSlot ? IO::fresh()
-                                    : s.pool[static_cast<size_t>(slot[c]) * kBlockVoxels + intra_of(x, y, z)];
-      }
+      for (int c = 0; c < 8; ++c)
+        if ((c < 4 ? lo[c & 3] : hi[c & 3]) == kNoSlot) raw[c] = IO::fresh();
       return;
     }
     inb = 0U;
@@ -237,8 +215,39 @@ struct Sampler {
       inb |= 1U << c;
     }
   }
-  // blend_tsdf over loaded corners (the same float operations as tsdf()).
+  // blend_tsdf over loaded corners, without branches: a corner outside the
+  // grid (its bit of inb clear), unobserved or not finite adds +0 to both sums,
+  // which leaves them unchanged (neither sum is ever -0: they start at +0 and
+  // a round-to-nearest sum is -0 only when both terms are).  All: every corner
+  // lies inside the grid (inb is not looked at; a separate instance, so that
+  // the march's common case carries no corner mask).
+  template <bool All = false>
   __device__ inline bool blend(const Stencil& st, const typename IO::Raw (&raw)[8], unsigned inb, bool require_all,
+                               float& out) const {
+    float acc = 0.0F, wsum = 0.0F;
+    int valid = 0;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      float t, w;
+      bool obs, fin;
+      IO::unpack(raw[c], t, w, obs, fin);
+      const unsigned in = All ? 1U : inb >> c;
+      const bool use = (static_cast<unsigned>(obs) & static_cast<unsigned>(fin) & in) != 0U;
+      const float cw = axis_w(st.fr.x, c & 1) * axis_w(st.fr.y, (c >> 1) & 1) * axis_w(st.fr.z, c >> 2);
+      acc += use ? cw * t : 0.0F;
+      wsum += use ? cw : 0.0F;
+      valid += use ? 1 : 0;
+    }
+    if (!st.ok || (require_all && valid < 8)) return false;
+    if (wsum <= 1.0e-6F) return false;
+    const float d = acc / wsum;
+    if (!isfinite(d)) return false;
+    out = d;
+    return true;
+  }
+
+  // The same of a cell at the grid's edge, corner by corner.
+  __device__ inline bool blend_edge(const Stencil& st, const typename IO::Raw (&raw)[8], unsigned inb, bool require_all,
                                float& out) const {
     if (!st.ok) return false;
     float acc = 0.0F, wsum = 0.0F;
@@ -262,34 +271,6 @@ struct Sampler {
     out = d;
     return true;
   }
-
-  // blend() of a cell whose eight corners all lie inside the grid, without
-  // branches: a corner that is unobserved or not finite adds +0 to both sums,
-  // which leaves them unchanged (neither sum is ever -0: they start at +0 and
-  // a round-to-nearest sum is -0 only when both terms are).
-  __device__ inline bool blend_all(const Stencil& st, const typename IO::Raw (&raw)[8], bool require_all,
-                                   float& out) const {
-    float acc = 0.0F, wsum = 0.0F;
-    int valid = 0;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      float t, w;
-      bool obs, fin;
-      IO::unpack(raw[c], t, w, obs, fin);
-      const bool use = obs && fin;
-      const float cw = axis_w(st.fr.x, c & 1) * axis_w(st.fr.y, (c >> 1) & 1) * axis_w(st.fr.z, c >> 2);
-      acc += use ? cw * t : 0.0F;
-      wsum += use ? cw : 0.0F;
-      valid += use ? 1 : 0;
-    }
-    if (require_all && valid < 8) return false;
-    if (wsum <= 1.0e-6F) return false;
-    const float d = acc / wsum;
-    if (!isfinite(d)) return false;
-    out = d;
-    return true;
-  }
-
   // TrilinearSampler::tsdf + blend_tsdf.
   __device__ bool tsdf(V3 p, bool require_all, float& out) const {
     SlotCache cache;
@@ -303,16 +284,18 @@ struct Sampler {
     if (!st.ok) return false;
     typename IO::Raw raw[8];
     if constexpr (Store::kDirect) {
-      // the eight corners as four x-pair loads; blend_all() and blend() are
-      // the same float sequence
+      // the eight corners as four x-pair loads
       if (st.interior) {
         s.cell(g, st.bx, st.by, st.bz, raw);
-        return blend_all(st, raw, require_all, out);
+        return blend<true>(st, raw, 0xFFU, require_all, out);
       }
     }
     unsigned inb;
     load8(st, raw, inb, cache);
-    return blend(st, raw, inb, require_all, out);
+    // the two blends of a direct store must not share code: merged, the march's
+    // interior cells wait for this path's registers (60 -> 68 us at 160x120)
+    if constexpr (Store::kDirect) return blend_edge(st, raw, inb, require_all, out);
+    else return blend(st, raw, inb, require_all, out);
   }
 
   // blend_color.
@@ -326,7 +309,9 @@ struct Sampler {
     const V3 fr = sub3(gg, fl);
     V3 acc = mk3(0.0F, 0.0F, 0.0F);
     float wsum = 0.0F;
-    SlotCache cache;
+    float4 c[2][4];
+    s.colors4(g, bx, by, bz, c[0]);
+    s.colors4(g, bx, by, bz + 1, c[1]);
 #pragma unroll
     for (int oz = 0; oz <= 1; ++oz)
 #pragma unroll
@@ -334,11 +319,10 @@ struct Sampler {
 #pragma unroll
         for (int ox = 0; ox <= 1; ++ox) {
           const int x = bx + ox, y = by + oy, z = bz + oz;
-          if (x < 0 || y < 0 || z < 0 || x >= g.nx || y >= g.ny || z >= g.nz) continue;
-          const float4 c = s.color_cached(g, x, y, z, cache);
-          if (c.w <= 0.0F) continue;
+          const float4 v = c[oz][oy * 2 + ox];
+          if (x < 0 || y < 0 || z < 0 || x >= g.nx || y >= g.ny || z >= g.nz || v.w <= 0.0F) continue;
           const float cw = axis_w(fr.x, ox) * axis_w(fr.y, oy) * axis_w(fr.z, oz);
-          acc = add3(acc, scale3(mk3(c.x, c.y, c.z), cw));
+          acc = add3(acc, scale3(mk3(v.x, v.y, v.z), cw));
           wsum += cw;
         }
     if (wsum <= 1.0e-6F) return false;
@@ -351,29 +335,51 @@ struct Sampler {
   // reference's order.  Two samples at a time (not all six) bound the
   // register use of the raycaster, where the normal's peak would otherwise
   // set the register allocation, and so the occupancy, of the whole march.
-  __device__ bool normal(V3 p, bool require_all, V3& out) const {
-    // the six samples kBatch at a time: a direct store reads two at once; a
-    // hashed store's slot probes take too many registers for two
-    constexpr int kBatch = Store::kDirect ? 2 : 1;
-    float v[6];
+  __device__ __forceinline__ bool normal(V3 p, bool require_all, V3& out) const {
+    V3 dir = mk3(0.0F, 0.0F, 0.0F);
+    if constexpr (Store::kDirect) {
+      float v[6];
 #pragma unroll
-    for (int a0 = 0; a0 < 6; a0 += kBatch) {
-      Stencil st[kBatch];
-      typename IO::Raw raw[kBatch][8];
-      unsigned inb[kBatch];
-      SlotCache cache;
+      for (int a0 = 0; a0 < 6; a0 += 2) {
+        Stencil st[2];
+        typename IO::Raw raw[2][8];
+        unsigned inb[2];
+        SlotCache cache;
 #pragma unroll
-      for (int i = 0; i < kBatch; ++i) {
-        const int axis = (a0 + i) >> 1;
-        const V3 off = scale3(mk3(axis == 0 ? 1.0F : 0.0F, axis == 1 ? 1.0F : 0.0F, axis == 2 ? 1.0F : 0.0F), g.voxel);
-        st[i] = stencil(((a0 + i) & 1) == 0 ? add3(p, off) : sub3(p, off));
-        load8(st[i], raw[i], inb[i], cache);
+        for (int i = 0; i < 2; ++i) {
+          const int axis = (a0 + i) >> 1;
+          const V3 off = scale3(mk3(axis == 0 ? 1.0F : 0.0F, axis == 1 ? 1.0F : 0.0F, axis == 2 ? 1.0F : 0.0F), g.voxel);
+          st[i] = stencil(((a0 + i) & 1) == 0 ? add3(p, off) : sub3(p, off));
+          load8(st[i], raw[i], inb[i], cache);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          if (!blend(st[i], raw[i], inb[i], require_all, v[a0 + i])) return false;
       }
-#pragma unroll
-      for (int i = 0; i < kBatch; ++i)
-        if (!blend(st[i], raw[i], inb[i], require_all, v[a0 + i])) return false;
+      dir = mk3(v[0] - v[1], v[2] - v[3], v[4] - v[5]);
+    } else {
+      // one sample at a time in a loop that is not unrolled: unrolled, the six
+      // probes and their chain walks were 54 KB of code, a call out of the
+      // march that kept the sampler in scratch memory for all of it
+      SlotCache cache;
+      float plus = 0.0F;
+#pragma unroll 1
+      for (int k = 0; k < 6; ++k) {
+        const int axis = k >> 1;
+        const V3 off = scale3(mk3(axis == 0 ? 1.0F : 0.0F, axis == 1 ? 1.0F : 0.0F, axis == 2 ? 1.0F : 0.0F), g.voxel);
+        const Stencil st = stencil((k & 1) == 0 ? add3(p, off) : sub3(p, off));
+        typename IO::Raw raw[8];
+        unsigned inb;
+        load8(st, raw, inb, cache);
+        float v;
+        if (!blend(st, raw, inb, require_all, v)) return false;
+        const float d = plus - v;
+        if ((k & 1) == 0) plus = v;
+        else if (axis == 0) dir.x = d;
+        else if (axis == 1) dir.y = d;
+        else dir.z = d;
+      }
     }
-    const V3 dir = mk3(v[0] - v[1], v[2] - v[3], v[4] - v[5]);
     const float len = norm3(dir);
     if (len <= 0.0F) return false;
     out = div3(dir, len);

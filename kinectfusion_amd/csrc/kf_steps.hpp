@@ -25,6 +25,16 @@ namespace kf {
 // result stays below 2^(e+1) adds the same d = round(S)*u, and k of them add
 // k*d exactly.  Ties and the addition that leaves the binade are taken one at
 // a time, as are lengths outside the normal range this covers.
+KF_STEPS_HD inline int steps_floor(int n, int d) {
+  // floor(n / d) for 0 <= n < 2^24 + d, 0 < d < 2^24: a float quotient is
+  // within one of it for quotients below 2^20, and an exact remainder decides
+  // (a third of an integer division's instructions)
+  if (n >= (1 << 24) || d < 16) return n / d;
+  const int q = static_cast<int>(static_cast<float>(n) / static_cast<float>(d));
+  const int r = n - q * d;
+  return r < 0 ? q - 1 : (r >= d ? q + 1 : q);
+}
+
 KF_STEPS_HD inline float advance_to(float len, float step, float lim, float& last) {
   while (len < lim) {
     const float next = len + step;  // the loop's own rounded addition
@@ -48,13 +58,13 @@ KF_STEPS_HD inline float advance_to(float len, float step, float lim, float& las
     }
     const int m = static_cast<int>((bits & 0x7FFFFFU) | 0x800000U);
     const int dm = static_cast<int>((next - len) * inv_u);  // next - len is exact (next < 2 len)
-    const int kmax = ((1 << 24) - 1 - m) / dm;             // steps whose results stay below top (>= 1)
-    int k = kmax + 1;                                       // lim at or beyond top: all of them, then on
-    if (lim < top) {
-      const int lm = static_cast<int>(lim * inv_u);  // lim lies in (len, top): a multiple of u
-      k = (lm - m + dm - 1) / dm;                    // the first k with m + k*dm >= lm
-    }
-    const int take = k <= kmax ? k : kmax;
+    // lim lies in (len, top) as a multiple of u, or at or beyond top: then every
+    // step whose result stays below top (>= 1 of them)
+    const bool inside = lim < top;
+    const int lm = inside ? static_cast<int>(lim * inv_u) : (1 << 24) - 1;
+    // inside: the first k with m + k * dm >= lm, but no more than stay below top
+    int take = steps_floor(inside ? lm - m + dm - 1 : lm - m, dm);
+    if (inside && take * dm > (1 << 24) - 1 - m) --take;
     last = static_cast<float>(m + (take - 1) * dm) * u;
     len = static_cast<float>(m + take * dm) * u;
   }
