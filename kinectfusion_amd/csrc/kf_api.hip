@@ -303,8 +303,8 @@ void upload_pose(kf_context* ctx, const double* pose) {
   KF_HIP(hipMemcpyAsync(ctx->icp->pose, pose, 16 * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
 }
 
-void fetch_state(kf_context* ctx) {
-  KF_HIP(hipMemcpyAsync(ctx->icp_host, ctx->icp, sizeof(IcpState), hipMemcpyDeviceToHost, ctx->stream));
+void fetch_state(kf_context* ctx, bool restore = false) {
+  launch_icp_publish(ctx, restore);
   KF_HIP(hipStreamSynchronize(ctx->stream));
 }
 
@@ -319,11 +319,6 @@ void report_sync_timeouts(kf_context* ctx) {
   fail(KF_ERR_DEVICE,
        "ICP: a one-launch tracking level timed out waiting for its trials (is another context tracking on "
        "this device at the same time?); the frame was not integrated");
-}
-
-void fetch_state_checked(kf_context* ctx) {
-  fetch_state(ctx);
-  report_sync_timeouts(ctx);
 }
 
 // filtered: level 0's depth already holds the filtered frame
@@ -629,11 +624,12 @@ kf_status kf_create(const kf_config* cfg, kf_context** out) {
     ctx->counters = dalloc<uint32_t>(4);
     ctx->fused = dalloc<unsigned long long>(4);
     KF_HIP(hipMemsetAsync(ctx->fused, 0, 4 * sizeof(unsigned long long), ctx->stream));
-    ctx->partials = dalloc<float>(512 * 32);
+    ctx->partials = dalloc<float>(2 * 256 * 32);  // two steps' rows
     ctx->frame_w2c = dalloc<float>(16);
     ctx->icp = dalloc<IcpState>(1);
     KF_HIP(hipMemsetAsync(ctx->icp, 0, sizeof(IcpState), ctx->stream));
     KF_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctx->icp_host), sizeof(IcpState), hipHostMallocDefault));
+    KF_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&ctx->icp_mapped), ctx->icp_host, 0));
     if (c.init_mode == KF_INIT_LEARNED) {
       const LevelBuffers& L = ctx->lv[c.levels - 1];
       ctx->prev_coarse = dalloc<uint16_t>(static_cast<size_t>(L.w) * L.h);
@@ -820,7 +816,8 @@ kf_status kf_icp_reduce(kf_context* ctx, const float* lv, const float* ln, int32
                            lw, lh, reinterpret_cast<const float4*>(mv),
                            reinterpret_cast<const float4*>(mn), mw, mh, Intr{k[0], k[1], k[2], k[3]},
                            camera, model, max_dist, min_dot);
-    fetch_state_checked(ctx);
+    KF_HIP(hipStreamSynchronize(ctx->stream));
+    report_sync_timeouts(ctx);
     for (int i = 0; i < 29; ++i) sums[i] = static_cast<double>(ctx->icp_host->sums32[i]);
     *count = static_cast<int64_t>(__builtin_bit_cast(uint32_t, ctx->icp_host->sums32[29]));
   });
@@ -853,27 +850,15 @@ kf_status kf_icp_track_maps(kf_context* ctx, const float* lv, const float* ln, i
     require(lw > 0 && lh > 0 && mw > 0 && mh > 0, "kf_icp_track_maps: empty maps");
     require(iterations >= 1, "kf_icp_track_maps: iterations must be >= 1");
     const DeviceIcpParams p = to_device_params(*opt);
-    // running pose = model pose for the level setup, then the initial pose
-    KF_HIP(hipMemsetAsync(&ctx->icp->frame_failed, 0, sizeof(int), ctx->stream));
-    upload_pose(ctx, model_pose);
-    launch_icp_begin_level(ctx, 0);
-    upload_pose(ctx, pose_inout);
-    KF_HIP(hipMemcpyAsync(ctx->icp->level_pose0, pose_inout, 16 * sizeof(double), hipMemcpyHostToDevice,
-                          ctx->stream));
-    KF_HIP(hipMemcpyAsync(ctx->icp->best_pose, pose_inout, 16 * sizeof(double), hipMemcpyHostToDevice,
-                          ctx->stream));
+    launch_icp_begin_maps(ctx, model_pose, pose_inout);
     launch_icp_level(ctx, reinterpret_cast<const float4*>(lv), reinterpret_cast<const float4*>(ln), lw, lh,
                      reinterpret_cast<const float4*>(mv), reinterpret_cast<const float4*>(mn), mw, mh,
                      Intr{k[0], k[1], k[2], k[3]}, iterations, p, 0);
-    fetch_state(ctx);
+    fetch_state(ctx, true);  // leaves the context's tracking state untouched by this standalone call
     const kf_icp_result& r = ctx->icp_host->results[0];
     if (result != nullptr) *result = r;
     if (r.status == 0 || r.status == 1) std::memcpy(pose_inout, ctx->icp_host->pose, 16 * sizeof(double));
-    // leave the context's tracking state untouched by this standalone call
-    KF_HIP(hipMemcpyAsync(ctx->icp->pose, ctx->icp->prev_pose, 16 * sizeof(double),
-                          hipMemcpyDeviceToDevice, ctx->stream));
     ctx->icp_host->frame_failed = 0;
-    KF_HIP(hipMemsetAsync(&ctx->icp->frame_failed, 0, sizeof(int), ctx->stream));
     report_sync_timeouts(ctx);
   });
 }
@@ -886,12 +871,9 @@ kf_status kf_track(kf_context* ctx, const kf_icp_options* opt, double* pose_inou
     upload_pose(ctx, pose_inout);
     KF_HIP(hipMemsetAsync(&ctx->icp->frame_failed, 0, sizeof(int), ctx->stream));
     track_levels(ctx, p, false, ctx->cfg.icp_iterations);
-    fetch_state(ctx);
+    fetch_state(ctx, true);
     std::memcpy(pose_inout, ctx->icp_host->pose, 16 * sizeof(double));
     if (results != nullptr) copy_results(ctx, results);
-    KF_HIP(hipMemcpyAsync(ctx->icp->pose, ctx->icp->prev_pose, 16 * sizeof(double),
-                          hipMemcpyDeviceToDevice, ctx->stream));
-    KF_HIP(hipMemsetAsync(&ctx->icp->frame_failed, 0, sizeof(int), ctx->stream));
     report_sync_timeouts(ctx);
   });
 }

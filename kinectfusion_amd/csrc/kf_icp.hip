@@ -6,27 +6,36 @@
 // icp_correspondence.cu:216-343) with its host epilogue
 // (src/kinectfusion/icp_optimizer.cpp:82-169).
 //
-// Two kernels per Gauss-Newton / LM trial:
-//  * every thread matches its pixels (five at a time, their memory reads in
-//    flight together) and keeps the 29 per-correspondence terms (21 J^T J,
-//    6 J^T r, distance, r^2) in FP32 registers;
-//  * a wave reduces them with an xor butterfly, the four waves of a
-//    workgroup combine in a fixed order through LDS, and each workgroup
-//    writes one partial row -- no float atomics, so the sums do not depend
-//    on scheduling;
-//  * a one-workgroup kernel adds the partial rows in a fixed order with
-//    Kahan-compensated FP32 (a kernel boundary, not a device-scope fence in
-//    every sweep workgroup, makes the rows visible: such a fence writes back
-//    the L2 and costs more than the sweep itself);
-//  * one thread of it converts the sums to FP64 and runs the trial: FP64
-//    pivoted LDL^T solve, caps, Rodrigues increment and pose composition in
-//    FP64, convergence and failure latches.
-// Once a level's status latches (converged or failed) the remaining trial
-// kernels return at once, so a converged level costs no further sweeps.  The
-// stability spectrum (FP64 Jacobi) is checked once per level, by the level's
-// last trial, as in the reference's device loop.  A pass that usually exits
-// at once runs each level in one launch instead (icp_level_kernel).
+// One kernel per Gauss-Newton / LM trial (icp_step_kernel):
+//  * every workgroup reduces the partial rows that the step before wrote, in a
+//    fixed order with Kahan-compensated FP32, and its first wave runs that
+//    step's trial on the sums: FP64 pivoted LDL^T solve, caps, Rodrigues
+//    increment and pose composition, convergence and failure latches.  All
+//    do the same work, so no launch and no device-scope fence stands between a
+//    trial and the next sweep (such a fence in every sweep workgroup writes
+//    back the L2 and costs more than the sweep itself);
+//  * then every thread matches its pixels (up to five at a time, without
+//    branches, their memory reads in flight together) and keeps the 29
+//    per-correspondence terms (21 J^T J, 6 J^T r, distance, r^2) in FP32
+//    registers;
+//  * a wave reduces them by halves, the four waves of a workgroup combine in a
+//    fixed order through LDS, and each workgroup writes one partial row -- no
+//    float atomics, so the sums do not depend on scheduling.
+// What bounds it: latency, not rate.  A 640 x 480 sweep reads 20 MB (4 us of a
+// copy's rate) with one wave per SIMD; back to back, a launch costs 2.2 us
+// before it does anything and 4.4 us with its reads from another die.  A step
+// takes 14 us (sweep 5, trial 5) where the sweep and the one-thread trial as
+// two launches took 20, and a level of 10 steps, 3 of them active, 85 us for
+// 122.  kf_icp_track_maps over 640 x 480 maps: 105 us for 173.
+// Once a level's status latches (converged or failed) the remaining steps pass
+// the record on and return.  The stability spectrum (FP64) is checked once per
+// level, by its last kernel, as in the reference's device loop.  A pass that
+// usually exits at once runs each level in one launch instead
+// (icp_level_kernel).
+#include <cstddef>
+#include <cstring>
 #include <mutex>
+#include <type_traits>
 
 #include "kf_internal.hpp"
 
@@ -54,95 +63,106 @@ struct Maps {
 };
 
 // match() (icp_correspondence.hpp:44-110) in two halves so that a thread
-// can keep the memory reads of several pixels in flight together.
-// Front: read the live vertex and normal, transform, project into the model
-// maps; returns false when rejected before the model read.
+// can keep the memory reads of several pixels in flight together, and without
+// branches, so that the arithmetic of several pixels overlaps as well: a wave
+// has its SIMD to itself, and nothing else hides its latencies.
+// Front: transform the live vertex and project it into the model maps; false
+// (and model pixel 0) when rejected before the model read.
 __device__ inline bool match_front(const Maps& m, const Rigid& cam, const Rigid& mod, V3 lv, V3 ln, V3& src,
                                    size_t& mi) {
-  if (!finite3(lv) || !finite3(ln)) return false;
   src = xform(cam, lv);
   const V3 sim = xform(mod, src);
-  if (!finite3(sim) || sim.z <= 0.0F) return false;
   float u, v;
   project(m.k, sim, u, v);
-  int col, row;
-  if (!round_index(u, m.mw, col) || !round_index(v, m.mh, row)) return false;
-  mi = static_cast<size_t>(row) * m.mw + col;
-  return true;
+  const float col = roundf(u), row = roundf(v);  // lround into [0, size); a NaN fails
+  const bool ok = finite3(lv) & finite3(ln) & finite3(sim) & (sim.z > 0.0F) & (col >= 0.0F) &
+                  (col < static_cast<float>(m.mw)) & (row >= 0.0F) & (row < static_cast<float>(m.mh));
+  mi = ok ? static_cast<size_t>(static_cast<int>(row)) * m.mw + static_cast<int>(col) : 0;
+  return ok;
 }
 
 // Back: with the model vertex and normal read, the distance and normal
-// tests and the point-to-plane row (J, residual).
-__device__ inline bool match_back(const Rigid& cam, float max_dist, float min_dot, V3 ln, V3 src, V3 mv, V3 mn,
-                                  float* J, float& res, float& dist) {
-  if (!finite3(mv) || !finite3(mn)) return false;
-  const V3 sn = normalize3(rot(cam, ln));
-  dist = norm3(sub3(src, mv));
-  if (dist > max_dist) return false;
-  if (dot3(sn, mn) < min_dot) return false;
+// tests and the point-to-plane row (J, residual), zero if there is no match.
+__device__ inline bool match_back(const Rigid& cam, float max_dist, float min_dot, bool ok, V3 ln, V3 src, V3 mv,
+                                  V3 mn, float* J, float& res, float& dist) {
+  const V3 r = rot(cam, ln);
+  const float len = norm3(r);
+  const V3 q = div3(r, len);
+  const bool unit = len > 0.0F;
+  const V3 sn = mk3(unit ? q.x : 0.0F, unit ? q.y : 0.0F, unit ? q.z : 0.0F);
+  const float d = norm3(sub3(src, mv));
+  ok = ok & finite3(mv) & finite3(mn) & !(d > max_dist) & !(dot3(sn, mn) < min_dot);
   const V3 r3 = cross3(src, mn);
-  J[0] = r3.x;
-  J[1] = r3.y;
-  J[2] = r3.z;
-  J[3] = mn.x;
-  J[4] = mn.y;
-  J[5] = mn.z;
-  res = dot3(mn, sub3(mv, src));
-  return true;
+  const float e = dot3(mn, sub3(mv, src));
+  J[0] = ok ? r3.x : 0.0F;
+  J[1] = ok ? r3.y : 0.0F;
+  J[2] = ok ? r3.z : 0.0F;
+  J[3] = ok ? mn.x : 0.0F;
+  J[4] = ok ? mn.y : 0.0F;
+  J[5] = ok ? mn.z : 0.0F;
+  res = ok ? e : 0.0F;
+  dist = ok ? d : 0.0F;
+  return ok;
 }
 
 // Pixels a thread matches per pass (grid-stride order): their live reads,
 // then their model reads, are issued together; the terms are added in pixel
-// order.
-constexpr int kPixBatch = 5;
+// order (a rejected pixel adds +0, which changes no sum: none is ever -0).
+// Five fill the widest grid's share of a 640 x 480 level in one pass; a grid
+// whose threads have one or two pixels each takes a pass of that size (with
+// five, a 160 x 120 sweep took 8.0 us for 4.8: four fifths of it on nothing).
+template <int Batch>
+struct LiveBatch {
+  V3 v[Batch], n[Batch];
+};
+
+__device__ inline int sweep_base(int blk) {
+  return blk * static_cast<int>(blockDim.x) + static_cast<int>(threadIdx.x);
+}
+
+// The live pixels of a pass, the last one again past the end.
+template <int Batch>
+__device__ __forceinline__ void read_live(const Maps& m, int base, int stride, LiveBatch<Batch>& live) {
+  const int last = m.lw * m.lh - 1;
+#pragma unroll
+  for (int j = 0; j < Batch; ++j) {
+    const int p = min(base + j * stride, last);
+    live.v[j] = ld3(m.lv[p]);
+    live.n[j] = ld3(m.ln[p]);
+  }
+}
 
 // Per-workgroup sweep: sums of block `blk`'s pixels (of `nblk` sweeping
-// blocks) into partial[blk].
-__device__ inline void sweep_block(const Maps& m, const Rigid& cam, const Rigid& mod, float max_dist,
-                                   float min_dot, float* __restrict__ partial, float (*lds)[kSums + 1],
-                                   int blk, int nblk) {
+// blocks) into partial[blk].  live: the first pass's pixels, read by the
+// caller (ahead of whatever it waits for).
+template <int Batch>
+__device__ __forceinline__ void sweep_block(const Maps& m, const Rigid& cam, const Rigid& mod, float max_dist,
+                                            float min_dot, float* __restrict__ partial, float (*lds)[kSums + 1],
+                                            int blk, int nblk, LiveBatch<Batch>& live) {
   float s[kSums];
 #pragma unroll
   for (int i = 0; i < kSums; ++i) s[i] = 0.0F;
   unsigned int cnt = 0;
   const int n = m.lw * m.lh;
   const int stride = nblk * static_cast<int>(blockDim.x);
-  for (int base = blk * static_cast<int>(blockDim.x) + static_cast<int>(threadIdx.x); base < n;
-       base += kPixBatch * stride) {
-    V3 lv[kPixBatch], ln[kPixBatch];
-    bool ok[kPixBatch];
+  for (int base = sweep_base(blk); base < n;) {
+    V3 src[Batch], mv[Batch], mn[Batch];
+    size_t mi[Batch];
+    bool ok[Batch];
 #pragma unroll
-    for (int j = 0; j < kPixBatch; ++j) {
-      const int p = base + j * stride;
-      ok[j] = p < n;
-      lv[j] = mk3(0.0F, 0.0F, 0.0F);
-      ln[j] = lv[j];
-      if (ok[j]) {
-        lv[j] = ld3(m.lv[p]);
-        ln[j] = ld3(m.ln[p]);
-      }
-    }
-    V3 src[kPixBatch], mv[kPixBatch], mn[kPixBatch];
-    size_t mi[kPixBatch];
-#pragma unroll
-    for (int j = 0; j < kPixBatch; ++j) {
-      src[j] = mk3(0.0F, 0.0F, 0.0F);
-      mi[j] = 0;
-      ok[j] = ok[j] && match_front(m, cam, mod, lv[j], ln[j], src[j], mi[j]);
+    for (int j = 0; j < Batch; ++j) {
+      ok[j] = match_front(m, cam, mod, live.v[j], live.n[j], src[j], mi[j]);
+      ok[j] = ok[j] & (base + j * stride < n);
     }
 #pragma unroll
-    for (int j = 0; j < kPixBatch; ++j) {
-      mv[j] = mk3(0.0F, 0.0F, 0.0F);
-      mn[j] = mv[j];
-      if (ok[j]) {
-        mv[j] = ld3(m.mv[mi[j]]);
-        mn[j] = ld3(m.mn[mi[j]]);
-      }
+    for (int j = 0; j < Batch; ++j) {
+      mv[j] = ld3(m.mv[mi[j]]);
+      mn[j] = ld3(m.mn[mi[j]]);
     }
 #pragma unroll
-    for (int j = 0; j < kPixBatch; ++j) {
+    for (int j = 0; j < Batch; ++j) {
       float J[6], res, dist;
-      if (!ok[j] || !match_back(cam, max_dist, min_dot, ln[j], src[j], mv[j], mn[j], J, res, dist)) continue;
+      ok[j] = match_back(cam, max_dist, min_dot, ok[j], live.n[j], src[j], mv[j], mn[j], J, res, dist);
       int e = 0;
 #pragma unroll
       for (int r = 0; r < 6; ++r)
@@ -152,29 +172,47 @@ __device__ inline void sweep_block(const Maps& m, const Rigid& cam, const Rigid&
       for (int r = 0; r < 6; ++r) s[21 + r] += J[r] * res;
       s[27] += dist;
       s[28] += res * res;
-      ++cnt;
+      cnt += ok[j] ? 1U : 0U;
     }
+    base += Batch * stride;
+    if (base < n) read_live(m, base, stride, live);
   }
-  // wave butterfly
+  // The wave's sums: at each step a lane keeps half of its values and takes
+  // the other lanes' halves of them, so 31 exchanges reduce all 30 (a
+  // butterfly of every value takes 180); each value is the same tree of
+  // pairwise sums over lanes 32, 16, ..., 1 apart.  Lane 2 i ends with value i.
+  // The count is summed as a float, exact below 2^24.
+  float v[16];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
+  for (int i = 0; i < 16; ++i) {
+    const float lo = s[i], hi = i + 16 < kSums ? s[i + 16] : (i + 16 == kSums ? static_cast<float>(cnt) : 0.0F);
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
+    v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
 #pragma unroll
-    for (int i = 0; i < kSums; ++i) s[i] += __shfl_xor(s[i], off);
-    cnt += __shfl_xor(cnt, off);
+  for (int i = 0; i < 8; ++i) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 8]), false, false);
+    v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
   }
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (lane == 0) {
 #pragma unroll
-    for (int i = 0; i < kSums; ++i) lds[wave][i] = s[i];
-    lds[wave][kSums] = __uint_as_float(cnt);
+  for (int half = 4; half > 0; half >>= 1) {  // lanes 8, 4 and 2 apart
+    const bool upper = (lane & (2 * half)) != 0;
+#pragma unroll
+    for (int i = 0; i < half; ++i) {
+      const float keep = upper ? v[i + half] : v[i], give = upper ? v[i] : v[i + half];
+      v[i] = keep + __shfl_xor(give, 2 * half);
+    }
   }
+  v[0] += __shfl_xor(v[0], 1);
+  if ((lane & 1) == 0 && lane <= 2 * kSums) lds[wave][lane >> 1] = v[0];
   __syncthreads();
   if (threadIdx.x < kSums) {
     const int i = threadIdx.x;
     partial[blk * kPartialStride + i] = (lds[0][i] + lds[1][i]) + (lds[2][i] + lds[3][i]);
   } else if (threadIdx.x == kSums) {
-    const unsigned int c = __float_as_uint(lds[0][kSums]) + __float_as_uint(lds[1][kSums]) +
-                           __float_as_uint(lds[2][kSums]) + __float_as_uint(lds[3][kSums]);
+    unsigned int c = 0;
+    for (int w = 0; w < 4; ++w) c += static_cast<unsigned int>(lds[w][kSums]);
     partial[blk * kPartialStride + kSums] = __uint_as_float(c);
   }
 }
@@ -184,29 +222,27 @@ __device__ inline void sweep_block(const Maps& m, const Rigid& cam, const Rigid&
 // split over 8 threads: part q adds rows q, q + 8, ... with Kahan, then
 // thread c adds the 8 part sums (net of their compensations) in order
 // q = 0..7.  The order is fixed, so the result does not depend on scheduling.
-__device__ inline void combine_partials(const float* __restrict__ partial, int nblocks, float* out) {
+// (256 threads; the reads apart, so that a caller can issue them ahead.)
+using Quad = float __attribute__((ext_vector_type(4)));  // stays in registers (a float4 array goes to scratch)
+struct RowBatch {
+  Quad v[kMaxBlocks * kPartialStride / 4 / 256];
+};
+
+__device__ __forceinline__ void read_rows(const float* __restrict__ partial, int nblocks, RowBatch& rows) {
+  const int last = nblocks * kPartialStride / 4 - 1;
+#pragma unroll
+  for (int j = 0; j < kMaxBlocks * kPartialStride / 4 / 256; ++j)  // every row in flight at once
+    rows.v[j] = reinterpret_cast<const Quad*>(partial)[min(static_cast<int>(threadIdx.x) + j * 256, last)];
+}
+
+__device__ __forceinline__ void combine_rows(const RowBatch& batch, int nblocks, float* out) {
   __shared__ __align__(16) float rows[kMaxBlocks * kPartialStride];
   __shared__ float part_sum[8][kPartialStride];
   __shared__ float part_comp[8][kPartialStride];
   __shared__ unsigned part_cnt[8];
-  {
-    // every row in flight at once (8 float4 per thread), not one round trip
-    // per loop iteration
-    constexpr int kQuads = kMaxBlocks * kPartialStride / 4 / 256;
-    const int quads = nblocks * kPartialStride / 4;
-    const float4* src = reinterpret_cast<const float4*>(partial);
-    float4 v[kQuads];
 #pragma unroll
-    for (int j = 0; j < kQuads; ++j) {
-      const int i = static_cast<int>(threadIdx.x) + j * 256;
-      v[j] = i < quads ? src[i] : make_float4(0.0F, 0.0F, 0.0F, 0.0F);
-    }
-#pragma unroll
-    for (int j = 0; j < kQuads; ++j) {
-      const int i = static_cast<int>(threadIdx.x) + j * 256;
-      if (i < quads) reinterpret_cast<float4*>(rows)[i] = v[j];
-    }
-  }
+  for (int j = 0; j < kMaxBlocks * kPartialStride / 4 / 256; ++j)  // past nblocks: never read
+    reinterpret_cast<Quad*>(rows)[static_cast<int>(threadIdx.x) + j * 256] = batch.v[j];
   __syncthreads();
   const int col = threadIdx.x & 31, q = threadIdx.x >> 5;  // 256 threads: 32 columns x 8 parts
   float sum = 0.0F, comp = 0.0F;
@@ -241,108 +277,129 @@ __device__ inline void combine_partials(const float* __restrict__ partial, int n
   }
 }
 
+__device__ __forceinline__ void combine_partials(const float* __restrict__ partial, int nblocks, float* out) {
+  RowBatch rows;
+  read_rows(partial, nblocks, rows);
+  combine_rows(rows, nblocks, out);
+}
+
 // FP64 LDL^T with symmetric diagonal pivoting (largest remaining |d| first),
 // the factorisation Eigen::LDLT uses in the reference host solve
 // (icp_optimizer.cpp:391): a pivot with |d| <= DBL_MIN contributes a zero
 // solution component, so a damped semidefinite system still solves; the
 // solve fails only on a non-finite solution.
-__device__ inline void swap_d(double& a, double& b) {
-  const double t = a;
-  a = b;
-  b = t;
+//
+// By a wave: lane 8 r + c holds element (r, c) of the matrix, column 6 the
+// right-hand side (so the forward substitution runs along with the
+// elimination) and column 7 the row's place in the solution.  A lane divides
+// for itself the two factors that its element's update takes; one thread
+// eliminating alone spends 21 divisions and the swaps of every pivot one
+// after the other.  A whole trial takes 7400 cycles, 9000 that way (12000
+// with the steps unrolled or the solution in scratch memory).  Every operation is the scalar form's, in its order.  A
+// solution that is not finite leaves x (in LDS) as it was.
+__device__ inline void wave_sync() {  // LDS writes of a wave's lanes before the others' reads
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
-__device__ bool solve6(const double* eq, int damping_mode, double scale, double* x) {
-  // Every index below is a compile-time constant after unrolling (the pivot
-  // swap is predicated), so the factorisation lives in registers.
-  double a[6][6];
-  {
-    int e = 0;
-#pragma unroll
-    for (int r = 0; r < 6; ++r)
-#pragma unroll
-      for (int c = r; c < 6; ++c, ++e) {
-        a[r][c] = eq[e];
-        a[c][r] = eq[e];
-      }
-  }
-#pragma unroll
-  for (int r = 0; r < 6; ++r) {
-    if (damping_mode == 1) a[r][r] += scale;
-    else if (damping_mode == 2) a[r][r] += scale * a[r][r];
-  }
-  int perm[6] = {0, 1, 2, 3, 4, 5};
-  double d[6];
-#pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    int piv = k;
-    double best = fabs(a[k][k]);
-#pragma unroll
-    for (int i = k + 1; i < 6; ++i) {
-      const double v = fabs(a[i][i]);
-      if (v > best) {
-        best = v;
-        piv = i;
-      }
-    }
-#pragma unroll
-    for (int i = k + 1; i < 6; ++i) {
-      if (piv == i) {
-#pragma unroll
-        for (int c = 0; c < 6; ++c) swap_d(a[k][c], a[i][c]);
-#pragma unroll
-        for (int r = 0; r < 6; ++r) swap_d(a[r][k], a[r][i]);
-        const int tp = perm[k];
-        perm[k] = perm[i];
-        perm[i] = tp;
-      }
-    }
-    d[k] = a[k][k];
-    const bool zero = fabs(d[k]) <= 2.2250738585072014e-308;
-#pragma unroll
-    for (int i = k + 1; i < 6; ++i) a[i][k] = zero ? 0.0 : a[i][k] / d[k];
-#pragma unroll
-    for (int i = k + 1; i < 6; ++i)
-#pragma unroll
-      for (int jj = k + 1; jj <= i; ++jj) {
-        a[i][jj] -= a[i][k] * d[k] * a[jj][k];
-        a[jj][i] = a[i][jj];
-      }
-  }
-  double y[6];
-#pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    double s = eq[21 + perm[i]];
-#pragma unroll
-    for (int q = 0; q < i; ++q) s -= a[i][q] * y[q];
-    y[i] = s;
-  }
-#pragma unroll
-  for (int i = 0; i < 6; ++i) y[i] = fabs(d[i]) <= 2.2250738585072014e-308 ? 0.0 : y[i] / d[i];
-  double z[6];
-#pragma unroll
-  for (int i = 5; i >= 0; --i) {
-    double s = y[i];
-#pragma unroll
-    for (int q = i + 1; q < 6; ++q) s -= a[q][i] * z[q];
-    z[i] = s;
-  }
+__device__ inline double lane_value(double v, int lane) {  // lane: the same in every lane
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u), lane));
+  const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u >> 32), lane));
+  return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+__device__ inline double shuffled(double v, int address) {  // address: 4 times the lane
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(address, static_cast<int>(u)));
+  const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(address, static_cast<int>(u >> 32)));
+  return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+// The place of the largest |diagonal| element from k on, the first of equal
+// ones; a NaN is never larger, and nothing is larger than one at k.  Almost
+// always the upper halves alone decide, in scalar registers.
+__device__ __forceinline__ int pivot_of(double a, int lane, int k) {
+  const uint32_t high = static_cast<uint32_t>(__builtin_bit_cast(uint64_t, a) >> 32) & 0x7FFFFFFFU;
+  const bool diagonal = (lane >> 3) == (lane & 7) && (lane >> 3) >= k && lane < 46;
+  const uint32_t key = diagonal ? high : 0U;
+  uint32_t most = 0;
 #pragma unroll
   for (int i = 0; i < 6; ++i)
-#pragma unroll
-    for (int jj = 0; jj < 6; ++jj)
-      if (perm[i] == jj) x[jj] = z[i];
+    most = max(most, static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key), 9 * i)));
+  const uint64_t at = __ballot(key == most);
+  if (most != 0 && most < 0x7FF00000U && __builtin_popcountll(at) == 1) return __builtin_ctzll(at) >> 3;
+  int piv = k;
+  double best = fabs(lane_value(a, 9 * k));
+#pragma unroll 1
+  for (int i = k + 1; i < 6; ++i) {
+    const double v = fabs(lane_value(a, 9 * i));
+    if (v > best) {
+      best = v;
+      piv = i;
+    }
+  }
+  return __builtin_amdgcn_readfirstlane(piv);
+}
+
+__device__ __forceinline__ bool solve6(const double* eq, int damping_mode, double scale, double* x) {
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const int row = lane >> 3, col = lane & 7;
+  const int hi = max(row, col), lo = min(row, col);
+  const bool rhs = col == 6;
+  double a = eq[row < 6 && col < 6 ? lo * 6 - lo * (lo - 1) / 2 + hi - lo : 21 + min(row, 5)];
+  a = col == 7 ? static_cast<double>(row) : a;
+  if (damping_mode != 0) {
+    const double damped = a + (damping_mode == 1 ? scale : scale * a);
+    a = col == row ? damped : a;
+  }
+  double quotient = 0.0;  // (row, 6): y / d
+  int upper_at = 4 * (8 * (rhs ? row : min(hi, 5)));
+  int lower_at = 4 * (rhs ? 6 : 8 * min(lo, 5));
+  const int lower_step = rhs ? 32 : 4;
+#pragma unroll 1
+  for (int k = 0; k < 6; ++k) {
+    const int piv = pivot_of(a, lane, k);
+    if (piv != k) {  // the rows and the columns k and piv change places
+      const int from_row = row == k ? piv : (row == piv ? k : row);
+      const int from_col = col == k ? piv : (col == piv ? k : col);
+      a = shuffled(a, 4 * (8 * from_row + from_col));
+    }
+    const double d = lane_value(a, 9 * k);
+    const bool zero = fabs(d) <= 2.2250738585072014e-308;
+    // below the pivot: a -= (l_hi d) l_lo, and the right-hand side less l y
+    const double upper = shuffled(a, upper_at);
+    const double lower = shuffled(a, lower_at);
+    upper_at += 4;
+    lower_at += lower_step;
+    const double l = zero ? 0.0 : upper / d;  // (row, 6): of this row
+    const double q = zero ? 0.0 : lower / d;  // (row, 6): y_k / d
+    const double less = (rhs ? l : l * d) * (rhs ? lower : q);
+    const bool inside = row > k && row < 6;
+    if (rhs && row == k) quotient = q;
+    if (inside && col == k) a = l;
+    if (inside && col > k && col < 7) a -= less;
+  }
+  double z[6], own = 0.0;
   bool ok = true;
 #pragma unroll
-  for (int i = 0; i < 6; ++i) ok = ok && isfinite(x[i]);
+  for (int i = 5; i >= 0; --i) {
+    double v = lane_value(quotient, 8 * i + 6);
+#pragma unroll
+    for (int j = i + 1; j < 6; ++j) v -= lane_value(a, 8 * j + i) * z[j];
+    z[i] = v;
+    own = row == i ? v : own;
+    ok = ok && isfinite(v);
+  }
+  if (ok && col == 7 && row < 6) x[static_cast<int>(a)] = own;
+  wave_sync();
   return ok;
 }
 
 // pose <- exp([w]) pose in FP64 (Rodrigues; left-multiplied world-frame
-// increment, icp_optimizer.cpp:286).
-__device__ void compose_increment(const double* x, double* pose) {
-  const double wx = x[0], wy = x[1], wz = x[2];
-  const double angle = sqrt(wx * wx + wy * wy + wz * wz);
+// increment, icp_optimizer.cpp:286), by a wave: a lane writes an element.
+__device__ __forceinline__ void compose_increment(const double* x, double angle, double* pose) {
+  const double wx = x[0], wy = x[1], wz = x[2];  // angle: their length
   double R[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
   if (angle > 1.0e-12) {
     const double ux = wx / angle, uy = wy / angle, uz = wz / angle;
@@ -359,17 +416,19 @@ __device__ void compose_increment(const double* x, double* pose) {
     R[7] = uz * uy * oc + ux * s;
     R[8] = c + uz * uz * oc;
   }
-  double out[12];
-  for (int r = 0; r < 3; ++r) {
-    for (int c = 0; c < 3; ++c)
-      out[r * 4 + c] = R[r * 3 + 0] * pose[0 * 4 + c] + R[r * 3 + 1] * pose[1 * 4 + c] +
-                       R[r * 3 + 2] * pose[2 * 4 + c];
-    out[r * 4 + 3] = R[r * 3 + 0] * pose[3] + R[r * 3 + 1] * pose[7] + R[r * 3 + 2] * pose[11] + x[3 + r];
-  }
-  for (int i = 0; i < 12; ++i) pose[i] = out[i];
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const int r = (lane >> 2) & 3, c = lane & 3;
+  const double r0 = r == 0 ? R[0] : (r == 1 ? R[3] : R[6]);
+  const double r1 = r == 0 ? R[1] : (r == 1 ? R[4] : R[7]);
+  const double r2 = r == 0 ? R[2] : (r == 1 ? R[5] : R[8]);
+  const double t = x[3 + min(r, 2)];
+  double out = r0 * pose[c] + r1 * pose[4 + c] + r2 * pose[8 + c];
+  if (c == 3) out += t;
+  wave_sync();  // every lane has read the pose
+  if (lane < 12) pose[lane] = out;
 }
 
-__device__ void sym_eig6(const double* eq, double* ev);
+__device__ __noinline__ void sym_eig6(const double* eq, double* ev);
 
 // check_system_stability (icp_optimizer.cpp:319-347) on FP64 sums.
 __device__ bool stable_from_eigenvalues(const double* ev, const DeviceIcpParams& p, double* min_eig, double* cond);
@@ -377,7 +436,7 @@ __device__ bool stable_from_eigenvalues(const double* ev, const DeviceIcpParams&
 __device__ bool stable_system(const double* eq, long long count, const DeviceIcpParams& p,
                               double* min_eig, double* cond) {
   if (count < p.min_corr) return false;
-  double ev[6];
+  __shared__ double ev[6];  // a wave's lanes write the same values
   sym_eig6(eq, ev);
   return stable_from_eigenvalues(ev, p, min_eig, cond);
 }
@@ -395,87 +454,195 @@ __device__ bool stable_from_eigenvalues(const double* ev, const DeviceIcpParams&
   return mn >= static_cast<double>(p.min_eig) && mx / mn <= static_cast<double>(p.max_cond);
 }
 
-// One trial on the combined sums (solve_update_kernel semantics).  A failing
-// trial reports kUnconstrainedSystem when the undamped system is unstable,
-// as the reference host loop vetoes before solving (icp_optimizer.cpp:263-270).
-__device__ void run_trial(IcpState* st, const DeviceIcpParams& p, const float* sums32) {
-  double sums[kSums];
-  for (int i = 0; i < kSums; ++i) sums[i] = static_cast<double>(sums32[i]);
+// One trial on the combined sums (solve_update_kernel semantics), by the first
+// wave of a workgroup, its record and the sums in LDS.  A failing trial
+// reports kUnconstrainedSystem when the undamped system is unstable, as the
+// reference host loop vetoes before solving (icp_optimizer.cpp:263-270).
+__device__ __forceinline__ void run_trial(IcpTrial* t, const DeviceIcpParams& p, const float* sums32) {
+  const int lane = static_cast<int>(threadIdx.x);
+  const double sum = lane < kSums ? static_cast<double>(sums32[lane]) : 0.0;
   const long long count = static_cast<long long>(__float_as_uint(sums32[kSums]));
   if (count < p.min_corr) {
-    for (int i = 0; i < kSums; ++i) st->eq[i] = sums[i];
-    st->eq_count = count;
-    st->status = 2;
+    if (lane < kSums) t->eq[lane] = sum;
+    if (lane == 0) {
+      t->eq_count = count;
+      t->status = 2;
+    }
     return;
   }
-  if (st->trials == 0) st->lambda = p.lambda0;
+  const int trials = t->trials;
+  double lambda = trials == 0 ? static_cast<double>(p.lambda0) : t->lambda;
   const bool damping = p.damping_mode != 0;
   const bool adaptive = damping && p.adaptive != 0;
   bool accepted = true;
+  long long eq_count = count;
+  double eq = sum;
   if (adaptive) {
-    const double cost = sums[28] / static_cast<double>(count);
-    accepted = st->trials == 0 || cost <= st->best_cost;
+    const double cost = static_cast<double>(sums32[28]) / static_cast<double>(count);
+    accepted = trials == 0 || cost <= t->best_cost;
+    wave_sync();  // every lane has read what lane 0 writes
     if (accepted) {
-      st->best_cost = cost;
-      for (int i = 0; i < kSums; ++i) st->best_eq[i] = sums[i];
-      st->best_count = count;
-      for (int i = 0; i < 16; ++i) st->best_pose[i] = st->pose[i];
-      st->lambda = fmax(st->lambda * p.dec, static_cast<double>(p.lmin));
+      if (lane < kSums) t->best_eq[lane] = sum;
+      if (lane < 16) t->best_pose[lane] = t->pose[lane];
+      if (lane == 0) {
+        t->best_cost = cost;
+        t->best_count = count;
+      }
+      lambda = fmax(lambda * p.dec, static_cast<double>(p.lmin));
     } else {
-      ++st->rejected;
-      for (int i = 0; i < 16; ++i) st->pose[i] = st->best_pose[i];
-      st->lambda = fmin(st->lambda * p.inc, static_cast<double>(p.lmax));
+      if (lane < 16) t->pose[lane] = t->best_pose[lane];
+      if (lane == 0) ++t->rejected;
+      lambda = fmin(lambda * p.inc, static_cast<double>(p.lmax));
+      if (lane < kSums) eq = t->best_eq[lane];
+      eq_count = t->best_count;
     }
-    for (int i = 0; i < kSums; ++i) st->eq[i] = st->best_eq[i];
-    st->eq_count = st->best_count;
-  } else {
-    for (int i = 0; i < kSums; ++i) st->eq[i] = sums[i];
-    st->eq_count = count;
   }
-  ++st->trials;
+  wave_sync();
+  if (lane < kSums) t->eq[lane] = eq;
+  wave_sync();
   const int attempts = damping ? 8 : 1;
-  double x[6] = {0, 0, 0, 0, 0, 0};
-  double scale = st->lambda, used = st->lambda, ut = 0.0, ang = 0.0;
+  __shared__ double x[6];
+  double scale = lambda, ut = 0.0, ang = 0.0;
   bool solved = false;
   for (int a = 0; a < attempts; ++a) {
-    double xs[6];
-    if (solve6(st->eq, p.damping_mode, scale, xs)) {
+    if (solve6(t->eq, p.damping_mode, scale, x)) {
       solved = true;
-      used = scale;
-      for (int i = 0; i < 6; ++i) x[i] = xs[i];
+      lambda = scale;
       ang = sqrt(x[0] * x[0] + x[1] * x[1] + x[2] * x[2]);
       ut = sqrt(x[3] * x[3] + x[4] * x[4] + x[5] * x[5]);
       if (!damping || (ut <= p.max_t && ang <= p.max_r)) break;
     }
     scale = fmin(scale * p.inc, static_cast<double>(p.lmax));
   }
-  if (!solved) {
-    st->status = (!damping && !stable_system(st->eq, st->eq_count, p, nullptr, nullptr)) ? 5 : 3;
-    return;
+  int status = 0;
+  if (!solved || ut > p.max_t || ang > p.max_r) {
+    const bool unstable = !damping && !stable_system(t->eq, eq_count, p, nullptr, nullptr);
+    status = unstable ? 5 : (solved ? 4 : 3);
+  } else {
+    compose_increment(x, ang, t->pose);
+    if (accepted && ut < p.min_t && ang < p.min_r) status = 1;
   }
-  st->lambda = used;
-  st->update_t = ut;
-  st->update_r = ang;
-  if (ut > p.max_t || ang > p.max_r) {
-    st->status = (!damping && !stable_system(st->eq, st->eq_count, p, nullptr, nullptr)) ? 5 : 4;
-    return;
+  if (lane == 0) {
+    t->eq_count = eq_count;
+    t->trials = trials + 1;
+    t->lambda = lambda;
+    if (solved) {
+      t->update_t = ut;
+      t->update_r = ang;
+    }
+    t->status = status;
   }
-  compose_increment(x, st->pose);
-  if (accepted && ut < p.min_t && ang < p.min_r) st->status = 1;
 }
 
-__device__ void finish_level_block(IcpState* st, const DeviceIcpParams& p, int level, float check_rms);
+template <typename State>
+__device__ void finish_level_block(IcpState* st, const State* t, const DeviceIcpParams& p, int level, float check_rms);
 
-// One trial's correspondence sweep: one partial row per workgroup.
-__global__ void __launch_bounds__(256) icp_trial_sweep_kernel(Maps m, DeviceIcpParams p, IcpState* st,
-                                                               float* __restrict__ partial) {
+// The trial fields of a level's state, and their return (a whole workgroup of
+// at least 32 threads; the caller synchronises).
+template <typename To, typename From>
+__device__ inline void copy_trial(To* to, const From* from) {
+  const int i = static_cast<int>(threadIdx.x);
+  if (i < 16) {
+    to->pose[i] = from->pose[i];
+    to->best_pose[i] = from->best_pose[i];
+  }
+  if (i < kSums) {
+    to->eq[i] = from->eq[i];
+    to->best_eq[i] = from->best_eq[i];
+  }
+  if (i == 0) {
+    to->best_cost = from->best_cost;
+    to->lambda = from->lambda;
+    to->update_t = from->update_t;
+    to->update_r = from->update_r;
+    to->eq_count = from->eq_count;
+    to->best_count = from->best_count;
+    to->status = from->status;
+    to->trials = from->trials;
+    to->rejected = from->rejected;
+  }
+}
+
+// One step of a level: the previous step's trial (its reduction and FP64
+// solve), then this step's correspondence sweep.  Every workgroup solves the
+// same trial for itself from the same rows, so a trial needs no launch of its
+// own and no fence: a step reads the rows and the trial record the step before
+// wrote (one of two, in turn) and writes the other.  Two launches per trial
+// took 2 launch latencies and, once a level had latched, 2 empty launches.
+__device__ inline void copy_record(IcpTrial* to, const IcpTrial* from) {  // by 256 threads
+  static_assert(sizeof(IcpTrial) % 4 == 0 && sizeof(IcpTrial) / 4 <= 256, "a word per thread");
+  if (threadIdx.x < sizeof(IcpTrial) / 4)
+    reinterpret_cast<uint32_t*>(to)[threadIdx.x] = reinterpret_cast<const uint32_t*>(from)[threadIdx.x];
+}
+
+// The rows of step k.
+__device__ inline float* step_rows(float* rows, int k) { return rows + (k & 1) * kMaxBlocks * kPartialStride; }
+
+// The trial that follows a step, its record in LDS, from the step's rows.
+__device__ __forceinline__ void solve_step(const DeviceIcpParams& p, const RowBatch& rows, int nblocks, IcpTrial* t,
+                                  float* combined) {
+  combine_rows(rows, nblocks, combined);
+  __syncthreads();
+  if (threadIdx.x < 64) run_trial(t, p, combined);
+  __syncthreads();
+}
+
+// What a step reads -- the record and the rows of the step before, then the
+// live pixels -- is in flight before the work that waits for it, as each read
+// comes from another die's memory (about a microsecond).
+template <int Batch>
+__global__ void __launch_bounds__(256) icp_step_kernel(Maps m, DeviceIcpParams p, IcpState* st,
+                                                        float* __restrict__ rows, int k) {
   __shared__ float lds[4][kSums + 1];
-  if (st->status != 0 || st->frame_failed) return;  // latched: nothing to do
-  // the trial's pose, and the level's model pose inverse (kept in float by
-  // the level's preparation)
-  const Rigid cam = rigid_from_pose64(st->pose), mod = rigid_from12(st->model_inv);
-  sweep_block(m, cam, mod, p.max_dist, p.min_dot, partial, lds, static_cast<int>(blockIdx.x),
-                static_cast<int>(gridDim.x));
+  __shared__ float combined[kSums + 1];
+  __shared__ IcpTrial t;
+  const int blk = static_cast<int>(blockIdx.x), nblk = static_cast<int>(gridDim.x);
+  const int failed = st->frame_failed;
+  const Rigid mod = rigid_from12(st->model_inv);
+  LiveBatch<Batch> live;
+  Rigid cam;
+  if (k == 0) {
+    cam = rigid_from_pose64(st->pose);
+    if (failed != 0) return;
+    read_live(m, sweep_base(blk), nblk * static_cast<int>(blockDim.x), live);
+    if (blk == 0) copy_trial(&st->trial[0], st);  // the level's start as the first record
+  } else {
+    RowBatch before;
+    read_rows(step_rows(rows, k - 1), nblk, before);
+    copy_record(&t, &st->trial[(k - 1) & 1]);
+    __syncthreads();
+    if (failed != 0) return;
+    const bool latched = t.status != 0;  // the record is passed on
+    if (!latched) {
+      read_live(m, sweep_base(blk), nblk * static_cast<int>(blockDim.x), live);
+      solve_step(p, before, nblk, &t, combined);
+    }
+    if (blk == 0) copy_record(&st->trial[k & 1], &t);
+    if (t.status != 0) return;
+    cam = rigid_from_pose64(t.pose);
+  }
+  sweep_block(m, cam, mod, p.max_dist, p.min_dot, step_rows(rows, k), lds, blk, nblk, live);
+}
+
+// The end of a level after its last step (one workgroup): the last trial, the
+// record's fields back in the state, the stability check and result, and the
+// learned warm start's check.
+__global__ void __launch_bounds__(256) icp_finish_steps_kernel(DeviceIcpParams p, IcpState* st,
+                                                                float* __restrict__ rows, int nblocks, int steps,
+                                                                int level, float check_rms) {
+  __shared__ float combined[kSums + 1];
+  __shared__ IcpTrial t;
+  RowBatch before;
+  read_rows(step_rows(rows, steps - 1), nblocks, before);
+  copy_record(&t, &st->trial[(steps - 1) & 1]);
+  const int failed = st->frame_failed;
+  __syncthreads();
+  if (failed == 0) {
+    if (t.status == 0) solve_step(p, before, nblocks, &t, combined);
+    copy_trial(st, &t);
+    __syncthreads();
+  }
+  finish_level_block(st, &t, p, level, check_rms);
 }
 
 // Ticket protocol: returns true in the workgroup that finished last, after
@@ -506,11 +673,13 @@ __device__ inline bool last_block(unsigned int* ticket) {
 // timed-out launch leaves short is reset when the next level begins.
 // st->level_sync: [0] ticket, [1] epoch (only ever advanced: a launch reads
 // its base before any workgroup can advance it).
+template <int Batch>
 __global__ void __launch_bounds__(256) icp_level_kernel(Maps m, DeviceIcpParams p, IcpState* st,
                                                         float* __restrict__ partial, long long timeout_ticks,
                                                         int iterations, int level) {
   __shared__ float lds[4][kSums + 1];
   __shared__ float combined[kSums + 1];
+  __shared__ IcpTrial t;
   __shared__ float xf[24];
   __shared__ int go, timed_out;
   if (st->frame_failed) return;
@@ -529,16 +698,21 @@ __global__ void __launch_bounds__(256) icp_level_kernel(Maps m, DeviceIcpParams 
     __syncthreads();
     if (go == 0) break;
     const Rigid cam = rigid_from12(xf), mod = rigid_from12(xf + 12);
+    LiveBatch<Batch> live;
+    read_live(m, sweep_base(blockIdx.x), static_cast<int>(gridDim.x * blockDim.x), live);
     sweep_block(m, cam, mod, p.max_dist, p.min_dot, partial, lds, static_cast<int>(blockIdx.x),
-                static_cast<int>(gridDim.x));
+                static_cast<int>(gridDim.x), live);
     const unsigned int target = base + static_cast<unsigned int>(it) + 1U;
     if (last_block(&sync[0])) {
+      copy_trial(&t, st);
       combine_partials(partial, gridDim.x, combined);
       __syncthreads();
-      if (threadIdx.x <= kSums) st->sums32[threadIdx.x] = combined[threadIdx.x];
+      if (threadIdx.x < 64) run_trial(&t, p, combined);
+      __syncthreads();
+      copy_trial(st, &t);
+      __syncthreads();
       if (threadIdx.x == 0) {
         sync[0] = 0U;
-        run_trial(st, p, combined);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         __hip_atomic_store(&sync[1], target, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
@@ -564,44 +738,32 @@ __global__ void __launch_bounds__(256) icp_level_kernel(Maps m, DeviceIcpParams 
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
   }
-  if (blockIdx.x == 0) finish_level_block(st, p, level, 0.0F);
-}
-
-// The trial's reduction (one workgroup: the partial rows into st->sums32)
-// and its FP64 solve and pose update (one thread).  A kernel of its own, so
-// the partial rows of every sweep workgroup are visible without a
-// device-scope fence in each of them.
-__global__ void __launch_bounds__(256) icp_trial_solve_kernel(DeviceIcpParams p, IcpState* st,
-                                                               const float* __restrict__ partial, int nblocks,
-                                                               int finish_level, float check_rms) {
-  __shared__ float combined[kSums + 1];
-  if (st->status == 0 && st->frame_failed == 0) {
-    combine_partials(partial, nblocks, combined);
-    __syncthreads();
-    if (threadIdx.x <= kSums) st->sums32[threadIdx.x] = combined[threadIdx.x];
-    if (threadIdx.x == 0) run_trial(st, p, combined);
-  }
-  if (finish_level >= 0) {
-    __syncthreads();
-    finish_level_block(st, p, finish_level, check_rms);
-  }
+  if (blockIdx.x == 0) finish_level_block(st, st, p, level, 0.0F);
 }
 
 // Single sweep with explicit float transforms (kf_icp_reduce), then its
 // reduction into st->sums32.
+template <int Batch>
 __global__ void __launch_bounds__(256) icp_sweep_kernel(Maps m, Rigid cam, Rigid mod, float max_dist,
                                                          float min_dot, float* __restrict__ partial) {
   __shared__ float lds[4][kSums + 1];
+  LiveBatch<Batch> live;
+  read_live(m, sweep_base(blockIdx.x), static_cast<int>(gridDim.x * blockDim.x), live);
   sweep_block(m, cam, mod, max_dist, min_dot, partial, lds, static_cast<int>(blockIdx.x),
-              static_cast<int>(gridDim.x));
+              static_cast<int>(gridDim.x), live);
 }
 
-__global__ void __launch_bounds__(256) icp_combine_kernel(IcpState* st, const float* __restrict__ partial,
-                                                           int nblocks) {
+// The reduction into the host's mirror of the state (mapped memory, seen by
+// the host once the stream is synchronised): a copy of the state took as long
+// as the sweep and the reduction together.
+__global__ void __launch_bounds__(256) icp_combine_kernel(const IcpState* st, const float* __restrict__ partial,
+                                                           int nblocks, IcpState* __restrict__ host) {
   __shared__ float combined[kSums + 1];
+  const int timeouts = st->sync_timeouts;
   combine_partials(partial, nblocks, combined);
   __syncthreads();
-  if (threadIdx.x <= kSums) st->sums32[threadIdx.x] = combined[threadIdx.x];
+  if (threadIdx.x <= kSums) host->sums32[threadIdx.x] = combined[threadIdx.x];
+  if (threadIdx.x == 32) host->sync_timeouts = timeouts;
 }
 
 // The same reduction into caller memory: the 29 sums widened to FP64 and the
@@ -617,7 +779,7 @@ __global__ void __launch_bounds__(256) icp_combine_out_kernel(const float* __res
 }
 
 // FP64 cyclic Jacobi eigenvalues of the symmetric 6x6 system.
-__device__ void sym_eig6(const double* eq, double* ev) {
+__device__ __noinline__ void sym_eig6(const double* eq, double* ev) {
   double a[6][6];
   int e = 0;
   for (int r = 0; r < 6; ++r)
@@ -760,9 +922,7 @@ __device__ void sym_eig6_wave(const double* eq, double* ev) {
 #pragma unroll
     for (int i = 0; i < 5; ++i) tri[6 + i] = e[i];
   }
-  // lane 0's LDS writes precede every lane's reads in the wave's program order
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
+  wave_sync();
   double d[6], e2[5];
   bool finite = true;
   double lo = 1.0e308, hi = -1.0e308;
@@ -799,8 +959,7 @@ __device__ void sym_eig6_wave(const double* eq, double* ev) {
     hi = nhi;
   }
   if (k < 6 && j == 1) ev[k] = finite ? 0.5 * (lo + hi) : __builtin_nan("");
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
+  wave_sync();
 }
 
 // Prepare a level: status cleared, model pose = running pose.
@@ -808,22 +967,56 @@ __global__ void __launch_bounds__(64) icp_begin_level_kernel(IcpState* st, int l
   if (threadIdx.x == 0) icp_begin_level(st, level);
 }
 
+struct Pose64 {
+  double m[16];
+};
+
+// A level between maps of the caller's: the model maps' pose and the start.
+__global__ void __launch_bounds__(64) icp_begin_maps_kernel(IcpState* st, Pose64 model, Pose64 start) {
+  const int i = static_cast<int>(threadIdx.x);
+  if (i == 0) st->frame_failed = 0;
+  if (i < 16) st->pose[i] = model.m[i];
+  __syncthreads();
+  if (i == 0) icp_begin_level(st, 0);
+  __syncthreads();
+  if (i < 16) {
+    st->pose[i] = start.m[i];
+    st->level_pose0[i] = start.m[i];
+    st->best_pose[i] = start.m[i];
+  }
+}
+
+// The state into the host's mirror (mapped memory; all but the steps' records,
+// its end); then, after a standalone track, the context's own pose back.
+__global__ void __launch_bounds__(256) icp_publish_kernel(IcpState* st, IcpState* __restrict__ host, int restore) {
+  constexpr unsigned words = offsetof(IcpState, trial) / 8;
+  static_assert(offsetof(IcpState, trial) % 8 == 0, "copied in 8-byte words");
+  for (unsigned i = threadIdx.x; i < words; i += blockDim.x)
+    reinterpret_cast<uint64_t*>(host)[i] = reinterpret_cast<const uint64_t*>(st)[i];
+  if (restore == 0) return;
+  __syncthreads();
+  if (threadIdx.x < 16) st->pose[threadIdx.x] = st->prev_pose[threadIdx.x];
+  if (threadIdx.x == 0) st->frame_failed = 0;
+}
+
 // Stability check and result record of a level (icp_optimizer.cpp:108-169),
 // by a whole workgroup (the Jacobi sweeps take its first wave), then, when
 // check_rms > 0, the learned warm start's check of this level.
-__device__ void finish_level_block(IcpState* st, const DeviceIcpParams& p, int level, float check_rms) {
+// t: the level's trial fields (the state itself, or a copy of them in LDS).
+template <typename State>
+__device__ void finish_level_block(IcpState* st, const State* t, const DeviceIcpParams& p, int level, float check_rms) {
   __shared__ double ev[6];
   __shared__ int skip, check;
   if (threadIdx.x == 0) {
     skip = st->frame_failed;
-    check = (st->status == 0 || st->status == 1) && st->eq_count >= p.min_corr ? 1 : 0;
+    check = skip == 0 && (t->status == 0 || t->status == 1) && t->eq_count >= p.min_corr ? 1 : 0;
   }
   __syncthreads();
   if (skip == 0) {
-    if (check != 0 && threadIdx.x < 64) sym_eig6_wave(st->eq, ev);  // the first wave
+    if (check != 0 && threadIdx.x < 64) sym_eig6_wave(t->eq, ev);  // the first wave
     if (threadIdx.x == 0) {
       kf_icp_result& r = st->results[level];
-      int status = st->status;
+      int status = t->status;
       r.min_eigenvalue = 0.0;
       r.condition_number = 0.0;
       if (status == 0 || status == 1) {
@@ -831,16 +1024,16 @@ __device__ void finish_level_block(IcpState* st, const DeviceIcpParams& p, int l
         if (!stable && p.damping_mode == 0) status = 5;
       }
       r.status = status;
-      r.trials = st->trials;
-      r.rejected = st->rejected;
-      r.correspondences = st->eq_count;
-      if (st->eq_count > 0) {
-        r.mean_distance = st->eq[27] / static_cast<double>(st->eq_count);
-        r.mean_squared_residual = st->eq[28] / static_cast<double>(st->eq_count);
+      r.trials = t->trials;
+      r.rejected = t->rejected;
+      r.correspondences = t->eq_count;
+      if (t->eq_count > 0) {
+        r.mean_distance = t->eq[27] / static_cast<double>(t->eq_count);
+        r.mean_squared_residual = t->eq[28] / static_cast<double>(t->eq_count);
       }
-      r.update_translation = st->update_t;
-      r.update_rotation = st->update_r;
-      r.lambda = st->lambda;
+      r.update_translation = t->update_t;
+      r.update_rotation = t->update_r;
+      r.lambda = t->lambda;
       st->status = status;
       if (status >= 2) {
         // failure: the outcome keeps the level's initial pose
@@ -856,7 +1049,7 @@ __device__ void finish_level_block(IcpState* st, const DeviceIcpParams& p, int l
 // A level with no trial: its finish alone.
 __global__ void __launch_bounds__(64) icp_finish_level_kernel(IcpState* st, DeviceIcpParams p, int level,
                                                                float check_rms) {
-  finish_level_block(st, p, level, check_rms);
+  finish_level_block(st, st, p, level, check_rms);
 }
 
 Maps make_maps(const float4* lv_v, const float4* lv_n, int lw, int lh, const float4* md_v,
@@ -889,6 +1082,51 @@ DeviceIcpParams to_device_params(const kf_icp_options& o) {
   return p;
 }
 
+namespace {
+
+// f(the pixels of a pass): as many as a thread has, to five.
+template <typename F>
+void for_batch(const Maps& m, int nb, const F& f) {
+  const int64_t threads = static_cast<int64_t>(nb) * 256, pixels = static_cast<int64_t>(m.lw) * m.lh;
+  if (pixels <= threads) f(std::integral_constant<int, 1>{});
+  else if (pixels <= 2 * threads) f(std::integral_constant<int, 2>{});
+  else f(std::integral_constant<int, 5>{});
+}
+
+void launch_single_level(const Maps& m, int nb, kf_context* ctx, const DeviceIcpParams& p, int iterations, int level) {
+  for_batch(m, nb, [&](auto batch) {
+    static int resident = -1;  // workgroups of this kernel resident at once on this device
+    if (resident < 0) {
+      int per_cu = 0, dev = 0;
+      KF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, icp_level_kernel<batch.value>, 256, 0));
+      KF_HIP(hipGetDevice(&dev));
+      hipDeviceProp_t prop{};
+      KF_HIP(hipGetDeviceProperties(&prop, dev));
+      resident = per_cu * prop.multiProcessorCount;
+    }
+    if (nb > resident) fail(KF_ERR_DEVICE, "icp level: the grid does not fit on the device at once");
+    hipLaunchKernelGGL(icp_level_kernel<batch.value>, dim3(nb), dim3(256), 0, ctx->stream, m, p, ctx->icp,
+                       ctx->partials, ctx->sync_timeout_ticks, iterations, level);
+    KF_HIP(hipGetLastError());
+  });
+}
+
+}  // namespace
+
+void launch_icp_begin_maps(kf_context* ctx, const double* model_pose, const double* pose) {
+  Pose64 model, start;
+  std::memcpy(model.m, model_pose, sizeof(model.m));
+  std::memcpy(start.m, pose, sizeof(start.m));
+  hipLaunchKernelGGL(icp_begin_maps_kernel, dim3(1), dim3(64), 0, ctx->stream, ctx->icp, model, start);
+  KF_HIP(hipGetLastError());
+}
+
+void launch_icp_publish(kf_context* ctx, bool restore) {
+  hipLaunchKernelGGL(icp_publish_kernel, dim3(1), dim3(256), 0, ctx->stream, ctx->icp, ctx->icp_mapped,
+                     restore ? 1 : 0);
+  KF_HIP(hipGetLastError());
+}
+
 void launch_icp_begin_level(kf_context* ctx, int level) {
   hipLaunchKernelGGL(icp_begin_level_kernel, dim3(1), dim3(64), 0, ctx->stream, ctx->icp, level);
   KF_HIP(hipGetLastError());
@@ -907,29 +1145,17 @@ void launch_icp_level(kf_context* ctx, const float4* lv_v, const float4* lv_n, i
   }
   if (single_launch) {
     if (check_max_rms > 0.0F) fail(KF_ERR_INVALID_ARGUMENT, "icp level: the learned check needs two-kernel trials");
-    static int resident = -1;  // workgroups of icp_level_kernel resident at once on this device
-    if (resident < 0) {
-      int per_cu = 0, dev = 0;
-      KF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, icp_level_kernel, 256, 0));
-      KF_HIP(hipGetDevice(&dev));
-      hipDeviceProp_t prop{};
-      KF_HIP(hipGetDeviceProperties(&prop, dev));
-      resident = per_cu * prop.multiProcessorCount;
-    }
-    if (nb > resident) fail(KF_ERR_DEVICE, "icp level: the grid does not fit on the device at once");
-    hipLaunchKernelGGL(icp_level_kernel, dim3(nb), dim3(256), 0, ctx->stream, m, p, ctx->icp, ctx->partials,
-                       ctx->sync_timeout_ticks, iterations, level);
-    KF_HIP(hipGetLastError());
+    launch_single_level(m, nb, ctx, p, iterations, level);
     return;
   }
-  // the level's last trial also finishes the level (and runs the learned check)
-  for (int it = 0; it < iterations; ++it) {
-    const int finish = it + 1 == iterations ? level : -1;
-    hipLaunchKernelGGL(icp_trial_sweep_kernel, dim3(nb), dim3(256), 0, ctx->stream, m, p, ctx->icp,
-                       ctx->partials);
-    hipLaunchKernelGGL(icp_trial_solve_kernel, dim3(1), dim3(256), 0, ctx->stream, p, ctx->icp, ctx->partials, nb,
-                       finish, finish >= 0 ? check_max_rms : 0.0F);
-  }
+  // one launch per trial, and one that ends the level (and runs the learned check)
+  for_batch(m, nb, [&](auto batch) {
+    for (int it = 0; it < iterations; ++it)
+      hipLaunchKernelGGL(icp_step_kernel<batch.value>, dim3(nb), dim3(256), 0, ctx->stream, m, p, ctx->icp,
+                         ctx->partials, it);
+  });
+  hipLaunchKernelGGL(icp_finish_steps_kernel, dim3(1), dim3(256), 0, ctx->stream, p, ctx->icp, ctx->partials, nb,
+                     iterations, level, check_max_rms);
   KF_HIP(hipGetLastError());
 }
 
@@ -939,9 +1165,12 @@ void launch_icp_reduce_once(kf_context* ctx, const float4* lv_v, const float4* l
                             float min_dot) {
   const Maps m = make_maps(lv_v, lv_n, lw, lh, md_v, md_n, mw, mh, k);
   const int nb = blocks_for(lw * lh);
-  hipLaunchKernelGGL(icp_sweep_kernel, dim3(nb), dim3(256), 0, ctx->stream, m,
-                     rigid_from12(camera12), rigid_from12(model12), max_dist, min_dot, ctx->partials);
-  hipLaunchKernelGGL(icp_combine_kernel, dim3(1), dim3(256), 0, ctx->stream, ctx->icp, ctx->partials, nb);
+  for_batch(m, nb, [&](auto batch) {
+    hipLaunchKernelGGL(icp_sweep_kernel<batch.value>, dim3(nb), dim3(256), 0, ctx->stream, m,
+                       rigid_from12(camera12), rigid_from12(model12), max_dist, min_dot, ctx->partials);
+  });
+  hipLaunchKernelGGL(icp_combine_kernel, dim3(1), dim3(256), 0, ctx->stream, ctx->icp, ctx->partials, nb,
+                     ctx->icp_mapped);
   KF_HIP(hipGetLastError());
 }
 
@@ -974,8 +1203,10 @@ void launch_icp_reduce_static(hipStream_t stream, const float4* lv_v, const floa
   float* rows = static_scratch_rows();
   const Maps m = make_maps(lv_v, lv_n, lw, lh, md_v, md_n, mw, mh, k);
   const int nb = blocks_for(lw * lh);  // <= kMaxBlocks rows, every one written by the sweep
-  hipLaunchKernelGGL(icp_sweep_kernel, dim3(nb), dim3(256), 0, stream, m, rigid_from12(camera12),
-                     rigid_from12(model12), max_dist, min_dot, rows);
+  for_batch(m, nb, [&](auto batch) {
+    hipLaunchKernelGGL(icp_sweep_kernel<batch.value>, dim3(nb), dim3(256), 0, stream, m, rigid_from12(camera12),
+                       rigid_from12(model12), max_dist, min_dot, rows);
+  });
   hipLaunchKernelGGL(icp_combine_out_kernel, dim3(1), dim3(256), 0, stream, rows, nb, sums, count);
   KF_HIP(hipGetLastError());
 }

@@ -249,6 +249,18 @@ struct HashView {
 // ---------------------------------------------------------------------------
 // ICP device state, one per context (device memory).
 // ---------------------------------------------------------------------------
+// The fields of a level that its trials change, as the steps hand them on.
+struct IcpTrial {
+  double pose[16];
+  double best_pose[16];
+  double eq[29];
+  double best_eq[29];
+  double best_cost, lambda;
+  double update_t, update_r;
+  long long eq_count, best_count;
+  int status, trials, rejected, pad;
+};
+
 struct IcpState {
   double pose[16];        // running camera_to_world
   double model_pose[16];  // render pose of the current level's model maps
@@ -285,6 +297,7 @@ struct IcpState {
   // trials, and reset when a level begins, after a timed-out launch left it
   // short), [1] epoch (only ever advanced)
   unsigned int level_sync[2];
+  IcpTrial trial[2];  // the steps' records, written in turn
 };
 
 // Prepare a tracking level (one thread): the level's result reads "not run",
@@ -472,7 +485,8 @@ struct kf_context {
   long long sync_timeout_ticks = 2000000;  // 20 ms
   int seen_timeouts = 0;
   kf::IcpState* icp = nullptr;    // device
-  kf::IcpState* icp_host = nullptr;  // pinned mirror for results
+  kf::IcpState* icp_host = nullptr;    // pinned mirror for results
+  kf::IcpState* icp_mapped = nullptr;  // its device address
   double* trajectory = nullptr;   // device, 16 doubles per frame
   int64_t traj_capacity = 0;
   int64_t frames = 0;
@@ -557,6 +571,12 @@ void launch_icp_reduce_static(hipStream_t stream, const float4* lv_v, const floa
                               const float* camera12, const float* model12, float max_dist, float min_dot,
                               double* sums, int64_t* count);
 void launch_icp_begin_level(kf_context* ctx, int level_index);
+// A level between the caller's maps: the context's own pose and failure mark
+// are set aside until launch_icp_publish(ctx, true).
+void launch_icp_begin_maps(kf_context* ctx, const double* model_pose, const double* pose);
+// The state into ctx->icp_host once the stream is synchronised; restore: then
+// the context's own pose back, and no failure.
+void launch_icp_publish(kf_context* ctx, bool restore);
 // The learned warm start's fallback pass (every level: raycast, then the
 // trials) as one launch that returns at once when the learned run was kept;
 // false when its grid cannot be resident at once on this device (the caller
