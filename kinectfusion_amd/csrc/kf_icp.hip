@@ -75,8 +75,8 @@ __device__ inline bool match_front(const Maps& m, const Rigid& cam, const Rigid&
   float u, v;
   project(m.k, sim, u, v);
   const float col = roundf(u), row = roundf(v);  // lround into [0, size); a NaN fails
-  const bool ok = finite3(lv) & finite3(ln) & finite3(sim) & (sim.z > 0.0F) & (col >= 0.0F) &
-                  (col < static_cast<float>(m.mw)) & (row >= 0.0F) & (row < static_cast<float>(m.mh));
+  const bool ok = finite3(lv) && finite3(ln) && finite3(sim) && sim.z > 0.0F && col >= 0.0F &&
+                  col < static_cast<float>(m.mw) && row >= 0.0F && row < static_cast<float>(m.mh);
   mi = ok ? static_cast<size_t>(static_cast<int>(row)) * m.mw + static_cast<int>(col) : 0;
   return ok;
 }
@@ -91,7 +91,7 @@ __device__ inline bool match_back(const Rigid& cam, float max_dist, float min_do
   const bool unit = len > 0.0F;
   const V3 sn = mk3(unit ? q.x : 0.0F, unit ? q.y : 0.0F, unit ? q.z : 0.0F);
   const float d = norm3(sub3(src, mv));
-  ok = ok & finite3(mv) & finite3(mn) & !(d > max_dist) & !(dot3(sn, mn) < min_dot);
+  ok = ok && finite3(mv) && finite3(mn) && !(d > max_dist) && !(dot3(sn, mn) < min_dot);
   const V3 r3 = cross3(src, mn);
   const float e = dot3(mn, sub3(mv, src));
   J[0] = ok ? r3.x : 0.0F;
@@ -152,7 +152,7 @@ __device__ __forceinline__ void sweep_block(const Maps& m, const Rigid& cam, con
 #pragma unroll
     for (int j = 0; j < Batch; ++j) {
       ok[j] = match_front(m, cam, mod, live.v[j], live.n[j], src[j], mi[j]);
-      ok[j] = ok[j] & (base + j * stride < n);
+      ok[j] = ok[j] && base + j * stride < n;
     }
 #pragma unroll
     for (int j = 0; j < Batch; ++j) {

@@ -789,6 +789,7 @@ class Scratch {
 struct kf_mesh {
   void* block = nullptr;
   size_t vertices = 0, triangles = 0;
+  std::shared_ptr<kf::HostStage> stage;
   float* positions() const { return static_cast<float*>(block); }
   float* normals() const { return positions() + 3 * vertices; }
   float* colors() const { return normals() + 3 * vertices; }
@@ -951,6 +952,7 @@ kf_status kf_mesh_extract(kf_context* ctx, float min_weight, kf_mesh** out) {
   *out = nullptr;
   auto* mesh = new (std::nothrow) kf_mesh();
   if (mesh == nullptr) return KF_ERR_OUT_OF_MEMORY;
+  mesh->stage = ctx->stage;
   kf_status status = KF_OK;
   auto attempt = [&](auto&& body) {
     try {
@@ -996,13 +998,12 @@ kf_status kf_mesh_size(const kf_mesh* mesh, int64_t* vertices, int64_t* triangle
 
 kf_status kf_mesh_copy(const kf_mesh* mesh, float* positions, float* normals, float* colors, uint32_t* triangles) {
   if (mesh == nullptr) return KF_ERR_INVALID_ARGUMENT;
-  const auto copy = [](void* to, const void* from, size_t bytes) {
-    return to == nullptr || bytes == 0 || hipMemcpy(to, from, bytes, hipMemcpyDeviceToHost) == hipSuccess;
-  };
   const size_t v = 12 * mesh->vertices;
-  const bool ok = copy(positions, mesh->positions(), v) && copy(normals, mesh->normals(), v) &&
-                  copy(colors, mesh->colors(), v) && copy(triangles, mesh->faces(), 12 * mesh->triangles);
-  return ok ? KF_OK : KF_ERR_DEVICE;
+  const HostStage::Piece out[4] = {{positions, mesh->positions(), v},
+                                   {normals, mesh->normals(), v},
+                                   {colors, mesh->colors(), v},
+                                   {triangles, mesh->faces(), 12 * mesh->triangles}};
+  return mesh->stage->copy(out, 4, nullptr) == hipSuccess ? KF_OK : KF_ERR_DEVICE;
 }
 
 void kf_mesh_free(kf_mesh* mesh) { delete mesh; }

@@ -721,6 +721,7 @@ int blocks_for(long long n, int per = 256) { return static_cast<int>((n + per - 
 struct kf_posenet {
   kf_posenet_config cfg{};
   std::string error;
+  kf::HostStage stage;
   hipStream_t stream = nullptr;
   std::vector<Shape> shapes;
   size_t n_params = 0;
@@ -1190,8 +1191,8 @@ const char* kf_posenet_last_error(const kf_posenet* net) {
 kf_status kf_posenet_get_parameters(kf_posenet* net, float* params) {
   return net_guard(net, [&] {
     if (net == nullptr || params == nullptr) fail(KF_ERR_INVALID_ARGUMENT, "null argument");
-    KF_HIP(hipMemcpyAsync(params, net->w, net->n_params * sizeof(float), hipMemcpyDeviceToHost, net->stream));
-    KF_HIP(hipStreamSynchronize(net->stream));
+    const kf::HostStage::Piece out{params, net->w, net->n_params * sizeof(float)};
+    KF_HIP(net->stage.copy(&out, 1, net->stream));
   });
 }
 
@@ -1229,10 +1230,8 @@ kf_status kf_posenet_gradients(kf_posenet* net, const uint16_t* pairs, const flo
     forward(net, net->stream, batch);
     backward(net, net->stream, targets, batch);
     KF_HIP(hipMemcpyAsync(net->loss_host, net->loss, sizeof(float), hipMemcpyDeviceToHost, net->stream));
-    if (grads != nullptr) {
-      KF_HIP(hipMemcpyAsync(grads, net->grad, net->n_params * sizeof(float), hipMemcpyDeviceToHost, net->stream));
-    }
-    KF_HIP(hipStreamSynchronize(net->stream));
+    const kf::HostStage::Piece out{grads, net->grad, net->n_params * sizeof(float)};
+    KF_HIP(net->stage.copy(&out, 1, net->stream));
     if (loss != nullptr) *loss = *net->loss_host;
   });
 }
