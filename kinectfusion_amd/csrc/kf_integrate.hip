@@ -17,6 +17,7 @@
 //  3. integrate   -- persistent waves walk the list, one brick per wave: a
 //     lane owns an (x, y) column of 8 voxels, and each z-slice of the brick
 //     is 4 rows of 16 contiguous voxels.
+#include <cmath>
 #include <type_traits>
 
 #include "kf_internal.hpp"
@@ -40,6 +41,9 @@ struct FrameParams {
   // to skip) to frame_w2c once; the later launches read them.
   const IcpState* st;
   float* frame_w2c;
+  // How near the nearest pixel's centre an approximate projection decides it
+  // (fuse_column): half a pixel less a margin, per axis.
+  float near_u, near_v;
 };
 
 // world_to_camera of this frame (false: the frame failed, skip the pass).
@@ -321,8 +325,9 @@ __device__ inline bool same_raw(Raw a, Raw b) {
   }
 }
 
-// observe + fuse (tsdf_integration.hpp:184-252) of N voxels of one thread,
-// in phases so that the N pixel-record loads, then the N voxel loads, are in
+// observe + fuse (tsdf_integration.hpp:184-252) of N voxels of a z-column, from
+// z0 (the same for the whole wave) at vox[first], vox[first + stride], ..., in
+// phases so that the N pixel-record loads, then the N voxel loads, are in
 // flight together: (1) project, (2) read the pixel records, (3) decide,
 // (4) read the voxels, (5) update.  any: some voxel fused; ones_ok: every
 // fused voxel reads tsdf exactly 1 afterwards; complete: every voxel was
@@ -332,18 +337,27 @@ __device__ inline bool same_raw(Raw a, Raw b) {
 // complete now or the part was free before (an unfused voxel keeps its
 // value).
 //
-// Most voxels are decided without IEEE divisions: the projection and the
-// signed distance are first computed with the hardware reciprocal and square
-// root (relative error below 2^-21), and the exact IEEE computation runs only
-// when an approximate value lies within a safety margin of a decision
-// boundary (a half-integer pixel coordinate, -truncation, +truncation).  Away
-// from the boundaries the approximate value decides the same way as the exact
-// one, so the outcome is bit-identical:
-//  * the pixel: lround(u) = floor(u' + 0.5) when u' is farther than
-//    3e-4 + 2e-6 |q'| from a half-integer (q' = fx x / z): u' differs from
-//    the exact float u by less than 2e-6 |q'| (the reciprocal and two
-//    roundings) plus the float rounding of both (below 1.3e-4 wherever the
-//    pixel can be in the image, |u| < 1024); farther out both land outside;
+// What bounds it: the reads' latencies (pixel, voxel, colour) and the
+// instructions between them, about evenly: a 512^3 room frame moves 130 MB in
+// 54 us, 26 at a copy's rate, with the vector units issuing 7 cycles in 10.
+// Batches of 8 (62 us) or 2 (57) lose more waves, or more reads in flight, than
+// they gain.  Branch-free projection, the colours of a batch read together and
+// flags written only where they change took 58 us to 54, and 61 to 54 with
+// float voxels.
+//
+// Most voxels are decided without IEEE divisions and square roots: the
+// projection and the signed distance are first computed with the hardware
+// reciprocal and square root (relative error below 2^-21), and the exact
+// computation runs only when an approximate value lies within a safety margin
+// of a decision boundary (a half-integer pixel coordinate, -truncation,
+// +truncation).  Away from the boundaries the approximate value decides the
+// same way as the exact one, so the outcome is bit-identical:
+//  * the pixel: lround(u) is the integer n nearest u' when |u' - n| is less than
+//    half less 3e-4 + 2e-6 Q, Q the largest |q'| = |fx x / z| of a pixel of the
+//    image: u' differs from the exact float u by less than 2e-6 |q'| (the
+//    reciprocal and two roundings) plus the float rounding of both (below
+//    1.3e-4 for |u| < 1024, and within 2e-6 Q farther out); where |q'| is
+//    larger both land outside;
 //  * sd >= truncation (free space): tsdf = clamp(sd / trunc) = 1 exactly and
 //    no colour; the update ((t0 w0) + (1 w)) / (w0 + w) is 1 exactly when
 //    t0 = 1 (numerator and denominator are the same rounded sum), so the
@@ -351,103 +365,93 @@ __device__ inline bool same_raw(Raw a, Raw b) {
 //  * sd < -truncation: rejected.
 // A voxel whose stored bits do not change (saturated free space) is not
 // written back.
-template <int Kind, bool Color, bool Count, int N, bool Column = false>
-__device__ inline void fuse_batch(const Grid& g, const FrameParams& f, const Rigid& w2c,
-                                  const float4* __restrict__ pix, const uint32_t* __restrict__ color_img,
-                                  typename VoxelIO<Kind>::Raw* __restrict__ vox, float4* __restrict__ colors,
-                                  const int (&xs)[N], const int (&ys)[N], const int (&zs)[N],
-                                  const size_t (&vis)[N], const bool (&inside)[N], unsigned int& my_fused,
-                                  unsigned int& my_color, bool& any, bool& ones_ok, bool& complete) {
+template <int Kind, bool Color, bool Count, int N>
+__device__ __forceinline__ void fuse_column(const Grid& g, const FrameParams& f, const Rigid& w2c,
+                                            const float4* __restrict__ pix, const uint32_t* __restrict__ color_img,
+                                            typename VoxelIO<Kind>::Raw* __restrict__ vox,
+                                            float4* __restrict__ colors, int x, int y, int z0, size_t first,
+                                            size_t stride, unsigned int& my_fused, unsigned int& my_color, bool& any,
+                                            bool& ones_ok, bool& complete) {
   using IO = VoxelIO<Kind>;
+  // the same float sequence as xform(w2c, centre): ((r.x cx + r.y cy) + r.z cz) + t
+  const float cx = g.ox + ((static_cast<float>(x) + 0.5F) * g.voxel);
+  const float cy = g.oy + ((static_cast<float>(y) + 0.5F) * g.voxel);
+  const float a0 = (w2c.r0.x * cx) + (w2c.r0.y * cy);
+  const float a1 = (w2c.r1.x * cx) + (w2c.r1.y * cy);
+  const float a2 = (w2c.r2.x * cx) + (w2c.r2.y * cy);
+  const float last_u = static_cast<float>(f.w - 1), last_v = static_cast<float>(f.h - 1);
   int pi[N];
   V3 cp[N];
-  // A column (every voxel at the same x, y): the voxel centre's x and y and
-  // each row's first two products and their sum are the same for all of
-  // them, so they are formed once; the rest of xform(w2c, centre) is the
-  // same float sequence: ((r.x cx + r.y cy) + r.z cz) + t.
-  float a0 = 0.0F, a1 = 0.0F, a2 = 0.0F;
-  if constexpr (Column) {
-    const float cx = g.ox + ((static_cast<float>(xs[0]) + 0.5F) * g.voxel);
-    const float cy = g.oy + ((static_cast<float>(ys[0]) + 0.5F) * g.voxel);
-    a0 = (w2c.r0.x * cx) + (w2c.r0.y * cy);
-    a1 = (w2c.r1.x * cx) + (w2c.r1.y * cy);
-    a2 = (w2c.r2.x * cx) + (w2c.r2.y * cy);
+  bool hit[N], slow[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const float cz = g.oz + ((static_cast<float>(z0 + k) + 0.5F) * g.voxel);
+    cp[k] = mk3((a0 + (w2c.r0.z * cz)) + w2c.t.x, (a1 + (w2c.r1.z * cz)) + w2c.t.y, (a2 + (w2c.r2.z * cz)) + w2c.t.z);
+    const bool front = z0 + k < g.nz && cp[k].z > 0.0F;
+    const float rz = __builtin_amdgcn_rcpf(cp[k].z);
+    const float u = __builtin_fmaf(f.k.fx * cp[k].x, rz, f.k.cx), v = __builtin_fmaf(f.k.fy * cp[k].y, rz, f.k.cy);
+    const float nu = __builtin_rintf(u), nv = __builtin_rintf(v);
+    const bool near = fabsf(u - nu) < f.near_u && fabsf(v - nv) < f.near_v;  // a NaN is not
+    const float iu = __builtin_amdgcn_fmed3f(nu, 0.0F, last_u), iv = __builtin_amdgcn_fmed3f(nv, 0.0F, last_v);
+    pi[k] = static_cast<int>(iv) * f.w + static_cast<int>(iu);
+    hit[k] = front && near && iu == nu && iv == nv;
+    slow[k] = front && !near;
   }
 #pragma unroll
   for (int k = 0; k < N; ++k) {
-    pi[k] = -1;
-    cp[k] = mk3(0.0F, 0.0F, 0.0F);
-    if (!inside[k]) continue;
-    if constexpr (Column) {
-      const float cz = g.oz + ((static_cast<float>(zs[k]) + 0.5F) * g.voxel);
-      cp[k] = mk3((a0 + (w2c.r0.z * cz)) + w2c.t.x, (a1 + (w2c.r1.z * cz)) + w2c.t.y, (a2 + (w2c.r2.z * cz)) + w2c.t.z);
-    } else {
-      cp[k] = xform(w2c, g.center(xs[k], ys[k], zs[k]));
-    }
-    if (cp[k].z <= 0.0F) continue;
-    const float rz = __builtin_amdgcn_rcpf(cp[k].z);
-    const float qx = (f.k.fx * cp[k].x) * rz, qy = (f.k.fy * cp[k].y) * rz;
-    const float ua = qx + f.k.cx, va = qy + f.k.cy;
-    // the nearest pixel; u' lies within the margin of a half-integer when
-    // |u' - n| >= 0.5 - margin (a NaN projection fails the test too)
-    const float nu = floorf(ua + 0.5F), nv = floorf(va + 0.5F);
-    const bool fast = fabsf(ua - nu) < (0.5F - 3.0e-4F) - 2.0e-6F * fabsf(qx) &&
-                      fabsf(va - nv) < (0.5F - 3.0e-4F) - 2.0e-6F * fabsf(qy);
+    if (!slow[k]) continue;
+    float u, v;
     int col, row;
-    if (!fast) {
-      float u, v;
-      project(f.k, cp[k], u, v);
-      if (!round_index(u, f.w, col) || !round_index(v, f.h, row)) continue;
-    } else {
-      col = static_cast<int>(nu);
-      row = static_cast<int>(nv);
-      if (col < 0 || col >= f.w || row < 0 || row >= f.h) continue;
-    }
+    project(f.k, cp[k], u, v);
+    if (!round_index(u, f.w, col) || !round_index(v, f.h, row)) continue;
     pi[k] = row * f.w + col;
+    hit[k] = true;
   }
   float4 p[N];
 #pragma unroll
-  for (int k = 0; k < N; ++k) p[k] = pi[k] >= 0 ? pix[pi[k]] : make_float4(-1.0F, 1.0F, 0.0F, 1.0F);
+  for (int k = 0; k < N; ++k) p[k] = pix[pi[k]];
   // mode: 0 no fuse, 1 free space (tsdf 1, no colour), 2 in the band (exact
   // sd), 3 no fuse at an in-image pixel without depth: the voxel is read
   // only to learn whether it already holds an observed 1 (a depth dropout
   // inside free space then does not break the part's completeness).
-  // The decisions are selects; only voxels whose approximate distance lies
-  // within a margin of the band take the exact (IEEE) path.
   int mode[N];
   float sd[N];
-  bool exact[N];
+  bool band[N];
 #pragma unroll
   for (int k = 0; k < N; ++k) {
-    const bool has_depth = !(p[k].x < 0.0F || p[k].z <= 0.0F);  // no depth, or w <= 0 drops the fuse
-    int m = (!has_depth && pi[k] >= 0) ? 3 : 0;
-    float s = 0.0F;
-    bool ex = false;
-    if (f.projective) {
-      const float sa = __builtin_amdgcn_sqrtf(dot3(cp[k], cp[k])) * __builtin_amdgcn_rcpf(p[k].y);
-      const float sda = p[k].x - sa;
-      const float margin = 1.0e-6F + 4.0e-6F * sa;
-      const bool fr = sda >= p[k].w + margin;
-      const bool rj = sda < -p[k].w - margin;
-      m = has_depth ? (fr ? 1 : (rj ? 0 : 2)) : m;
-      ex = has_depth && !fr && !rj;
-    } else {
-      s = p[k].x - cp[k].z;
-      m = has_depth ? (s >= p[k].w ? 1 : (s < -p[k].w ? 0 : 2)) : m;
-    }
-    mode[k] = m;
-    sd[k] = s;
-    exact[k] = ex;
+    const bool weighs = hit[k] && !(p[k].x < 0.0F || p[k].z <= 0.0F);  // no depth, or w <= 0, drops the fuse
+    const float sa = __builtin_amdgcn_sqrtf(dot3(cp[k], cp[k])) * __builtin_amdgcn_rcpf(p[k].y);
+    const float sda = p[k].x - sa, margin = 1.0e-6F + 4.0e-6F * sa;
+    const bool free = f.projective != 0 && sda >= p[k].w + margin;
+    const bool behind = f.projective != 0 && sda < -p[k].w - margin;
+    band[k] = weighs && !free && !behind;
+    mode[k] = weighs ? (free ? 1 : 0) : (hit[k] ? 3 : 0);
+    sd[k] = 0.0F;
   }
 #pragma unroll
   for (int k = 0; k < N; ++k) {
-    if (!exact[k]) continue;
-    sd[k] = p[k].x - (norm3(cp[k]) / p[k].y);
-    if (sd[k] < -p[k].w) mode[k] = 0;
+    if (!band[k]) continue;
+    sd[k] = p[k].x - (f.projective != 0 ? norm3(cp[k]) / p[k].y : cp[k].z);
+    mode[k] = f.projective == 0 && sd[k] >= p[k].w ? 1 : (sd[k] < -p[k].w ? 0 : 2);
   }
   typename IO::Raw raw[N];
 #pragma unroll
-  for (int k = 0; k < N; ++k) raw[k] = mode[k] != 0 ? vox[vis[k]] : IO::fresh();
+  for (int k = 0; k < N; ++k) raw[k] = mode[k] != 0 ? vox[first + k * stride] : IO::fresh();
+  bool tinted[N];
+  uint32_t px[N];
+  float4 old[N];
+  if constexpr (Color) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      tinted[k] = mode[k] == 2 && color_img != nullptr && sd[k] <= p[k].w * 0.5F;
+      px[k] = 0;
+      old[k] = make_float4(0.0F, 0.0F, 0.0F, 0.0F);
+      if (tinted[k]) {
+        px[k] = color_img[pi[k]];
+        old[k] = colors[first + k * stride];
+      }
+    }
+  }
   ones_ok = true;
   complete = true;
 #pragma unroll
@@ -473,63 +477,33 @@ __device__ inline void fuse_batch(const Grid& g, const FrameParams& f, const Rig
     }
     const float tw = fmin_ref(w0 + w, f.max_weight);
     const typename IO::Raw nv = IO::pack(avg, tw);
-    if (!same_raw(nv, raw[k])) vox[vis[k]] = nv;
+    if (!same_raw(nv, raw[k])) vox[first + k * stride] = nv;
     IO::unpack(nv, t0, w0, obs, fin);
     ones_ok = ones_ok && t0 == 1.0F;
     any = true;
     if (Count) ++my_fused;
-    if (Color && mode[k] == 2) {
-      if (color_img != nullptr && sd[k] <= p[k].w * 0.5F) {
-        const uint32_t px = color_img[pi[k]];
-        const V3 c = mk3(static_cast<float>(px & 0xFFU), static_cast<float>((px >> 8U) & 0xFFU),
-                         static_cast<float>((px >> 16U) & 0xFFU));
-        const float4 old = colors[vis[k]];
-        const float cw = old.w;
+    if constexpr (Color) {
+      if (tinted[k]) {
+        const V3 c = mk3(static_cast<float>(px[k] & 0xFFU), static_cast<float>((px[k] >> 8U) & 0xFFU),
+                         static_cast<float>((px[k] >> 16U) & 0xFFU));
+        const float cw = old[k].w;
         const float den = cw + w;
-        colors[vis[k]] = make_float4(((old.x * cw) + (c.x * w)) / den, ((old.y * cw) + (c.y * w)) / den,
-                                     ((old.z * cw) + (c.z * w)) / den, fmin_ref(cw + w, f.max_weight));
+        colors[first + k * stride] =
+            make_float4(((old[k].x * cw) + (c.x * w)) / den, ((old[k].y * cw) + (c.y * w)) / den,
+                        ((old[k].z * cw) + (c.z * w)) / den, fmin_ref(cw + w, f.max_weight));
         if (Count) ++my_color;
       }
     }
   }
 }
 
-// The voxel updates of one z-part (4 voxels from z0) of an (x, y) column.
-template <int Kind, bool Color, bool Count>
-__device__ inline bool integrate_column(const Grid& g, const FrameParams& f, const Rigid& w2c,
-                                        const float4* __restrict__ pix, const uint32_t* __restrict__ color_img,
-                                        typename VoxelIO<Kind>::Raw* __restrict__ vox,
-                                        float4* __restrict__ colors, int x, int y, int z0,
-                                        unsigned int& my_fused, unsigned int& my_color, bool& ones_ok,
-                                        bool& complete) {
-  constexpr int kHalf = kBrickZ / 2;  // one z-part of a block
-  int xs[kHalf], ys[kHalf], zs[kHalf];
-  size_t vis[kHalf];
-  bool inside[kHalf];
-  const size_t v0 = g.flat(x, y, z0), slice = static_cast<size_t>(g.nx) * static_cast<size_t>(g.ny);
-#pragma unroll
-  for (int k = 0; k < kHalf; ++k) {
-    xs[k] = x;
-    ys[k] = y;
-    zs[k] = z0 + k;
-    inside[k] = zs[k] < g.nz;
-    vis[k] = inside[k] ? v0 + k * slice : 0;
-  }
-  bool any = false;
-  fuse_batch<Kind, Color, Count, kHalf, true>(g, f, w2c, pix, color_img, vox, colors, xs, ys, zs, vis, inside,
-                                              my_fused, my_color, any, ones_ok, complete);
-  return any;
-}
-
 // Part bits of block fb: bit `part` (y-half * 2 + z-half) of its nibble.
-__device__ inline void set_part(uint32_t* part_bits, int fb, int part, bool on) {
-  const uint32_t bit = 1U << ((fb & 7) * 4 + part);
-  if (on) atomicOr(&part_bits[fb >> 3], bit);
-  else atomicAnd(&part_bits[fb >> 3], ~bit);
-}
+__device__ inline uint32_t part_bit(int fb, int part) { return 1U << ((fb & 7) * 4 + part); }
 
+// 8 waves per SIMD without colours (62 us for 66 in a hashed hall); with them
+// that many would spill (91 us for 54).
 template <int Kind, bool Color, bool Count>
-__global__ void __launch_bounds__(256) integrate_kernel(Grid g, FrameParams f,
+__global__ void __launch_bounds__(256, Color ? 1 : 8) integrate_kernel(Grid g, FrameParams f,
                                                          const float4* __restrict__ pix,
                                                          const uint32_t* __restrict__ color_img,
                                                          typename VoxelIO<Kind>::Raw* __restrict__ vox,
@@ -543,6 +517,8 @@ __global__ void __launch_bounds__(256) integrate_kernel(Grid g, FrameParams f,
   // (x = lane % 16, y = lane / 16) owns the brick's z-column of 8 voxels,
   // both z-halves of its block.  Lanes 8j .. 8j + 7 of each 16 are block j's
   // row (j = 0, 1), so kBlockRows selects block j's 32 lanes of a ballot.
+  // Lane = z-half h * 2 + block j (lanes < 4) keeps part (y-half, h) of block
+  // j, and j's observed bit.
   constexpr unsigned long long kBlockRows = 0x00FF00FF00FF00FFULL;
   Rigid w2c;
   if (!block_w2c(f, w2c)) return;
@@ -552,31 +528,38 @@ __global__ void __launch_bounds__(256) integrate_kernel(Grid g, FrameParams f,
   const uint32_t waves = gridDim.x * (blockDim.x >> 6);
   unsigned int my_fused = 0, my_color = 0;
   for (uint32_t li = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); li < n; li += waves) {
-    const uint32_t b = list[li];
+    const uint32_t b = __builtin_amdgcn_readfirstlane(list[li]);  // the wave's: its slices are scalars
     const int bx = static_cast<int>(b & 0xFFU), by = static_cast<int>((b >> 8U) & 0x3FFU),
               bz = static_cast<int>(b >> 18U);
     const int x = bx * kBrickX + tx, y = by * kBrickY + ty, z0 = bz * kBrickZ;
+    // The flags as they stand, read ahead: in most frames few change, and an
+    // atomic to a word that other waves' blocks share costs more than a read
+    // (8 of 58 us).  A part's bit is this wave's alone in the launch; an
+    // observed bit that another wave has just set is set again.
+    const int j = lane & 1, h = lane >> 1, blk_x = bx * 2 + j;
+    const bool mine = lane < 4 && blk_x < bm.bx;
+    const int fb = mine ? bm.flat(blk_x, (by * kBrickY) >> 3, z0 >> 3) : 0;
+    const uint32_t bit = part_bit(fb, (((by * kBrickY) >> 2) & 1) * 2 + (h & 1));
+    const uint32_t parts = part_bits[fb >> 3], observed = obs_bits[fb >> 5];
     bool any0 = false, any1 = false, ok0 = false, ok1 = false, cpl0 = false, cpl1 = false;
     if (x < g.nx && y < g.ny) {
-      any0 = integrate_column<Kind, Color, Count>(g, f, w2c, pix, color_img, vox, colors, x, y, z0, my_fused,
-                                                  my_color, ok0, cpl0);
-      any1 = integrate_column<Kind, Color, Count>(g, f, w2c, pix, color_img, vox, colors, x, y, z0 + kBrickZ / 2,
-                                                  my_fused, my_color, ok1, cpl1);
+      constexpr int kHalf = kBrickZ / 2;  // one z-part of a block
+      const size_t slice = static_cast<size_t>(g.nx) * static_cast<size_t>(g.ny), v0 = g.flat(x, y, z0);
+      fuse_column<Kind, Color, Count, kHalf>(g, f, w2c, pix, color_img, vox, colors, x, y, z0, v0, slice,
+                                             my_fused, my_color, any0, ok0, cpl0);
+      fuse_column<Kind, Color, Count, kHalf>(g, f, w2c, pix, color_img, vox, colors, x, y, z0 + kHalf,
+                                             v0 + kHalf * slice, slice, my_fused, my_color, any1, ok1, cpl1);
     }
     const unsigned long long om0 = __ballot(ok0), cm0 = __ballot(cpl0), om1 = __ballot(ok1),
                              cm1 = __ballot(cpl1), am = __ballot(any0 || any1);
-    if (lane < 4) {
-      // lane = z-half h * 2 + block j: part (y-half, h) of block j, and j's observed bit
-      const int j = lane & 1, h = lane >> 1;
-      const int blk_x = bx * 2 + j;
-      if (blk_x < bm.bx) {
-        const unsigned long long rows = kBlockRows << (8 * j);
-        const int fb = bm.flat(blk_x, (by * kBrickY) >> 3, z0 >> 3);
-        const bool ok = ((h != 0 ? om1 : om0) & rows) == rows, cpl = ((h != 0 ? cm1 : cm0) & rows) == rows;
-        const int part = (((by * kBrickY) >> 2) & 1) * 2 + h;
-        if (!ok || cpl) set_part(part_bits, fb, part, ok);
-        if (h == 0 && (am & rows) != 0ULL) atomicOr(&obs_bits[fb >> 5], 1U << (fb & 31));
-      }
+    if (mine) {
+      const unsigned long long rows = kBlockRows << (8 * j);
+      const bool ok = ((h != 0 ? om1 : om0) & rows) == rows, cpl = ((h != 0 ? cm1 : cm0) & rows) == rows;
+      const bool on = (parts & bit) != 0U;
+      if (ok && cpl && !on) atomicOr(&part_bits[fb >> 3], bit);
+      if (!ok && on) atomicAnd(&part_bits[fb >> 3], ~bit);
+      const uint32_t seen = 1U << (fb & 31);
+      if (h == 0 && (am & rows) != 0ULL && (observed & seen) == 0U) atomicOr(&obs_bits[fb >> 5], seen);
     }
   }
   if (Count) {
@@ -1097,8 +1080,9 @@ __global__ void __launch_bounds__(256) assign_slots_kernel(HashView hv, const ui
 // pool slot's 512.  Dense band: the list holds block keys and voxels sit at
 // their dense indices.  n: the list's length.
 template <int Kind, bool Color, bool Count, bool Dense>
-__global__ void __launch_bounds__(256) integrate_blocks_kernel(Grid g, FrameParams f, const float4* __restrict__ pix,
-                                                                const uint32_t* __restrict__ color_img,
+__global__ void __launch_bounds__(256, Color ? 1 : 8) integrate_blocks_kernel(Grid g, FrameParams f,
+                                                                const float4* __restrict__ pix,
+                                                                       const uint32_t* __restrict__ color_img,
                                                                 typename VoxelIO<Kind>::Raw* __restrict__ pool,
                                                                 float4* __restrict__ cpool,
                                                                 const uint32_t* __restrict__ block_of_slot,
@@ -1114,43 +1098,37 @@ __global__ void __launch_bounds__(256) integrate_blocks_kernel(Grid g, FramePara
   const uint32_t waves = gridDim.x * 4U;
   unsigned int my_fused = 0, my_color = 0;
   for (uint32_t li = blockIdx.x * 4U + (threadIdx.x >> 6); li < n; li += waves) {
-    const uint32_t slot = work[li];
-    const uint32_t key = Dense ? slot : block_of_slot[slot];
+    const uint32_t slot = __builtin_amdgcn_readfirstlane(work[li]);  // the wave's: its slices are scalars
+    const uint32_t key = Dense ? slot : __builtin_amdgcn_readfirstlane(block_of_slot[slot]);
     const int bx = static_cast<int>(key % static_cast<uint32_t>(bm.bx));
     const int by = static_cast<int>((key / static_cast<uint32_t>(bm.bx)) % static_cast<uint32_t>(bm.by));
     const int bz = static_cast<int>(key / static_cast<uint32_t>(bm.bx * bm.by));
     const int x = bx * 8 + (lane & 7), y = by * 8 + (lane >> 3);
+    const int fb = bm.flat(bx, by, bz);
+    const uint32_t parts = part_bits[fb >> 3], observed = obs_bits[fb >> 5];
     bool any = false, ones_ok = true, complete = true;
+    if (x < g.nx && y < g.ny) {
+      const size_t stride = Dense ? static_cast<size_t>(g.nx) * static_cast<size_t>(g.ny) : 64;
+      const size_t first = Dense ? g.flat(x, y, bz * 8) : static_cast<size_t>(slot) * kBlockVoxels + lane;
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      int xs[4], ys[4], zs[4];
-      size_t vis[4];
-      bool inside[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int zi = half * 4 + k;
-        xs[k] = x;
-        ys[k] = y;
-        zs[k] = bz * 8 + zi;
-        inside[k] = x < g.nx && y < g.ny && zs[k] < g.nz;
-        if constexpr (Dense) vis[k] = inside[k] ? g.flat(x, y, zs[k]) : 0;
-        else vis[k] = static_cast<size_t>(slot) * kBlockVoxels + static_cast<size_t>(zi * 64 + lane);
+      for (int half = 0; half < 2; ++half) {
+        bool a = false, o = true, c = true;
+        fuse_column<Kind, Color, Count, 4>(g, f, w2c, pix, color_img, pool, cpool, x, y, bz * 8 + half * 4,
+                                           first + half * 4 * stride, stride, my_fused, my_color, a, o, c);
+        any = any || a;
+        ones_ok = ones_ok && o;
+        complete = complete && c;
       }
-      bool a = false, o = true, c = true;
-      fuse_batch<Kind, Color, Count, 4, true>(g, f, w2c, pix, color_img, pool, cpool, xs, ys, zs, vis, inside,
-                                              my_fused, my_color, a, o, c);
-      any = any || a;
-      ones_ok = ones_ok && o;
-      complete = complete && c;
+    } else {
+      complete = false;
     }
     const bool any_fused = __ballot(any) != 0ULL, all_ok = __ballot(!ones_ok) == 0ULL,
                all_complete = __ballot(!complete) == 0ULL;
-    if (lane == 0) {
-      const int fb = bm.flat(bx, by, bz);
-      if (any_fused) atomicOr(&obs_bits[fb >> 5], 1U << (fb & 31));
-      const uint32_t nib = 0xFU << ((fb & 7) * 4);
-      if (!all_ok) atomicAnd(&part_bits[fb >> 3], ~nib);
-      else if (all_complete) atomicOr(&part_bits[fb >> 3], nib);  // else unchanged
+    if (lane == 0) {  // the block's flags are this wave's alone: only what changes is written
+      const uint32_t seen = 1U << (fb & 31), nib = 0xFU << ((fb & 7) * 4);
+      if (any_fused && (observed & seen) == 0U) atomicOr(&obs_bits[fb >> 5], seen);
+      if (!all_ok && (parts & nib) != 0U) atomicAnd(&part_bits[fb >> 3], ~nib);
+      if (all_ok && all_complete && (parts & nib) != nib) atomicOr(&part_bits[fb >> 3], nib);
     }
   }
   if (Count) {
@@ -1443,6 +1421,8 @@ void launch_integrate(kf_context* ctx, const kf_depth_frame& fr, bool count, boo
   f.angle_rule = c.tsdf_rule == KF_RULE_ANGLE_WEIGHTED;
   f.st = from_state ? ctx->icp : nullptr;
   f.frame_w2c = ctx->frame_w2c;
+  f.near_u = 0.5F - (3.0e-4F + 2.0e-6F * (std::fmax(std::fabs(fr.cx), std::fabs(fr.width - fr.cx)) + 1.0F));
+  f.near_v = 0.5F - (3.0e-4F + 2.0e-6F * (std::fmax(std::fabs(fr.cy), std::fabs(fr.height - fr.cy)) + 1.0F));
   const int tiles_x = (f.w + kTile - 1) / kTile, tiles_y = (f.h + kTile - 1) / kTile;
   // per-pixel and per-tile scratch is sized for the configured camera
   if (f.w > c.width || f.h > c.height)
