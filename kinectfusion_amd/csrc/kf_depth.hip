@@ -24,6 +24,11 @@ constexpr int kMaxRadius = 8;
 // relative error below 4e-16, the table staged in LDS) and rounded to
 // float, which matches a correctly rounded expf.
 //
+// What bounds it: vector issue, 32 instructions a tap (49 taps at radius 3),
+// 12 of the 17 us a 640 x 480 frame takes.  Fused sums in the exponential, its
+// reduction in float and its power of two applied to the float took 24 us to
+// 17.  Interleaving a row's exponentials by hand gained nothing.
+//
 // R > 0: the window's radius fixed at compile time and each row's taps
 // unrolled, so their exponentials overlap; the sums still add the taps in the
 // reference's row-major order, an unusable tap (outside the image or without
@@ -38,8 +43,7 @@ __global__ void __launch_bounds__(256) bilateral_kernel(const uint16_t* __restri
                                                          float scale, float lo, float hi, int radius_arg,
                                                          float ss, float sr, StageCopy stage) {
   const int radius = R > 0 ? R : radius_arg;
-  __shared__ float meters[(kTy + 2 * kMaxRadius) * (kTx + 2 * kMaxRadius)];
-  __shared__ float raws[(kTy + 2 * kMaxRadius) * (kTx + 2 * kMaxRadius)];
+  __shared__ float2 samples[(kTy + 2 * kMaxRadius) * (kTx + 2 * kMaxRadius)];  // metres (-1: unusable), raw
   __shared__ double exp_table[64];
   const int tw = kTx + 2 * radius, th = kTy + 2 * radius;
   const int x0 = blockIdx.x * kTx - radius, y0 = blockIdx.y * kTy - radius;
@@ -57,8 +61,7 @@ __global__ void __launch_bounds__(256) bilateral_kernel(const uint16_t* __restri
         r = static_cast<float>(raw);
       }
     }
-    meters[i] = m;  // -1 marks an unusable sample
-    raws[i] = r;
+    samples[i] = make_float2(m, r);
   }
   __syncthreads();
   const int col = blockIdx.x * kTx + threadIdx.x, row = blockIdx.y * kTy + threadIdx.y;
@@ -69,23 +72,30 @@ __global__ void __launch_bounds__(256) bilateral_kernel(const uint16_t* __restri
     if (stage.color_in != nullptr) stage.color[i] = stage.color_in[i];
   }
   const int cl = (threadIdx.y + radius) * tw + threadIdx.x + radius;
-  const float cm = meters[cl];
+  const float cm = samples[cl].x;
   uint16_t result = 0;
   if (R > 0 && cm >= 0.0F) {
     float wsum_v = 0.0F, wsum = 0.0F;
 #pragma unroll 1
     for (int dy = -R; dy <= R; ++dy) {
       const int base = (threadIdx.y + R + dy) * tw + threadIdx.x + R;
+      constexpr int N = 2 * R + 1;
+      float2 sample[N];
 #pragma unroll
-      for (int dx = -R; dx <= R; ++dx) {
-        const float sm = meters[base + dx];
+      for (int i = 0; i < N; ++i) sample[i] = samples[base + i - R];
+      float wt[N];
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const int dx = i - R;
         const float pd2 = static_cast<float>((dx * dx) + (dy * dy));
-        const float dd = sm - cm;
-        const float e = (pd2 * ss) + (dd * dd * sr);
-        const float wt = static_cast<float>(exp_nonpositive(static_cast<double>(e), exp_table));
-        const bool use = sm >= 0.0F;
-        wsum_v += use ? wt * raws[base + dx] : 0.0F;
-        wsum += use ? wt : 0.0F;
+        const float dd = sample[i].x - cm;
+        wt[i] = exp_weight((pd2 * ss) + (dd * dd * sr), exp_table);
+      }
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const bool use = sample[i].x >= 0.0F;
+        wsum_v += use ? wt[i] * sample[i].y : 0.0F;
+        wsum += use ? wt[i] : 0.0F;
       }
     }
     if (wsum > 0.0F) result = static_cast<uint16_t>(static_cast<long>(roundf(wsum_v / wsum)));
@@ -96,14 +106,15 @@ __global__ void __launch_bounds__(256) bilateral_kernel(const uint16_t* __restri
     for (int y = yb; y <= ye; ++y) {
       const int base = (y - y0) * tw - x0;
       for (int x = xb; x <= xe; ++x) {
-        const float sm = meters[base + x];
+        const float2 sample = samples[base + x];
+        const float sm = sample.x;
         if (sm < 0.0F) continue;
         const float pd2 =
             static_cast<float>(((x - col) * (x - col)) + ((y - row) * (y - row)));
         const float dd = sm - cm;
         const float e = (pd2 * ss) + (dd * dd * sr);
-        const float wt = static_cast<float>(exp_nonpositive(static_cast<double>(e), exp_table));
-        wsum_v += wt * raws[base + x];
+        const float wt = exp_weight(e, exp_table);
+        wsum_v += wt * sample.y;
         wsum += wt;
       }
     }
@@ -218,7 +229,10 @@ __global__ void __launch_bounds__(256) vertex_normal_kernel(const uint16_t* __re
 // level 1 and 32 x 16 of level 0; it stages level-0 depth with a 4-pixel
 // halo in LDS, derives level 1 with a 2-pixel halo and level 2 with a
 // 1-pixel halo from it (the same block rule as downsample_kernel), then
-// each level's vertices with a 1-pixel halo and the normals of its tile.
+// each level's vertices with a 1-pixel halo and the normals of its tile; a
+// level's vertices and normals are formed while the next one's depth is.
+// What bounds it: latency, a launch and four dependent phases (13 MB written
+// in 9.5 us); the phases one after the other took 9.8.
 // Every value is computed by the same arithmetic as the per-level kernels.
 constexpr int kP2x = 8, kP2y = 4;                           // level-2 tile
 constexpr int kP0w = 4 * kP2x + 8, kP0h = 4 * kP2y + 8;     // level-0 depth staged: 40 x 24
@@ -253,57 +267,11 @@ __global__ void __launch_bounds__(256) pyramid3_kernel(const uint16_t* __restric
     s0[i] = (gx >= 0 && gy >= 0 && gx < l0.w && gy < l0.h) ? d0[static_cast<size_t>(gy) * l0.w + gx] : 0;
   }
   __syncthreads();
-  // level 1, origin (X1 - 2, Y1 - 2): its 2 x 2 level-0 block starts at s0 (2 lx, 2 ly)
-  for (int i = tid; i < kP1h * kP1w; i += 256) {
-    const int lx = i % kP1w, ly = i / kP1w, gx = X1 - 2 + lx, gy = Y1 - 2 + ly;
-    uint16_t r = 0;
-    if (gx >= 0 && gy >= 0 && gx < l1.w && gy < l1.h) {
-      const uint16_t* b = s0 + (2 * ly) * kP0w + 2 * lx;
-      r = downsample_block(b[0], b[1], b[kP0w], b[kP0w + 1], scale, ds_jump);
-      if (lx >= 2 && ly >= 2 && lx < 2 + 2 * kP2x && ly < 2 + 2 * kP2y) l1.depth[static_cast<size_t>(gy) * l1.w + gx] = r;
-    }
-    s1[i] = r;
-  }
-  __syncthreads();
-  // level 2, origin (X2 - 1, Y2 - 1): its block starts at s1 (2 lx, 2 ly)
-  for (int i = tid; i < kP2h * kP2w; i += 256) {
-    const int lx = i % kP2w, ly = i / kP2w, gx = X2 - 1 + lx, gy = Y2 - 1 + ly;
-    uint16_t r = 0;
-    if (gx >= 0 && gy >= 0 && gx < l2.w && gy < l2.h) {
-      const uint16_t* b = s1 + (2 * ly) * kP1w + 2 * lx;
-      r = downsample_block(b[0], b[1], b[kP1w], b[kP1w + 1], scale, ds_jump);
-      if (lx >= 1 && ly >= 1 && lx < 1 + kP2x && ly < 1 + kP2y) l2.depth[static_cast<size_t>(gy) * l2.w + gx] = r;
-    }
-    s2[i] = r;
-  }
-  __syncthreads();
   // vertices with a one-pixel halo (NaN outside the image)
   auto vertex_at = [&](const uint16_t* sd, int sw, int sx, int sy, int gx, int gy, const PyrLevel& L) {
     if (gx < 0 || gy < 0 || gx >= L.w || gy >= L.h) return nan3();
     return vertex_of(sd[sy * sw + sx], gx, gy, L.k, scale, lo, hi);
   };
-  for (int i = tid; i < kV0h * kV0w; i += 256) {
-    const int lx = i % kV0w, ly = i / kV0w;
-    const V3 v = vertex_at(s0, kP0w, lx + 3, ly + 3, X0 - 1 + lx, Y0 - 1 + ly, l0);
-    v0[0][i] = v.x;
-    v0[1][i] = v.y;
-    v0[2][i] = v.z;
-  }
-  for (int i = tid; i < kV1h * kV1w; i += 256) {
-    const int lx = i % kV1w, ly = i / kV1w;
-    const V3 v = vertex_at(s1, kP1w, lx + 1, ly + 1, X1 - 1 + lx, Y1 - 1 + ly, l1);
-    v1[0][i] = v.x;
-    v1[1][i] = v.y;
-    v1[2][i] = v.z;
-  }
-  for (int i = tid; i < kP2h * kP2w; i += 256) {
-    const int lx = i % kP2w, ly = i / kP2w;
-    const V3 v = vertex_at(s2, kP2w, lx, ly, X2 - 1 + lx, Y2 - 1 + ly, l2);
-    v2[0][i] = v.x;
-    v2[1][i] = v.y;
-    v2[2][i] = v.z;
-  }
-  __syncthreads();
   // each level's tile: vertex and normal
   auto tile = [&](float* vx, float* vy, float* vz, int vw, int tw, int th, int X, int Y, const PyrLevel& L) {
     for (int i = tid; i < tw * th; i += 256) {
@@ -322,8 +290,54 @@ __global__ void __launch_bounds__(256) pyramid3_kernel(const uint16_t* __restric
       L.norm[o] = st3(n);
     }
   };
+  // level 1, origin (X1 - 2, Y1 - 2): its 2 x 2 level-0 block starts at s0 (2 lx, 2 ly)
+  for (int i = tid; i < kP1h * kP1w; i += 256) {
+    const int lx = i % kP1w, ly = i / kP1w, gx = X1 - 2 + lx, gy = Y1 - 2 + ly;
+    uint16_t r = 0;
+    if (gx >= 0 && gy >= 0 && gx < l1.w && gy < l1.h) {
+      const uint16_t* b = s0 + (2 * ly) * kP0w + 2 * lx;
+      r = downsample_block(b[0], b[1], b[kP0w], b[kP0w + 1], scale, ds_jump);
+      if (lx >= 2 && ly >= 2 && lx < 2 + 2 * kP2x && ly < 2 + 2 * kP2y) l1.depth[static_cast<size_t>(gy) * l1.w + gx] = r;
+    }
+    s1[i] = r;
+  }
+  for (int i = tid; i < kV0h * kV0w; i += 256) {
+    const int lx = i % kV0w, ly = i / kV0w;
+    const V3 v = vertex_at(s0, kP0w, lx + 3, ly + 3, X0 - 1 + lx, Y0 - 1 + ly, l0);
+    v0[0][i] = v.x;
+    v0[1][i] = v.y;
+    v0[2][i] = v.z;
+  }
+  __syncthreads();
+  // level 2, origin (X2 - 1, Y2 - 1): its block starts at s1 (2 lx, 2 ly)
+  for (int i = tid; i < kP2h * kP2w; i += 256) {
+    const int lx = i % kP2w, ly = i / kP2w, gx = X2 - 1 + lx, gy = Y2 - 1 + ly;
+    uint16_t r = 0;
+    if (gx >= 0 && gy >= 0 && gx < l2.w && gy < l2.h) {
+      const uint16_t* b = s1 + (2 * ly) * kP1w + 2 * lx;
+      r = downsample_block(b[0], b[1], b[kP1w], b[kP1w + 1], scale, ds_jump);
+      if (lx >= 1 && ly >= 1 && lx < 1 + kP2x && ly < 1 + kP2y) l2.depth[static_cast<size_t>(gy) * l2.w + gx] = r;
+    }
+    s2[i] = r;
+  }
+  for (int i = tid; i < kV1h * kV1w; i += 256) {
+    const int lx = i % kV1w, ly = i / kV1w;
+    const V3 v = vertex_at(s1, kP1w, lx + 1, ly + 1, X1 - 1 + lx, Y1 - 1 + ly, l1);
+    v1[0][i] = v.x;
+    v1[1][i] = v.y;
+    v1[2][i] = v.z;
+  }
   tile(v0[0], v0[1], v0[2], kV0w, 4 * kP2x, 4 * kP2y, X0, Y0, l0);
+  __syncthreads();
+  for (int i = tid; i < kP2h * kP2w; i += 256) {
+    const int lx = i % kP2w, ly = i / kP2w;
+    const V3 v = vertex_at(s2, kP2w, lx, ly, X2 - 1 + lx, Y2 - 1 + ly, l2);
+    v2[0][i] = v.x;
+    v2[1][i] = v.y;
+    v2[2][i] = v.z;
+  }
   tile(v1[0], v1[1], v1[2], kV1w, 2 * kP2x, 2 * kP2y, X1, Y1, l1);
+  __syncthreads();
   tile(v2[0], v2[1], v2[2], kP2w, kP2x, kP2y, X2, Y2, l2);
 }
 

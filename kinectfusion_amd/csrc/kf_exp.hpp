@@ -48,20 +48,41 @@ namespace kf {
    0x1.d5818dcfba487p+0, 0x1.da9e603db3285p+0, 0x1.dfc97337b9b5fp+0, 0x1.e502ee78b3ff6p+0,       \
    0x1.ea4afa2a490dap+0, 0x1.efa1bee615a27p+0, 0x1.f50765b6e4540p+0, 0x1.fa7c1819e90d8p+0}
 
+// 2^(j/64) exp(r) for x = n ln2/64 + r, n = 64 m + j: exp(x) less its factor
+// 2^m.  The products of the reduction and the polynomial are fused into their
+// sums (correctly rounded fma), which only takes roundings away.
+KF_EXP_HD inline double exp_mantissa(double x, double n, int j, const double* table) {
+  const double l_head = 0x1.62e42fefa0000p-7;   // ln2 / 64, head
+  const double l_tail = 0x1.cf79abc9e3b3ap-46;  // ln2 / 64 - head
+  const double r = std::fma(-n, l_tail, std::fma(-n, l_head, x));
+  const double q = std::fma(r, std::fma(r, std::fma(r, 1.0 / 120.0, 1.0 / 24.0), 1.0 / 6.0), 0.5);
+  const double p = std::fma(r * r, q, r);
+  const double t = table[j];
+  return std::fma(t, p, t);
+}
+
 // exp(x) for x <= 0, with `table` the 64 entries of KF_EXP2_J64_TABLE.
 KF_EXP_HD inline double exp_nonpositive(double x, const double* table) {
   if (!(x >= -110.0)) return 0.0;
-  const double inv_l = 0x1.71547652b82fep+6;      // 64 / ln2
-  const double l_head = 0x1.62e42fefa0000p-7;     // ln2 / 64, head
-  const double l_tail = 0x1.cf79abc9e3b3ap-46;    // ln2 / 64 - head
+  const double inv_l = 0x1.71547652b82fep+6;  // 64 / ln2
   const double n = std::rint(x * inv_l);
   const int ni = static_cast<int>(n);
   const int j = ni & 63;
-  const int m = (ni - j) / 64;
-  const double r = (x - n * l_head) - n * l_tail;
-  const double p = r + (r * r) * (0.5 + r * (1.0 / 6.0 + r * (1.0 / 24.0 + r * (1.0 / 120.0))));
-  const double t = table[j];
-  return std::ldexp(t + t * p, m);
+  return std::ldexp(exp_mantissa(x, n, j, table), (ni - j) / 64);
+}
+
+// The same for a float exponent, rounded to float.  n comes from a float
+// product: it may be the neighbour of the nearest, |r| <= 1.01 ln2/128, which
+// leaves the polynomial's truncation below 5e-17.  The power of two is applied
+// to the float, exactly as long as the result is normal (x > -87.3; below, a
+// denormal may be rounded twice).  Far below, where the float is 0, x is taken
+// as -200; so is a NaN, whose weight is 0.
+KF_EXP_HD inline float exp_weight(float x, const double* table) {
+  const float y = std::fmax(x, -200.0F);
+  const float n = std::rint(y * 0x1.715476p+6F);
+  const int ni = static_cast<int>(n);
+  return std::ldexp(static_cast<float>(exp_mantissa(static_cast<double>(y), static_cast<double>(n), ni & 63, table)),
+                    ni >> 6);
 }
 
 }  // namespace kf
