@@ -689,8 +689,24 @@ __global__ void __launch_bounds__(256) colsum_chunk_kernel(const uint16_t* x, in
     __syncthreads();
   }
 }
-__global__ void __launch_bounds__(256) colsum_final_kernel(const float* part, int chunks, int N, float* out) {
-  row_sum(RowSum{part, chunks, N}, static_cast<int>(blockIdx.x) * kSumCols, [&](int c, float s) { out[c] = s; });
+// The chunks of every layer's bias sum in one launch (blockIdx.y: the layer):
+// seven launches of a few microseconds' latency each took 27 us of a batch's
+// 540.
+constexpr int kLayerSums = kConv + 2;
+struct LayerSum {
+  RowSum chunks;
+  float* out;
+};
+struct LayerSums {
+  LayerSum sum[kLayerSums];
+  int count;
+  size_t used;  // floats of the chunks' buffer
+};
+__global__ void __launch_bounds__(256) colsum_final_kernel(LayerSums all) {
+  const LayerSum& l = all.sum[blockIdx.y];
+  const int c0 = static_cast<int>(blockIdx.x) * kSumCols;
+  if (c0 >= l.chunks.n) return;
+  row_sum(l.chunks, c0, [&](int c, float s) { l.out[c] = s; });
 }
 
 __global__ void adam_kernel(float* w, const float* g, float* m, float* v, uint16_t* wh, long long n, float lr,
@@ -868,10 +884,22 @@ Gemm make_gemm(const uint16_t* a, long long sam, long long sak, const uint16_t* 
   return g;
 }
 
-void colsum(kf_posenet* net, hipStream_t s, const uint16_t* x, int M, int N, float* out) {
-  const int chunks = (M + kColRows - 1) / kColRows;
-  hipLaunchKernelGGL(colsum_chunk_kernel, dim3(chunks), dim3(256), 0, s, x, M, N, net->colpart);
-  hipLaunchKernelGGL(colsum_final_kernel, dim3(blocks_for(N, kSumCols)), dim3(256), 0, s, net->colpart, chunks, N, out);
+int col_chunks(long long rows) { return static_cast<int>((rows + kColRows - 1) / kColRows); }
+
+// The chunks of a layer's bias sum; colsum_end adds those of all layers.
+void colsum(kf_posenet* net, hipStream_t s, const uint16_t* x, int M, int N, float* out, LayerSums& sums) {
+  const int chunks = col_chunks(M);
+  float* part = net->colpart + sums.used;
+  hipLaunchKernelGGL(colsum_chunk_kernel, dim3(chunks), dim3(256), 0, s, x, M, N, part);
+  KF_HIP(hipGetLastError());
+  sums.sum[sums.count++] = LayerSum{RowSum{part, chunks, N}, out};
+  sums.used += static_cast<size_t>(chunks) * N;
+}
+
+void colsum_end(hipStream_t s, const LayerSums& sums) {
+  int widest = 0;
+  for (int i = 0; i < sums.count; ++i) widest = std::max(widest, sums.sum[i].chunks.n);
+  hipLaunchKernelGGL(colsum_final_kernel, dim3(blocks_for(widest, kSumCols), sums.count), dim3(256), 0, s, sums);
   KF_HIP(hipGetLastError());
 }
 
@@ -919,6 +947,7 @@ void forward(kf_posenet* net, hipStream_t s, int batch) {
 void backward(kf_posenet* net, hipStream_t s, const float* targets, int batch) {
   hipLaunchKernelGGL(loss_kernel, dim3(1), dim3(256), 0, s, net->out, targets, batch, net->dz[0], net->loss);
   KF_HIP(hipGetLastError());
+  LayerSums sums{};
   // fc2: dW = dout^T h, db = colsum(dout), dh = dout W masked by h > 0
   const Shape& f2 = net->shapes[kConv + 1];
   const uint16_t* h = net->act[kConv + 1];
@@ -928,7 +957,7 @@ void backward(kf_posenet* net, hipStream_t s, const float* targets, int batch) {
     g.ofm = f2.fan_in;
     g.ofn = 1;
     gemm(net, s, g);
-    colsum(net, s, net->dz[0], batch, kOut, net->grad + f2.b_off);
+    colsum(net, s, net->dz[0], batch, kOut, net->grad + f2.b_off, sums);
     Gemm d = make_gemm(net->dz[0], kOut, 1, net->wh + f2.w_off, f2.fan_in, 1, batch, f2.fan_in, kOut);
     d.outf = net->tmp;
     d.ofm = f2.fan_in;
@@ -946,7 +975,7 @@ void backward(kf_posenet* net, hipStream_t s, const float* targets, int batch) {
     g.ofm = f1.fan_in;
     g.ofn = 1;
     gemm(net, s, g);
-    colsum(net, s, net->dz[1], batch, f1.cout, net->grad + f1.b_off);
+    colsum(net, s, net->dz[1], batch, f1.cout, net->grad + f1.b_off, sums);
     Gemm d = make_gemm(net->dz[1], f1.cout, 1, net->wh + f1.w_off, f1.fan_in, 1, batch, f1.fan_in, f1.cout);
     d.outf = net->tmp;
     d.ofm = f1.fan_in;
@@ -965,7 +994,7 @@ void backward(kf_posenet* net, hipStream_t s, const float* targets, int batch) {
     g.ofm = K;
     g.ofn = 1;
     gemm(net, s, g);
-    colsum(net, s, net->dz[cur], M, N, net->grad + sh.b_off);
+    colsum(net, s, net->dz[cur], M, N, net->grad + sh.b_off, sums);
     if (l == 0) break;
     Gemm d = make_gemm(net->dz[cur], N, 1, net->wh + sh.w_off, K, 1, M, K, N);
     d.outf = net->tmp;
@@ -978,6 +1007,7 @@ void backward(kf_posenet* net, hipStream_t s, const float* targets, int batch) {
     KF_HIP(hipGetLastError());
     cur = 1 - cur;
   }
+  colsum_end(s, sums);
 }
 
 void check_batch(const kf_posenet* net, int batch) {
@@ -1125,7 +1155,7 @@ kf_status kf_posenet_create(const kf_posenet_config* cfg, kf_posenet** out) {
     net->v = nalloc<float>(P);
     net->wh = nalloc<uint16_t>(P);
     const int B = cfg->batch_capacity;
-    size_t max_tmp = 0, max_dz = 0, max_m = 0;
+    size_t max_tmp = 0, max_dz = 0;
     net->act[0] = nalloc<uint16_t>(static_cast<size_t>(B) * kInH * kInW * 2);
     for (int l = 0; l < kLayers - 1; ++l) {
       const Shape& sh = net->shapes[l];
@@ -1134,7 +1164,6 @@ kf_status kf_posenet_create(const kf_posenet_config* cfg, kf_posenet** out) {
       if (l < kConv) net->col[l] = nalloc<uint16_t>(M * sh.fan_in);
       max_tmp = std::max(max_tmp, M * sh.fan_in);  // dcol / dx of any layer
       max_dz = std::max(max_dz, M * sh.cout);
-      max_m = std::max(max_m, M);
     }
     max_dz = std::max(max_dz, static_cast<size_t>(B) * kOut);
     net->out = nalloc<float>(static_cast<size_t>(B) * kOut);
@@ -1143,7 +1172,10 @@ kf_status kf_posenet_create(const kf_posenet_config* cfg, kf_posenet** out) {
     net->dz[1] = nalloc<uint16_t>(max_dz);
     net->partial_floats = static_cast<size_t>(8) << 20;
     net->partial = nalloc<float>(net->partial_floats);
-    net->colpart = nalloc<float>(((max_m + kColRows - 1) / kColRows) * 256);
+    size_t chunk_floats = 0;  // of every layer's bias sum (a dense layer's shape has one pixel)
+    for (const Shape& sh : net->shapes)
+      chunk_floats += static_cast<size_t>(col_chunks(static_cast<long long>(B) * pixels(sh))) * sh.cout;
+    net->colpart = nalloc<float>(chunk_floats);
     net->loss = nalloc<float>(1);
     KF_HIP(hipHostMalloc(reinterpret_cast<void**>(&net->loss_host), sizeof(float), hipHostMallocDefault));
     std::vector<float> w(P);

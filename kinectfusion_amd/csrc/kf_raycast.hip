@@ -74,15 +74,15 @@ void launch_t(kf_context* ctx, const RayParams& rp, const Rigid& pose, IcpState*
         HashedStore<Kind>{hash_view(ctx), static_cast<const Raw*>(ctx->voxels), ctx->colors}, ctx->grid,
         1.0F / ctx->grid.voxel};
     hipLaunchKernelGGL((raycast_kernel<Kind, HashedStore<Kind>>), grid, dim3(256), 0, ctx->stream, vol, rp, pose,
-                       state, L.model_pts, L.model_nrm, L.model_col, ctx->class_bits, ctx->nbr_obs, block_map(ctx->grid), ctx->coarse, coarse_map(ctx->grid),
-                       begin_level, shape);
+                       state, L.model_pts, L.model_nrm, L.model_col, ctx->class_bits, ctx->nbr_obs,
+                       block_map(ctx->grid), ctx->coarse, coarse_map(ctx->grid), begin_level, shape);
     return;
   }
   Sampler<Kind> vol{DenseStore<Kind>{static_cast<const Raw*>(ctx->voxels), ctx->colors}, ctx->grid,
                     1.0F / ctx->grid.voxel};
   hipLaunchKernelGGL((raycast_kernel<Kind, DenseStore<Kind>>), grid, dim3(256), 0, ctx->stream, vol, rp, pose, state,
-                     L.model_pts, L.model_nrm, L.model_col, ctx->class_bits, ctx->nbr_obs, block_map(ctx->grid), ctx->coarse, coarse_map(ctx->grid),
-                     begin_level, shape);
+                     L.model_pts, L.model_nrm, L.model_col, ctx->class_bits, ctx->nbr_obs, block_map(ctx->grid),
+                     ctx->coarse, coarse_map(ctx->grid), begin_level, shape);
 }
 
 }  // namespace
