@@ -851,22 +851,49 @@ __global__ void __launch_bounds__(256) coarse_distance_z_kernel(const uint8_t* _
 // Neighbour masks of the non-skip blocks: bit (dz + 1) * 9 + (dy + 1) * 3 +
 // (dx + 1) = the block at that offset lies in the grid and holds an observed
 // voxel.  A skip block keeps its old mask: the raycaster uses a mask only for
-// a non-skip block.  One thread per block.
+// a non-skip block.  A wave takes kNbrRun runs of 64 blocks, spread over the
+// grid, their skip words read together: nearly all are skip blocks, and one
+// thread for each (65536 workgroups at 2048^3) was bound by their dispatch (19
+// us, 16 now; 39 with the runs side by side, whose busy ones then queue).  The
+// words of a block's nine rows are read unguarded, so together.
+constexpr int kNbrRun = 4;
 __global__ void __launch_bounds__(256) neighbour_mask_kernel(const uint32_t* __restrict__ obs,
                                                               const uint32_t* __restrict__ skip,
                                                               uint32_t* __restrict__ nbr, BlockMap bm, int nblocks) {
-  const int b = static_cast<int>(blockIdx.x * 256 + threadIdx.x);
-  if (b >= nblocks || bm.bit(skip, b)) return;
-  const int x = b % bm.bx, y = (b / bm.bx) % bm.by, z = b / (bm.bx * bm.by);
-  uint32_t m = 0U;
-  for (int dz = -1; dz <= 1; ++dz)
-    for (int dy = -1; dy <= 1; ++dy)
-      for (int dx = -1; dx <= 1; ++dx) {
-        const int xx = x + dx, yy = y + dy, zz = z + dz;
-        if (xx < 0 || yy < 0 || zz < 0 || xx >= bm.bx || yy >= bm.by || zz >= bm.bz) continue;
-        if (bm.bit(obs, bm.flat(xx, yy, zz))) m |= 1U << ((dz + 1) * 9 + (dy + 1) * 3 + (dx + 1));
-      }
-  nbr[b] = m;
+  const int lane = static_cast<int>(threadIdx.x & 63);
+  const long long first = (static_cast<long long>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * 64 + lane;
+  const long long stride = static_cast<long long>(gridDim.x) * 256;
+  uint32_t word[kNbrRun];
+#pragma unroll
+  for (int r = 0; r < kNbrRun; ++r) word[r] = skip[min(first + stride * r, static_cast<long long>(nblocks - 1)) >> 5];
+#pragma unroll 1
+  for (int r = 0; r < kNbrRun; ++r) {
+    const long long at = first + stride * r;
+    uint32_t w = word[0];
+#pragma unroll
+    for (int k = 1; k < kNbrRun; ++k) w = k == r ? word[k] : w;
+    if (at >= nblocks || ((w >> (at & 31)) & 1U) != 0U) continue;
+    const int b = static_cast<int>(at);
+    const int x = b % bm.bx, y = (b / bm.bx) % bm.by, z = b / (bm.bx * bm.by);
+    const int left = x > 0 ? 1 : 0, right = x + 1 < bm.bx ? 1 : 0;
+    uint32_t below[9], mid[9], above[9];  // along x, per row around
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      const int f = bm.flat(x, min(max(y + k % 3 - 1, 0), bm.by - 1), min(max(z + k / 3 - 1, 0), bm.bz - 1));
+      below[k] = obs[(f - left) >> 5] >> ((f - left) & 31);
+      mid[k] = obs[f >> 5] >> (f & 31);
+      above[k] = obs[(f + right) >> 5] >> ((f + right) & 31);
+    }
+    uint32_t m = 0U;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      const int yy = y + k % 3 - 1, zz = z + k / 3 - 1;
+      const uint32_t three = (left != 0 ? below[k] & 1U : 0U) | (mid[k] & 1U) << 1 |
+                             (right != 0 ? above[k] & 1U : 0U) << 2;
+      m |= yy >= 0 && zz >= 0 && yy < bm.by && zz < bm.bz ? three << (3 * k) : 0U;
+    }
+    nbr[b] = m;
+  }
 }
 
 // observed bits from the voxel array (after an upload): one thread per block.
@@ -1023,17 +1050,20 @@ __global__ void __launch_bounds__(256) assign_slots_kernel(HashView hv, const ui
   const uint32_t frame = sp[3];
   const uint32_t first = blockIdx.x * (256U * kAssignRun) + threadIdx.x;
   unsigned long long e[kAssignRun];
+  uint32_t when[kAssignRun];
   uint32_t visited = 0U, fresh = 0U;  // bit r: bucket first + 256 r
 #pragma unroll
+  for (int r = 0; r < kAssignRun; ++r) {  // unguarded: a guarded read waits for the one before it (15 us, 10 so)
+    const uint32_t b = min(first + 256U * r, buckets - 1);
+    e[r] = hv.table[b];
+    when[r] = stamp[b];
+  }
+#pragma unroll
   for (int r = 0; r < kAssignRun; ++r) {
-    const uint32_t b = first + 256U * r;
-    e[r] = kHashEmpty;
-    if (b < buckets) {
-      e[r] = hv.table[b];
-      if (e[r] != kHashEmpty && stamp[b] == frame) {
-        visited |= 1U << r;
-        if (static_cast<uint32_t>(e[r]) == kPendingSlot) fresh |= 1U << r;
-      }
+    if (first + 256U * r >= buckets) e[r] = kHashEmpty;
+    if (e[r] != kHashEmpty && when[r] == frame) {
+      visited |= 1U << r;
+      if (static_cast<uint32_t>(e[r]) == kPendingSlot) fresh |= 1U << r;
     }
   }
   uint32_t total;
@@ -1376,7 +1406,8 @@ void launch_skip_map(kf_context* ctx, bool end_frame) {
                        ctx->coarse, cm, ncells);
   }
   if (ctx->nbr_obs != nullptr)
-    hipLaunchKernelGGL(neighbour_mask_kernel, dim3((nblocks + 255) / 256), dim3(256), 0, ctx->stream, ctx->obs_bits,
+    hipLaunchKernelGGL(neighbour_mask_kernel, dim3((nblocks + 256 * kNbrRun - 1) / (256 * kNbrRun)), dim3(256), 0,
+                       ctx->stream, ctx->obs_bits,
                        ctx->skip_bits, ctx->nbr_obs, bm, nblocks);
   KF_HIP(hipGetLastError());
 }
