@@ -1144,7 +1144,7 @@ void launch_icp_level(kf_context* ctx, const float4* lv_v, const float4* lv_n, i
     return;
   }
   if (single_launch) {
-    if (check_max_rms > 0.0F) fail(KF_ERR_INVALID_ARGUMENT, "icp level: the learned check needs two-kernel trials");
+    if (check_max_rms > 0.0F) fail(KF_ERR_INVALID_ARGUMENT, "icp level: the learned check needs a launch per trial");
     launch_single_level(m, nb, ctx, p, iterations, level);
     return;
   }

@@ -592,8 +592,8 @@ void launch_raycast(kf_context* ctx, int level, const double* pose_dev_or_null, 
 // single_launch: one kernel for the whole level (its workgroups run the
 // trials in step, with device-scope fences and a grid-wide wait between
 // trials) -- for passes that rarely run and whose launches are mostly early
-// exits (the learned warm start's fallback); otherwise two kernels per
-// trial, the last trial's second kernel also finishing the level.
+// exits (the learned warm start's fallback); otherwise one launch per trial
+// and one that finishes the level.
 void launch_icp_level(kf_context* ctx, const float4* lv_v, const float4* lv_n, int lw, int lh,
                       const float4* md_v, const float4* md_n, int mw, int mh, Intr k,
                       int iterations, const DeviceIcpParams& p, int level_index, bool single_launch = false,
