@@ -176,9 +176,16 @@ __device__ inline float region_max(const TilePyramid& p, int tx0, int tx1, int t
 // box projects to the hull of its corners), widened by a margin; every
 // voxel behind the deepest depth of that image region by more than the
 // truncation is rejected by the fusion test.
-__device__ inline bool brick_may_fuse(const Grid& g, const FrameParams& f, const Rigid& w2c, const TilePyramid& tp,
-                                      int bx, int by, int bz) {
-  const int tiles_x = tp.tx, tiles_y = tp.ty;
+// In two halves, so that the first, which needs no depth, runs while the tiles
+// are read from another die's memory (the cull of a 512^3 grid: 8.8 us, 8.0 so).
+struct BrickHull {
+  int tx0, tx1, ty0, ty1;  // the tiles its image covers
+  float zmin;
+  bool keep;
+};
+
+__device__ inline BrickHull brick_hull(const Grid& g, const FrameParams& f, const Rigid& w2c, int tiles_x, int tiles_y,
+                                       int bx, int by, int bz) {
   bool keep;
   const int xs[2] = {bx * kBrickX, min(bx * kBrickX + kBrickX - 1, g.nx - 1)};
   const int ys[2] = {by * kBrickY, min(by * kBrickY + kBrickY - 1, g.ny - 1)};
@@ -220,8 +227,14 @@ __device__ inline bool brick_may_fuse(const Grid& g, const FrameParams& f, const
     }
   }
   if (keep && (tx0 > tx1 || ty0 > ty1)) keep = false;
+  return BrickHull{tx0, tx1, ty0, ty1, zmin, keep};
+}
+
+__device__ inline bool brick_may_fuse(const Grid& g, const FrameParams& f, const TilePyramid& tp, const BrickHull& b) {
+  bool keep = b.keep;
+  const float zmin = b.zmin;
   if (keep) {
-    const float dmax = region_max(tp, tx0, tx1, ty0, ty1);
+    const float dmax = region_max(tp, b.tx0, b.tx1, b.ty0, b.ty1);
     if (!(dmax > 0.0F)) {
       keep = false;
     } else if (zmin > 1.0e-3F) {
@@ -258,14 +271,24 @@ __global__ void __launch_bounds__(256) brick_cull_kernel(Grid g, FrameParams f,
   // the workgroup's depth pyramid
   const int t1x = (tiles_x + 3) / 4, t1y = (tiles_y + 3) / 4, t2x = (t1x + 3) / 4, t2y = (t1y + 3) / 4;
   const int n1 = t1x * t1y, n_tiles = tiles_x * tiles_y;
+  float v[8];
+  auto read = [&](int i0) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = tile_max[min(i0 + k * 256 + static_cast<int>(threadIdx.x), n_tiles - 1)];
+  };
+  read(0);
+  BrickHull hull[kCullBricks];
+#pragma unroll
+  for (int k = 0; k < kCullBricks; ++k) {
+    const int b = min((static_cast<int>(blockIdx.x) * kCullBricks + k) * 256 + static_cast<int>(threadIdx.x), nb - 1);
+    hull[k] = brick_hull(g, f, w2c, tiles_x, tiles_y, b % bnx, (b / bnx) % bny, b / (bnx * bny));
+  }
   if (group_levels != 0)
     for (int i = static_cast<int>(threadIdx.x); i < n1 + t2x * t2y; i += 256) levels[i] = 0U;
   __syncthreads();
   float fmax_t = 0.0F;
   for (int i0 = 0; i0 < n_tiles; i0 += 8 * 256) {
-    float v[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = tile_max[min(i0 + k * 256 + static_cast<int>(threadIdx.x), n_tiles - 1)];
+    if (i0 != 0) read(i0);
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const int i = i0 + k * 256 + static_cast<int>(threadIdx.x);
@@ -286,7 +309,7 @@ __global__ void __launch_bounds__(256) brick_cull_kernel(Grid g, FrameParams f,
 #pragma unroll
   for (int k = 0; k < kCullBricks; ++k) {
     const int b = (static_cast<int>(blockIdx.x) * kCullBricks + k) * 256 + static_cast<int>(threadIdx.x);
-    const bool keep = b < nb && brick_may_fuse(g, f, w2c, tp, b % bnx, (b / bnx) % bny, b / (bnx * bny));
+    const bool keep = b < nb && brick_may_fuse(g, f, tp, hull[k]);
     kept[k] = __ballot(keep);
   }
   if (lane == 0) {
