@@ -25,9 +25,11 @@ constexpr int kMaxRadius = 8;
 // float, which matches a correctly rounded expf.
 //
 // What bounds it: vector issue, 32 instructions a tap (49 taps at radius 3),
-// 12 of the 17 us a 640 x 480 frame takes.  Fused sums in the exponential, its
-// reduction in float and its power of two applied to the float took 24 us to
-// 17.  Interleaving a row's exponentials by hand gained nothing.
+// 12 of the 17 us a 640 x 480 frame takes.  Fused sums in the exponential and
+// its reduction in float took 24 us to 17.  Interleaving a row's exponentials
+// by hand gained nothing, and neither does scaling the weight as a float after
+// its rounding (35.8 us for this kernel and the pyramid, both ways), which
+// rounds denormal weights twice.
 //
 // R > 0: the window's radius fixed at compile time and each row's taps
 // unrolled, so their exponentials overlap; the sums still add the taps in the

@@ -74,15 +74,15 @@ KF_EXP_HD inline double exp_nonpositive(double x, const double* table) {
 // The same for a float exponent, rounded to float.  n comes from a float
 // product: it may be the neighbour of the nearest, |r| <= 1.01 ln2/128, which
 // leaves the polynomial's truncation below 5e-17.  The power of two is applied
-// to the float, exactly as long as the result is normal (x > -87.3; below, a
-// denormal may be rounded twice).  Far below, where the float is 0, x is taken
-// as -200; so is a NaN, whose weight is 0.
+// to the double, so that the float is rounded once, also where it is denormal.
+// Far below, where the float is 0, x is taken as -200 (2^-289 is a normal
+// double); so is a NaN, whose weight is 0.
 KF_EXP_HD inline float exp_weight(float x, const double* table) {
   const float y = std::fmax(x, -200.0F);
   const float n = std::rint(y * 0x1.715476p+6F);
   const int ni = static_cast<int>(n);
-  return std::ldexp(static_cast<float>(exp_mantissa(static_cast<double>(y), static_cast<double>(n), ni & 63, table)),
-                    ni >> 6);
+  return static_cast<float>(
+      std::ldexp(exp_mantissa(static_cast<double>(y), static_cast<double>(n), ni & 63, table), ni >> 6));
 }
 
 }  // namespace kf
