@@ -805,8 +805,8 @@ struct kf_mesh {
 namespace kf {
 namespace {
 
-// Scratch kept between calls is at most this long; a longer block is returned
-// when its call ends.
+// The scratch blocks kept between calls are at most this long in all: beyond it
+// the longest are returned when their call ends.
 constexpr size_t kKeepBytes = size_t{256} << 20;
 
 void read_totals(kf_context* ctx) { KF_HIP(hipStreamSynchronize(ctx->stream)); }
@@ -932,11 +932,17 @@ void extract_t(kf_context* ctx, float min_weight, kf_mesh* mesh) {
 // and scratch beyond the bound returned.
 void end_extract(kf_context* ctx) {
   const hipError_t err = hipStreamSynchronize(ctx->stream);
-  for (auto& b : ctx->mesh_scratch)
-    if (b.bytes > kKeepBytes) {
-      (void)hipFree(b.p);
-      b = DeviceBlock{};
+  for (;;) {
+    size_t all = 0;
+    DeviceBlock* longest = ctx->mesh_scratch;
+    for (auto& b : ctx->mesh_scratch) {
+      all += b.bytes;
+      if (b.bytes > longest->bytes) longest = &b;
     }
+    if (all <= kKeepBytes) break;
+    (void)hipFree(longest->p);
+    *longest = DeviceBlock{};
+  }
   KF_HIP(err);
 }
 

@@ -1,6 +1,8 @@
 """Shared helpers for the parity tests: configurations of the synthetic
 workloads and conversions between the oracle's host arrays and the
 library's device tensors."""
+import ctypes as C
+
 import numpy as np
 
 INTR = (525.0, 525.0, 319.5, 239.5)
@@ -69,3 +71,37 @@ def first_mismatch(a, b):
     b32 = np.ascontiguousarray(b).view(np.uint32).reshape(-1)
     idx = np.nonzero(a32 != b32)[0]
     return (len(idx), idx[:5], a.reshape(-1)[idx[:5]], b.reshape(-1)[idx[:5]]) if len(idx) else None
+
+
+def noisy_pipeline(K, res, seed=0):
+    """A pipeline over res^3 voxels of random signs: about two triangles a voxel."""
+    p = K.Pipeline(K.PipelineConfig(voxel="bf16", color="none",
+                                    volume=K.VolumeGeometry((res,) * 3, 0.01, (0, 0, 0), 0.05)))
+    t = np.random.default_rng(seed).uniform(-1.0, 1.0, res ** 3).astype(np.float32)
+    vox = np.empty((res ** 3, 2), np.uint16)
+    vox[:, 0], vox[:, 1] = t.view(np.uint32) >> 16, 256
+    p.upload_volume(vox)
+    return p
+
+
+def extract_mesh(p):
+    """A mesh by the C entry points: its handle, vertices and triangles."""
+    from kinectfusion_amd import _native as N
+
+    lib, h, nv, nt = N.hip(), C.c_void_p(), C.c_int64(), C.c_int64()
+    N.check(lib.kf_mesh_extract(p.ctx, 0.0, C.byref(h)), p.ctx)
+    N.check(lib.kf_mesh_size(h, C.byref(nv), C.byref(nt)))
+    return h, nv.value, nt.value
+
+
+def copy_mesh(mesh):
+    """The status of kf_mesh_copy and its four arrays."""
+    from kinectfusion_amd import _native as N
+
+    h, nv, nt = mesh
+    out = [np.zeros((nv, 3), np.float32) for _ in range(3)] + [np.zeros((nt, 3), np.uint32)]
+    return N.hip().kf_mesh_copy(h, *(a.ctypes.data_as(C.c_void_p) for a in out)), out
+
+
+def same_mesh(a, b):
+    return all(np.array_equal(x.view(np.uint32), y.view(np.uint32)) for x, y in zip(a, b))
