@@ -11,7 +11,7 @@
  * Conventions
  *  - Every call returns kf_status; KF_OK is 0.  No C++ exception crosses
  *    the ABI.  kf_last_error(ctx) describes the last failure (ctx may be
- *    NULL for failures of kf_create).
+ *    NULL for failures of kf_create and kf_mesh_copy).
  *  - A context is confined to one host thread and owns one HIP stream; all
  *    device work of the context is ordered on it.  Calls that return host
  *    data synchronise that stream; the others only enqueue work.
@@ -409,7 +409,12 @@ kf_status kf_block_bitmaps(kf_context* ctx, uint32_t* observed, uint32_t* skip, 
  * cell classification, stream-compacted triangles and the reference's
  * first-encounter vertex welding order.  The mesh stays in device memory of
  * its own (36 B a vertex, 12 B a triangle) until kf_mesh_free, and may outlive
- * the context; kf_mesh_copy transfers it. */
+ * the context; kf_mesh_copy transfers it.  Neither waits for another stream's
+ * work (but for a hardware queue that the runtime shares between streams), and
+ * both may be called while the program captures a graph.  A context keeps the
+ * memory of freed meshes, up to 256 MB, for the next one; beyond that, and
+ * once the context is destroyed, kf_mesh_free waits for the device as hipFree
+ * does.  kf_last_error(NULL) describes a failed kf_mesh_copy. */
 kf_status kf_mesh_extract(kf_context* ctx, float min_weight, kf_mesh** out);
 kf_status kf_mesh_size(const kf_mesh* mesh, int64_t* vertices, int64_t* triangles);
 kf_status kf_mesh_copy(const kf_mesh* mesh, float* positions, float* normals, float* colors,

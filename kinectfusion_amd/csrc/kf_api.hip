@@ -38,6 +38,18 @@ namespace {
 
 thread_local std::string g_create_error;
 
+}  // namespace
+
+kf_status detached_error(hipError_t err, const char* what) noexcept {
+  try {
+    g_create_error = std::string(what) + ": " + hipGetErrorString(err);
+  } catch (...) {  // no memory for a text
+  }
+  return err == hipErrorOutOfMemory ? KF_ERR_OUT_OF_MEMORY : KF_ERR_DEVICE;
+}
+
+namespace {
+
 template <typename F>
 kf_status guard(kf_context* ctx, F&& body) {
   try {
@@ -418,6 +430,7 @@ hipError_t HostStage::run(const Piece* pieces, int n, hipStream_t stream) {
   if (parts >= kHelperParts) {
     try {
       helper = std::thread([&] {
+        const BesideCaptures allowed;  // a mesh's copy waits beside captures, in either thread
         for (size_t i = 1; i < parts; i += 2) {
           while (issued.load(std::memory_order_acquire) <= i) {
             if (stop.load(std::memory_order_acquire)) return;
@@ -886,6 +899,7 @@ void kf_destroy(kf_context* ctx) {
   dfree(ctx->work);
   dfree(ctx->sparse);
   for (auto& b : ctx->mesh_scratch) dfree(b.p);
+  ctx->share->release();
   if (ctx->mesh_totals != nullptr) (void)hipHostFree(ctx->mesh_totals);
   if (ctx->icp_host != nullptr) (void)hipHostFree(ctx->icp_host);
   for (auto& e : ctx->ev)
@@ -1233,7 +1247,7 @@ kf_status kf_volume_download(kf_context* ctx, void* voxels, float* colors) {
       try {
         launch_expand_hashed(ctx, dv, dc);
         const HostStage::Piece out[2] = {{voxels, dv, vb}, {colors, dc, cb}};
-        KF_HIP(ctx->stage->copy(out, 2, ctx->stream));
+        KF_HIP(ctx->share->stage.copy(out, 2, ctx->stream));
       } catch (...) {
         (void)hipStreamSynchronize(ctx->stream);
         dfree(dv);
@@ -1247,7 +1261,7 @@ kf_status kf_volume_download(kf_context* ctx, void* voxels, float* colors) {
     const HostStage::Piece out[2] = {
         {voxels, ctx->voxels, ctx->n_voxels * voxel_bytes(ctx->cfg.voxel_store)},
         {colors, ctx->colors, ctx->colors != nullptr ? ctx->n_voxels * sizeof(float4) : 0}};
-    KF_HIP(ctx->stage->copy(out, 2, ctx->stream));
+    KF_HIP(ctx->share->stage.copy(out, 2, ctx->stream));
   });
 }
 

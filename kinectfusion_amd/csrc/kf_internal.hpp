@@ -456,6 +456,43 @@ struct DeviceBlock {
   size_t bytes = 0;
 };
 
+// While one lives, its thread may allocate, free and wait beside a capture
+// that the program makes on a stream of its own: otherwise the runtime refuses
+// such calls, and ends that capture.
+struct BesideCaptures {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  BesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~BesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  BesideCaptures(const BesideCaptures&) = delete;
+  BesideCaptures& operator=(const BesideCaptures&) = delete;
+};
+
+// What a context shares with its meshes, which may outlive it: the ring of
+// their copies; a stream for the meshes' copies, which so wait for no other
+// stream; and the memory of freed meshes, kept for the next extraction, since
+// the runtime's free waits for the whole device.  Safe in any thread.
+class MeshShare {
+ public:
+  HostStage stage;
+  ~MeshShare();
+  hipStream_t stream();  // throws
+  // Memory for a mesh: a kept block of its size to twice that, else a new one,
+  // the kept ones being released (throws).
+  DeviceBlock take(size_t bytes);
+  // A freed mesh's memory: kept while the kept blocks are at most kKeepBytes
+  // and kBlocks, else freed at once.
+  void give(DeviceBlock block);
+  void release();
+
+ private:
+  static constexpr size_t kKeepBytes = size_t{256} << 20;
+  static constexpr int kBlocks = 8;
+  std::mutex mu_;
+  hipStream_t stream_ = nullptr;
+  DeviceBlock kept_[kBlocks];
+  int n_ = 0;
+};
+
 }  // namespace kf
 
 struct kf_context {
@@ -550,8 +587,7 @@ struct kf_context {
   bool timed_learned = false;
   // mesh extraction: device scratch kept between calls (bit maps; active
   // cells; vertices) and the pinned counts its scans write
-  // shared with the context's meshes, which may outlive it
-  std::shared_ptr<kf::HostStage> stage = std::make_shared<kf::HostStage>();
+  std::shared_ptr<kf::MeshShare> share = std::make_shared<kf::MeshShare>();
   kf::DeviceBlock mesh_scratch[3];
   unsigned long long* mesh_totals = nullptr;
 };
@@ -567,6 +603,8 @@ struct Failure {
 
 [[noreturn]] void fail(kf_status status, const std::string& message);
 void hip_check(hipError_t err, const char* what);
+// The failure of a call that has no context: its text is kf_last_error(NULL)'s.
+kf_status detached_error(hipError_t err, const char* what) noexcept;
 #define KF_HIP(expr) ::kf::hip_check((expr), #expr)
 
 // Launch helpers implemented per stage.

@@ -787,10 +787,11 @@ class Scratch {
 // A mesh on the device: positions, normals, colours (3 floats a vertex each)
 // and triangles, in one block that the mesh owns.
 struct kf_mesh {
-  void* block = nullptr;
+  kf::DeviceBlock block;
   size_t vertices = 0, triangles = 0;
-  std::shared_ptr<kf::HostStage> stage;
-  float* positions() const { return static_cast<float*>(block); }
+  std::shared_ptr<kf::MeshShare> share;
+  hipStream_t copies = nullptr;  // the share's
+  float* positions() const { return static_cast<float*>(block.p); }
   float* normals() const { return positions() + 3 * vertices; }
   float* colors() const { return normals() + 3 * vertices; }
   uint32_t* faces() const { return reinterpret_cast<uint32_t*>(colors() + 3 * vertices); }
@@ -798,11 +799,55 @@ struct kf_mesh {
   kf_mesh(const kf_mesh&) = delete;
   kf_mesh& operator=(const kf_mesh&) = delete;
   ~kf_mesh() {
-    if (block != nullptr) (void)hipFree(block);
+    if (block.p != nullptr) share->give(block);
   }
 };
 
 namespace kf {
+
+MeshShare::~MeshShare() {
+  release();
+  if (stream_ != nullptr) (void)hipStreamDestroy(stream_);
+}
+
+hipStream_t MeshShare::stream() {
+  const std::lock_guard<std::mutex> lock(mu_);
+  if (stream_ == nullptr) KF_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
+  return stream_;
+}
+
+DeviceBlock MeshShare::take(size_t bytes) {
+  const std::lock_guard<std::mutex> lock(mu_);
+  for (int i = 0; i < n_; ++i)
+    if (kept_[i].bytes >= bytes && kept_[i].bytes <= 2 * bytes) {
+      const DeviceBlock b = kept_[i];
+      kept_[i] = kept_[--n_];
+      return b;
+    }
+  while (n_ > 0) (void)hipFree(kept_[--n_].p);
+  DeviceBlock b{nullptr, bytes};
+  KF_HIP(hipMalloc(&b.p, bytes));
+  return b;
+}
+
+void MeshShare::give(DeviceBlock block) {
+  {
+    const std::lock_guard<std::mutex> lock(mu_);
+    size_t all = block.bytes;
+    for (int i = 0; i < n_; ++i) all += kept_[i].bytes;
+    if (all <= kKeepBytes && n_ < kBlocks) {
+      kept_[n_++] = block;
+      return;
+    }
+  }
+  (void)hipFree(block.p);
+}
+
+void MeshShare::release() {
+  const std::lock_guard<std::mutex> lock(mu_);
+  while (n_ > 0) (void)hipFree(kept_[--n_].p);
+}
+
 namespace {
 
 // The scratch blocks kept between calls are at most this long in all: beyond it
@@ -841,7 +886,8 @@ void run_mc(kf_context* ctx, const Sampler<Kind, Store>& vol, const Layout& o, c
   read_totals(ctx);
   const unsigned long long ntri = totals[0], nvert = totals[1];
   if (ntri >= (1ULL << 31) || nvert >= (1ULL << 31)) fail(KF_ERR_OUT_OF_MEMORY, "mesh exceeds 2^31 elements");
-  KF_HIP(hipMalloc(&mesh->block, 36 * nvert + 12 * ntri));
+  mesh->copies = mesh->share->stream();
+  mesh->block = mesh->share->take(36 * nvert + 12 * ntri);
   mesh->vertices = nvert;
   mesh->triangles = ntri;
   Scratch verts(ctx, 2, Scratch::padded(nvert * sizeof(Word)) + Scratch::padded(nvert * 4) + Scratch::padded(16));
@@ -958,7 +1004,7 @@ kf_status kf_mesh_extract(kf_context* ctx, float min_weight, kf_mesh** out) {
   *out = nullptr;
   auto* mesh = new (std::nothrow) kf_mesh();
   if (mesh == nullptr) return KF_ERR_OUT_OF_MEMORY;
-  mesh->stage = ctx->stage;
+  mesh->share = ctx->share;
   kf_status status = KF_OK;
   auto attempt = [&](auto&& body) {
     try {
@@ -1009,9 +1055,15 @@ kf_status kf_mesh_copy(const kf_mesh* mesh, float* positions, float* normals, fl
                                    {normals, mesh->normals(), v},
                                    {colors, mesh->colors(), v},
                                    {triangles, mesh->faces(), 12 * mesh->triangles}};
-  return mesh->stage->copy(out, 4, nullptr) == hipSuccess ? KF_OK : KF_ERR_DEVICE;
+  if (mesh->vertices == 0) return KF_OK;
+  const BesideCaptures allowed;
+  const hipError_t err = mesh->share->stage.copy(out, 4, mesh->copies);
+  return err == hipSuccess ? KF_OK : detached_error(err, "kf_mesh_copy");
 }
 
-void kf_mesh_free(kf_mesh* mesh) { delete mesh; }
+void kf_mesh_free(kf_mesh* mesh) {
+  const BesideCaptures allowed;
+  delete mesh;
+}
 
 }  // extern "C"

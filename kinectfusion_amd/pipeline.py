@@ -631,7 +631,7 @@ class MarchingCubes:
             tri = np.empty((nt.value, 3), np.uint32)
             vp = C.c_void_p
             N.check(L.kf_mesh_copy(h, pos.ctypes.data_as(vp), nrm.ctypes.data_as(vp), col.ctypes.data_as(vp),
-                                   tri.ctypes.data_as(vp)), pipeline.ctx)
+                                   tri.ctypes.data_as(vp)))
         finally:
             L.kf_mesh_free(h)
         return Mesh(pos, nrm, col, tri)
