@@ -178,7 +178,7 @@ __device__ __forceinline__ void sweep_block(const Maps& m, const Rigid& cam, con
     if (base < n) read_live(m, base, stride, live);
   }
   // The wave's sums: at each step a lane keeps half of its values and takes
-  // the other lanes' halves of them, so 31 exchanges reduce all 30 (a
+  // the other lanes' halves of them, so 32 exchanges reduce all 30 (a
   // butterfly of every value takes 180); each value is the same tree of
   // pairwise sums over lanes 32, 16, ..., 1 apart.  Lane 2 i ends with value i.
   // The count is summed as a float, exact below 2^24.
@@ -962,11 +962,6 @@ __device__ void sym_eig6_wave(const double* eq, double* ev) {
   wave_sync();
 }
 
-// Prepare a level: status cleared, model pose = running pose.
-__global__ void __launch_bounds__(64) icp_begin_level_kernel(IcpState* st, int level) {
-  if (threadIdx.x == 0) icp_begin_level(st, level);
-}
-
 struct Pose64 {
   double m[16];
 };
@@ -1124,11 +1119,6 @@ void launch_icp_begin_maps(kf_context* ctx, const double* model_pose, const doub
 void launch_icp_publish(kf_context* ctx, bool restore) {
   hipLaunchKernelGGL(icp_publish_kernel, dim3(1), dim3(256), 0, ctx->stream, ctx->icp, ctx->icp_mapped,
                      restore ? 1 : 0);
-  KF_HIP(hipGetLastError());
-}
-
-void launch_icp_begin_level(kf_context* ctx, int level) {
-  hipLaunchKernelGGL(icp_begin_level_kernel, dim3(1), dim3(64), 0, ctx->stream, ctx->icp, level);
   KF_HIP(hipGetLastError());
 }
 

@@ -646,17 +646,12 @@ void launch_icp_reduce_static(hipStream_t stream, const float4* lv_v, const floa
                               const float4* md_v, const float4* md_n, int mw, int mh, Intr k,
                               const float* camera12, const float* model12, float max_dist, float min_dot,
                               double* sums, int64_t* count);
-void launch_icp_begin_level(kf_context* ctx, int level_index);
 // A level between the caller's maps: the context's own pose and failure mark
 // are set aside until launch_icp_publish(ctx, true).
 void launch_icp_begin_maps(kf_context* ctx, const double* model_pose, const double* pose);
 // The state into ctx->icp_host once the stream is synchronised; restore: then
 // the context's own pose back, and no failure.
 void launch_icp_publish(kf_context* ctx, bool restore);
-// The learned warm start's fallback pass (every level: raycast, then the
-// trials) as one launch that returns at once when the learned run was kept;
-// false when its grid cannot be resident at once on this device (the caller
-// then launches each level on its own).
 void launch_fill_voxels(kf_context* ctx);
 // skip and free bits from the observed and part bits; end_frame: the launch
 // also records the frame's pose (trajectory slot, previous poses, counter)

@@ -119,7 +119,6 @@ __device__ inline void raycast_pixel(const Sampler<Kind, Store>& vol, const RayP
     int cur_blk = -1;
     bool cur_skip = false, cur_free = false, cur_empty = false;
     uint32_t cur_nbr = 0U;  // observed blocks among the current block's 3^3 (hashed store)
-    SlotCache slots;  // the last block a sample probed (hashed store)
     // The samples of a skip or free block that lie deeper than kSafe voxels
     // inside it on every axis are stepped in one run (the float additions of
     // the reference's loop, bit for bit): [enter, exit) is that stretch of
@@ -207,7 +206,7 @@ __device__ inline void raycast_pixel(const Sampler<Kind, Store>& vol, const RayP
           }
         }
         float t;
-        if (!vol.tsdf(point, rp.require_all != 0, t, slots)) {
+        if (!vol.tsdf(point, rp.require_all != 0, t)) {
           have_prev = false;
           len += base_step;
           continue;
@@ -300,7 +299,7 @@ __device__ inline void raycast_pixel(const Sampler<Kind, Store>& vol, const RayP
           continue;
         }
         float t;
-        if (!vol.tsdf(point, rp.require_all != 0, t, slots)) {
+        if (!vol.tsdf(point, rp.require_all != 0, t)) {
           have_prev = false;
           len += base_step;
           continue;

@@ -15,7 +15,8 @@ namespace kf {
 // volume_sampler.hpp:36-109 and block_rep.hpp:113-160).  A voxel of an
 // unallocated block reads as a fresh voxel and a colour voxel as zero: the
 // blends treat both exactly like the reference's missing (null) corners.
-// The last block a hashed store looked up (key, pool slot).
+// The last block that voxel_cached looked up in a hashed store (key, pool
+// slot).
 struct SlotCache {
   uint32_t key = kNoSlot;
   uint32_t slot = kNoSlot;
@@ -48,10 +49,6 @@ struct DenseStore {
   const Raw* __restrict__ vox;
   const float4* __restrict__ colors;
   __device__ inline Raw voxel(const Grid& g, int x, int y, int z) const { return vox[g.flat(x, y, z)]; }
-  // voxels (x, y, z) and (x + 1, y, z), both inside the grid
-  __device__ inline void pair(const Grid& g, int x, int y, int z, Raw& a, Raw& b) const {
-    load_pair<Raw>(vox + g.flat(x, y, z), a, b);
-  }
   // The eight corners of the cell at (x, y, z) (z -> y -> x order), all
   // inside the grid: one 64-bit index, then four x-pair loads at fixed
   // row and slice offsets.
@@ -63,9 +60,7 @@ struct DenseStore {
     load_pair<Raw>(p + slice, raw[4], raw[5]);
     load_pair<Raw>(p + slice + row, raw[6], raw[7]);
   }
-  __device__ inline Raw voxel_cached(const Grid& g, int x, int y, int z, SlotCache&) const {
-    return vox[g.flat(x, y, z)];
-  }
+  __device__ inline Raw voxel_cached(const Grid& g, int x, int y, int z, SlotCache&) const { return voxel(g, x, y, z); }
   // The colour voxels of the corners of the 2^3 stencil with base corner
   // (x, y, z), four of them (z fixed): a corner outside the grid reads a
   // clamped one, which the caller drops.
@@ -182,12 +177,22 @@ struct Sampler {
   }
   // Loads of the eight corners (z -> y -> x order); bit c of `inb` marks a
   // corner inside the grid.
-  __device__ inline void load8(const Stencil& st, typename IO::Raw (&raw)[8], unsigned& inb, SlotCache& cache) const {
+  __device__ inline void load8(const Stencil& st, typename IO::Raw (&raw)[8], unsigned& inb) const {
     if constexpr (Store::kDirect) {
       if (st.ok && st.interior) {  // four x-pairs
         s.cell(g, st.bx, st.by, st.bz, raw);
         inb = 0xFFU;
         return;
+      }
+      inb = 0U;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const int x = st.bx + (c & 1), y = st.by + ((c >> 1) & 1), z = st.bz + (c >> 2);
+        raw[c] = IO::fresh();
+        if (!st.ok) continue;
+        if (!st.interior && (x < 0 || y < 0 || z < 0 || x >= g.nx || y >= g.ny || z >= g.nz)) continue;
+        raw[c] = s.voxel(g, x, y, z);
+        inb |= 1U << c;
       }
     } else {
       // the eight slots in one round of reads, then the eight voxels
@@ -202,17 +207,6 @@ struct Sampler {
 #pragma unroll
       for (int c = 0; c < 8; ++c)
         if ((c < 4 ? lo[c & 3] : hi[c & 3]) == kNoSlot) raw[c] = IO::fresh();
-      return;
-    }
-    inb = 0U;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const int x = st.bx + (c & 1), y = st.by + ((c >> 1) & 1), z = st.bz + (c >> 2);
-      raw[c] = IO::fresh();
-      if (!st.ok) continue;
-      if (!st.interior && (x < 0 || y < 0 || z < 0 || x >= g.nx || y >= g.ny || z >= g.nz)) continue;
-      raw[c] = s.voxel_cached(g, x, y, z, cache);
-      inb |= 1U << c;
     }
   }
   // blend_tsdf over loaded corners, without branches: a corner outside the
@@ -273,13 +267,6 @@ struct Sampler {
   }
   // TrilinearSampler::tsdf + blend_tsdf.
   __device__ bool tsdf(V3 p, bool require_all, float& out) const {
-    SlotCache cache;
-    return tsdf(p, require_all, out, cache);
-  }
-  // The same with a block-slot cache that the caller keeps across samples: a
-  // hashed store probes a block once while consecutive samples stay in it
-  // (the table does not change during a launch).
-  __device__ bool tsdf(V3 p, bool require_all, float& out, SlotCache& cache) const {
     const Stencil st = stencil(p);
     if (!st.ok) return false;
     typename IO::Raw raw[8];
@@ -291,7 +278,7 @@ struct Sampler {
       }
     }
     unsigned inb;
-    load8(st, raw, inb, cache);
+    load8(st, raw, inb);
     // the two blends of a direct store must not share code: merged, the march's
     // interior cells wait for this path's registers (60 -> 68 us at 160x120)
     if constexpr (Store::kDirect) return blend_edge(st, raw, inb, require_all, out);
@@ -344,13 +331,12 @@ struct Sampler {
         Stencil st[2];
         typename IO::Raw raw[2][8];
         unsigned inb[2];
-        SlotCache cache;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           const int axis = (a0 + i) >> 1;
           const V3 off = scale3(mk3(axis == 0 ? 1.0F : 0.0F, axis == 1 ? 1.0F : 0.0F, axis == 2 ? 1.0F : 0.0F), g.voxel);
           st[i] = stencil(((a0 + i) & 1) == 0 ? add3(p, off) : sub3(p, off));
-          load8(st[i], raw[i], inb[i], cache);
+          load8(st[i], raw[i], inb[i]);
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -359,9 +345,9 @@ struct Sampler {
       dir = mk3(v[0] - v[1], v[2] - v[3], v[4] - v[5]);
     } else {
       // one sample at a time in a loop that is not unrolled: unrolled, the six
-      // probes and their chain walks were 54 KB of code, a call out of the
-      // march that kept the sampler in scratch memory for all of it
-      SlotCache cache;
+      // (when a slot took a probe of the table and a walk) were 54 KB of code, a
+      // call out of the march that kept the sampler in scratch memory for all of
+      // it
       float plus = 0.0F;
 #pragma unroll 1
       for (int k = 0; k < 6; ++k) {
@@ -370,7 +356,7 @@ struct Sampler {
         const Stencil st = stencil((k & 1) == 0 ? add3(p, off) : sub3(p, off));
         typename IO::Raw raw[8];
         unsigned inb;
-        load8(st, raw, inb, cache);
+        load8(st, raw, inb);
         float v;
         if (!blend(st, raw, inb, require_all, v)) return false;
         const float d = plus - v;
