@@ -361,8 +361,8 @@ __device__ inline bool same_raw(Raw a, Raw b) {
 // value).
 //
 // What bounds it: the reads' latencies (pixel, voxel, colour) and the
-// instructions between them, about evenly: a 512^3 room frame moves 130 MB in
-// 54 us, 26 at a copy's rate, with the vector units issuing 8 cycles in 10;
+// instructions between them, about evenly: a 512^3 room frame moves 168 MB in
+// 54 us, 33 at a copy's rate, with the vector units issuing 8 cycles in 10;
 // a variant with a quarter fewer instructions took as long.
 // Batches of 8 (62 us) or 2 (57) lose more waves, or more reads in flight, than
 // they gain.  Branch-free projection, the colours of a batch read together and

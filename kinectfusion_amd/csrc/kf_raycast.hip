@@ -44,13 +44,17 @@ __global__ void __launch_bounds__(256) raycast_kernel(Sampler<Kind, Store> vol, 
   raycast_pixel(vol, rp, pose, x, y, pts, nrm, col, class_bits, nbr_obs, bm, coarse, cm);
 }
 
-// Rays per wave.  A dense store's waves are full: its lanes do the same work
-// at every pass.  A hashed store's rays diverge (a wave runs the sampler at
-// nearly every pass for some lane), so where full waves leave the chip's wave
-// slots empty, a wave takes fewer rays: at most kSlots waves, at least 8 rays
-// each.  2048^3 hall, 16 and 8 rays a wave instead of 64: 358 -> 334 us at
-// 320x240, 324 -> 295 us at 160x120; 16 at 640x480 (19200 waves) was slower
-// (554 -> 1017 us), as were 2 at 160x120 (400 -> 500 us).
+// Rays per wave.  A dense store's waves are full: its lanes do much the same
+// work at every pass, and fewer lanes only mean more waves.  512^3 bf16 room,
+// 64, 32, 16 and 8 rays a wave: 325, 364, 429, 560 us at 640x480, 248, 254,
+// 265, 299 at 320x240 and 173, 172, 172, 181 at 160x120 (float voxels alike;
+// eight plain FP32 frames 4.07, 4.42, 5.22, 6.97 ms).
+// A hashed store's rays diverge (a wave runs the sampler at nearly every pass
+// for some lane), so where full waves leave the chip's wave slots empty, a
+// wave takes fewer rays: at most kSlots waves, at least 8 rays each.  2048^3
+// hall, 16 and 8 rays a wave instead of 64: 358 -> 334 us at 320x240, 324 ->
+// 295 us at 160x120; 16 at 640x480 (19200 waves) was slower (554 -> 1017 us),
+// as were 2 at 160x120 (400 -> 500 us).
 RayTile ray_tile(int w, int h, bool hashed_store) {
   constexpr long long kSlots = 5120;  // 256 CUs x 4 SIMDs x 5 waves
   RayTile t{3, 3};
