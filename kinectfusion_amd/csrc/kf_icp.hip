@@ -26,7 +26,7 @@
 // before it does anything and 4.4 us with its reads from another die.  A step
 // takes 14 us (sweep 5, trial 5) where the sweep and the one-thread trial as
 // two launches took 20, and a level of 10 steps, 3 of them active, 85 us for
-// 122.  kf_icp_track_maps over 640 x 480 maps: 105 us for 173.
+// 122.  kf_icp_track_maps over 640 x 480 maps: 112 us for 168.
 // Once a level's status latches (converged or failed) the remaining steps pass
 // the record on and return.  The stability spectrum (FP64) is checked once per
 // level, by its last kernel, as in the reference's device loop.  A pass that
