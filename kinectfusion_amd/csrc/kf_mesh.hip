@@ -817,14 +817,16 @@ hipStream_t MeshShare::stream() {
 }
 
 DeviceBlock MeshShare::take(size_t bytes) {
-  const std::lock_guard<std::mutex> lock(mu_);
-  for (int i = 0; i < n_; ++i)
-    if (kept_[i].bytes >= bytes && kept_[i].bytes <= 2 * bytes) {
-      const DeviceBlock b = kept_[i];
-      kept_[i] = kept_[--n_];
-      return b;
-    }
-  while (n_ > 0) (void)hipFree(kept_[--n_].p);
+  {
+    const std::lock_guard<std::mutex> lock(mu_);
+    for (int i = 0; i < n_; ++i)
+      if (kept_[i].bytes >= bytes && kept_[i].bytes <= 2 * bytes) {
+        const DeviceBlock b = kept_[i];
+        kept_[i] = kept_[--n_];
+        return b;
+      }
+  }
+  release();
   DeviceBlock b{nullptr, bytes};
   KF_HIP(hipMalloc(&b.p, bytes));
   return b;
@@ -844,8 +846,13 @@ void MeshShare::give(DeviceBlock block) {
 }
 
 void MeshShare::release() {
-  const std::lock_guard<std::mutex> lock(mu_);
-  while (n_ > 0) (void)hipFree(kept_[--n_].p);
+  DeviceBlock blocks[kBlocks];
+  int n = 0;
+  {
+    const std::lock_guard<std::mutex> lock(mu_);
+    while (n_ > 0) blocks[n++] = kept_[--n_];
+  }
+  while (n > 0) (void)hipFree(blocks[--n].p);  // waits for the device: not with the lock held
 }
 
 namespace {
@@ -866,6 +873,7 @@ void run_mc(kf_context* ctx, const Sampler<Kind, Store>& vol, const Layout& o, c
   hipLaunchKernelGGL(active_kernel<Layout>, dim3(wg), dim3(256), 0, s, o, usable, inside, active, chunks);
   hipLaunchKernelGGL(chunk_scan_kernel, dim3(1), dim3(256), 0, s, chunks, wg, totals);
   KF_HIP(hipGetLastError());
+  mesh->copies = mesh->share->stream();  // made, by the first extraction, while the device reads the volume
   read_totals(ctx);
   const unsigned long long n = totals[0];
   if (n >= (1ULL << 31)) fail(KF_ERR_OUT_OF_MEMORY, "mesh exceeds 2^31 elements");
@@ -886,7 +894,6 @@ void run_mc(kf_context* ctx, const Sampler<Kind, Store>& vol, const Layout& o, c
   read_totals(ctx);
   const unsigned long long ntri = totals[0], nvert = totals[1];
   if (ntri >= (1ULL << 31) || nvert >= (1ULL << 31)) fail(KF_ERR_OUT_OF_MEMORY, "mesh exceeds 2^31 elements");
-  mesh->copies = mesh->share->stream();
   mesh->block = mesh->share->take(36 * nvert + 12 * ntri);
   mesh->vertices = nvert;
   mesh->triangles = ntri;
